@@ -3,7 +3,7 @@
 //   RI    U, U'/r           src/ri.cu:77-110, pair loop :133-187
 //   NN2B  MLP U, U'         src/nn2b.cu:49-78, cutoff :80-92, loop :115-171
 //
-// Single-parameter-set kernels keep the reference's thread-per-atom pair loop
+// The RI single-parameter-set kernel keeps the reference's thread-per-atom pair loop
 // over the full neighbour list.  The RI population kernel reads, per bond,
 // the parameter-independent factors erfc(a r)/r, its radial derivative,
 // r^-6 and 1/r from a table built once per training set, so a lane only
@@ -311,99 +311,180 @@ int ri_population_occupancy(int block)
 
 constexpr int NN2B_MAX_PLAIN = 64;
 
-// One thread per atom, weights staged in LDS; the MLP is evaluated per bond as
-// the reference does (src/nn2b.cu:49-78), for any n <= 64.  species: the
-// first layer also takes the pair's species code t_i + t_j through the n
-// weights after the reference's parameters.
-__global__ void nn2b_plain(DevSet s, int n, int species, const float* __restrict__ w,
-                           float* __restrict__ f, float* __restrict__ virial,
-                           float* __restrict__ pe)
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// tanh x = sgn(x) (1 - e) / (1 + e) and 1 - tanh^2 x = 4 e / (1 + e)^2 with
+// e = exp(-2 |x|): about 1e-7 absolute, the derivative without a difference
+// of nearly equal numbers.
+__device__ __forceinline__ void tanh_sech2(float x, float& t, float& s)
 {
-  extern __shared__ float sw[];
-  const int V = n * (n + 4) + 1 + (species ? n : 0);
-  for (int v = threadIdx.x; v < V; v += blockDim.x) sw[v] = w[v];
-  __syncthreads();
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= s.N) return;
-  const float* w0 = sw;
-  const float* b0 = sw + n;
-  const float* w1 = sw + 2 * n;
-  const float* b1 = sw + n * (n + 2);
-  const float* w2 = sw + n * (n + 3);
-  const float bias2 = sw[n * (n + 4)];
-  const float* ws = sw + n * (n + 4) + 1;
-  const size_t N = s.N;
-  const int nn = s.nn[i], k0 = s.bond0[i];
+  const float e = fexp2(-2.0f * LOG2E * __builtin_fabsf(x));
+  const float r = frcp(1.0f + e);
+  t = __builtin_copysignf((1.0f - e) * r, x);
+  s = 4.0f * e * r * r;
+}
+
+// A wave takes NN2B_ATOMS consecutive atoms, whose bonds are consecutive, and
+// evaluates the network (src/nn2b.cu:49-78) for 32 bonds at a time: lane l
+// computes the first hidden layer and its derivative of bond l % 32 for the
+// input neurons m = 2 s + l / 32, which are the B operands (neuron x bond) of
+// v_mfma_f32_32x32x2_f32 with the weights W1 (output neuron x input neuron,
+// in registers for the whole launch) as A; lane l then holds the bond's
+// pre-activations of half of the output neurons, so the output layer is an
+// in-lane sum and one exchange with lane l ^ 32.  FP32 throughout.  The
+// bonds' (U, U'/r) pass through LDS to the atoms' sums, eight lanes an atom.
+// KS: pairs of input neurons (n <= 2 KS); NB: blocks of 32 output neurons.
+//
+// Bound by the hidden layer's MFMAs and the 2 n tanh per bond.  One thread
+// per atom with both layers in scratch memory (two scratch accesses an FMA,
+// 450 waves for 1024 SIMDs) took 4617 us on 28 800 atoms with 42 neighbours
+// and n = 32; this form 103 us.  Eight atoms a wave leave 5% of the tiles'
+// bonds empty there and give 3600 waves; with species, the code t_i + t_j
+// shifts the first layer's bias.
+constexpr int NN2B_ATOMS = 8;
+
+template <int KS, int NB>
+__global__ void __launch_bounds__(WAVE) nn2b_plain(DevSet s, int n, int species,
+                                                   const float* __restrict__ w,
+                                                   float* __restrict__ f,
+                                                   float* __restrict__ virial,
+                                                   float* __restrict__ pe)
+{
+  __shared__ float4 lr[32];
+  __shared__ float2 lu[32];
+  const int lane = threadIdx.x, col = lane & 31, half = lane >> 5;
+  const float* w0 = w;
+  const float* b0 = w + n;
+  const float* w1 = w + 2 * n;
+  const float* b1 = w + n * (n + 2);
+  const float* w2 = w + n * (n + 3);
+  const float bias2 = w[n * (n + 4)];
+  const float* ws = w + n * (n + 4) + 1;
+
+  // first-layer parameters of this lane's input neurons, W1's A operands (row
+  // 32 b + col), output-layer parameters of this lane's output neurons (rows
+  // 32 b + 8 (r / 4) + 4 half + r % 4); zero past n
+  float p0[KS], pb[KS], ps[KS], a[NB][KS], c1[NB][16], c2[NB][16];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    const int m = 2 * k + half;
+    const bool ok = m < n;
+    p0[k] = ok ? w0[m] : 0.0f;
+    pb[k] = ok ? b0[m] : 0.0f;
+    ps[k] = ok && species ? ws[m] : 0.0f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      a[b][k] = ok && 32 * b + col < n ? w1[(32 * b + col) * n + m] : 0.0f;
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int o = 32 * b + 8 * (r >> 2) + 4 * half + (r & 3);
+      c1[b][r] = o < n ? b1[o] : 0.0f;
+      c2[b][r] = o < n ? w2[o] : 0.0f;
+    }
+
+  const int i0 = blockIdx.x * NN2B_ATOMS, i1 = min(i0 + NN2B_ATOMS, s.N);
+  const int k0 = s.bond0[i0], k1 = s.bond0[i1 - 1] + s.nn[i1 - 1];
+  // the atom this lane sums for, every 8th of its bonds
+  const int i = i0 + lane / 8;
+  const bool on = i < i1;
+  const int m0 = on ? s.bond0[i] : 0, m1 = on ? m0 + s.nn[i] : 0;
   float fx = 0, fy = 0, fz = 0, wxx = 0, wyy = 0, wzz = 0, wxy = 0, wyz = 0, wzx = 0, e = 0;
-  float x1[NN2B_MAX_PLAIN], y1[NN2B_MAX_PLAIN];
-  for (int u = 0; u < nn; ++u) {
-    const float4 r = s.bond[k0 + u];
-    const float d = r.w;
-    const float code = species ? (float)s.ptype[k0 + u] : 0.0f;
-    for (int m = 0; m < n; ++m) {
+  for (int kt = k0; kt < k1; kt += 32) {
+    const int k = min(kt + col, k1 - 1);
+    const float4 rij = s.bond[k];
+    const float d = rij.w;
+    const float code = species ? (float)s.ptype[k] : 0.0f;
+    f32x16 z[NB], zd[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        z[b][r] = -c1[b][r];
+        zd[b][r] = 0.0f;
+      }
+#pragma unroll
+    for (int q = 0; q < KS; ++q) {
       // the species-pair input as a shift of the bias
-      const float bm = species ? b0[m] - ws[m] * code : b0[m];
-      x1[m] = tanhf(w0[m] * d - bm);
-      y1[m] = (1.0f - x1[m] * x1[m]) * w0[m];
+      float x, sg;
+      tanh_sech2(fmaf(p0[q], d, fmaf(ps[q], code, -pb[q])), x, sg);
+      const float y = sg * p0[q];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        z[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[b][q], x, z[b], 0, 0, 0);
+        zd[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[b][q], y, zd[b], 0, 0, 0);
+      }
     }
     float p = 0.0f, g = 0.0f;
-    for (int a = 0; a < n; ++a) {
-      float z = 0.0f, y = 0.0f;
-      for (int m = 0; m < n; ++m) {
-        z += w1[a * n + m] * x1[m];
-        y += w1[a * n + m] * y1[m];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float x, sg;
+        tanh_sech2(z[b][r], x, sg);
+        p = fmaf(c2[b][r], x, p);
+        g = fmaf(c2[b][r] * sg, zd[b][r], g);
       }
-      const float x2 = tanhf(z - b1[a]);
-      y *= 1.0f - x2 * x2;
-      p += w2[a] * x2;
-      g += w2[a] * y;
-    }
-    p -= bias2;
-    float fc, fcp;
+    p = (p + __shfl_xor(p, 32)) - bias2;
+    g += __shfl_xor(g, 32);
+    float fc = 0.0f, fcp = 0.0f;
     if (d < NN2B_R1) {
       fc = 1.0f;
-      fcp = 0.0f;
     } else if (d < NN2B_R2) {
       float sn, cs;
       sincosf(NN2B_PI_FACTOR * (d - NN2B_R1), &sn, &cs);
       fc = 0.5f * cs + 0.5f;
       fcp = -sn * NN2B_PI_FACTOR * 0.5f;
-    } else {
-      fc = 0.0f;
-      fcp = 0.0f;
     }
     const float p2 = p * fc;
     const float f2 = (g * fc + p2 * fcp) / d; // src/nn2b.cu:147-148
-    fx += r.x * f2;
-    fy += r.y * f2;
-    fz += r.z * f2;
-    wxx -= r.x * r.x * f2 * 0.5f;
-    wyy -= r.y * r.y * f2 * 0.5f;
-    wzz -= r.z * r.z * f2 * 0.5f;
-    wxy -= r.x * r.y * f2 * 0.5f;
-    wyz -= r.y * r.z * f2 * 0.5f;
-    wzx -= r.z * r.x * f2 * 0.5f;
-    e += p2 * 0.5f;
+    if (half == 0) {
+      lr[col] = rij;
+      lu[col] = make_float2(p2, f2);
+    }
+    __syncthreads();
+    const int t1 = min(m1, kt + 32);
+    for (int m = max(m0, kt) + (lane & 7); m < t1; m += 8) {
+      const float4 r = lr[m - kt];
+      const float2 u = lu[m - kt];
+      fx += r.x * u.y;
+      fy += r.y * u.y;
+      fz += r.z * u.y;
+      wxx -= r.x * r.x * u.y * 0.5f;
+      wyy -= r.y * r.y * u.y * 0.5f;
+      wzz -= r.z * r.z * u.y * 0.5f;
+      wxy -= r.x * r.y * u.y * 0.5f;
+      wyz -= r.y * r.z * u.y * 0.5f;
+      wzx -= r.z * r.x * u.y * 0.5f;
+      e += u.x * 0.5f;
+    }
+    __syncthreads();
   }
-  f[i] = fx;
-  f[i + N] = fy;
-  f[i + 2 * N] = fz;
-  virial[i] = wxx;
-  virial[i + N] = wyy;
-  virial[i + 2 * N] = wzz;
-  virial[i + 3 * N] = wxy;
-  virial[i + 4 * N] = wyz;
-  virial[i + 5 * N] = wzx;
-  pe[i] = e;
+  float out[10] = {fx, fy, fz, wxx, wyy, wzz, wxy, wyz, wzx, e};
+#pragma unroll
+  for (int q = 0; q < 10; ++q)
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) out[q] += __shfl_xor(out[q], o);
+  if (on && (lane & 7) == 0) {
+    const size_t N = s.N;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) f[i + q * N] = out[q];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) virial[i + q * N] = out[3 + q];
+    pe[i] = out[9];
+  }
 }
 
 void launch_nn2b_plain(const DevSet& s, int n, bool species, const float* w, float* f,
                        float* virial, float* pe, hipStream_t st)
 {
   if (n > NN2B_MAX_PLAIN) fail(strfmt("NN2B supports at most %d neurons", NN2B_MAX_PLAIN));
-  const int block = 128, grid = (s.N + block - 1) / block;
-  const size_t lds = sizeof(float) * (n * (n + 4) + 1 + (species ? n : 0));
-  nn2b_plain<<<grid, block, lds, st>>>(s, n, species ? 1 : 0, w, f, virial, pe);
+  const int grid = (s.N + NN2B_ATOMS - 1) / NN2B_ATOMS, sp = species ? 1 : 0;
+  if (n <= 16) nn2b_plain<8, 1><<<grid, WAVE, 0, st>>>(s, n, sp, w, f, virial, pe);
+  else if (n <= 32) nn2b_plain<16, 1><<<grid, WAVE, 0, st>>>(s, n, sp, w, f, virial, pe);
+  else nn2b_plain<32, 2><<<grid, WAVE, 0, st>>>(s, n, sp, w, f, virial, pe);
   GPUGA_HIP(hipGetLastError());
 }
 
