@@ -231,7 +231,8 @@ void Fitness::setup()
         fail("neighbour list is not symmetric (reverse bond missing)");
   // pair types on the host (the list is there); the geometry tables and the
   // atom records on the device, from the device copy of the list
-  const std::vector<int> ptype = bond_types(ts_, nl_, tersoff);
+  ptype_ = bond_types(ts_, nl_, tersoff);
+  const std::vector<int>& ptype = ptype_;
 
   hipStream_t st = stream_;
   ds_.Na.upload(ts_.Na, st);
@@ -339,20 +340,82 @@ void Fitness::setup()
     ds_.tri0.upload(std::vector<int>(ts_.N, 0), st);
     ds_.tri.upload(std::vector<float4>(1), st);
     build_geometry_device(ts_, dn, ds_.bond.get(), nullptr, st);
-    // the pair tables below are built on the host from the bond geometry
-    geo_.bond.resize(ds_.bond.size());
-    static_assert(sizeof(Vec4) == sizeof(float4), "layout");
-    ds_.bond.download(reinterpret_cast<float4*>(geo_.bond.data()), geo_.bond.size(), st);
-    GPUGA_HIP(hipStreamSynchronize(st));
-    dmin_ = 1e30f;
-    dmax_ = 0.0f;
-    for (int b = 0; b < nl_.total; ++b) {
-      dmin_ = std::min(dmin_, geo_.bond[b].w);
-      dmax_ = std::max(dmax_, geo_.bond[b].w);
+    dmin_ = dmax_ = 1.0f;
+    if (nl_.total > 0) {
+      DeviceBuffer<unsigned> range;
+      const unsigned none[2] = {0xffffffffu, 0u};
+      unsigned got[2];
+      range.upload(none, 2, st);
+      launch_bond_range(nl_.total, ds_.bond.get(), range.get(), st);
+      range.download(got, 2, st);
+      GPUGA_HIP(hipStreamSynchronize(st));
+      std::memcpy(&dmin_, &got[0], sizeof dmin_);
+      std::memcpy(&dmax_, &got[1], sizeof dmax_);
     }
-    if (nl_.total == 0) dmin_ = dmax_ = 1.0f;
+    if (spec_.type == POT_RI) {
+      ds_.ri_tab.resize(std::max(nl_.total, 1));
+      launch_ri_table((int)ds_.bond.size(), ds_.bond.get(), ds_.ri_tab.get(), st);
+    }
   }
   // the uploads above read host vectors of this scope
+  GPUGA_HIP(hipStreamSynchronize(st));
+  ds_.pe_ref.upload(ts_.pe_ref, st);
+  ds_.virial_ref.upload(ts_.virial_ref, st);
+  ds_.force_ref.upload(ts_.force_ref, st);
+  GPUGA_HIP(hipStreamSynchronize(st));
+
+  DevSet& v = ds_.view;
+  v.Nc = ts_.Nc;
+  v.Nc_force = ts_.Nc_force;
+  v.N = ts_.N;
+  v.N_force = ts_.N_force;
+  v.Na = ds_.Na.get();
+  v.Na_sum = ds_.Na_sum.get();
+  v.type = ds_.type.get();
+  v.nn = ds_.nn.get();
+  v.bond0 = ds_.bond0.get();
+  v.nl = ds_.nl.get();
+  v.rev = ds_.rev.get();
+  v.ptype = ds_.ptype.get();
+  v.bond = ds_.bond.get();
+  v.tri0 = ds_.tri0.get();
+  v.tri = ds_.tri.get();
+  v.rec = ds_.rec.get();
+  v.pe_ref = ds_.pe_ref.get();
+  v.virial_ref = ds_.virial_ref.get();
+  v.force_ref = ds_.force_ref.get();
+
+  if (!tersoff) {
+    setup_quad();
+    if (!quad_.on) build_pair_tables();
+  }
+
+  potential_ = make_potential(spec_, ds_);
+  potential_->initialize(ts_.N, ts_.max_Na);
+  // this device's fixed workspace of the allocation-free path, looked up
+  // here (set-up) so that the path's calls only use the kept address
+  ws_static_ = static_workspace();
+  d_pmin_.upload(spec_.pmin, st);
+  d_pmax_.upload(spec_.pmax, st);
+  GPUGA_HIP(hipStreamSynchronize(st));
+  d_f_.resize(3 * (size_t)ts_.N);
+  d_virial_.resize(6 * (size_t)ts_.N);
+  d_pe_.resize(ts_.N);
+  d_cerr_.resize(3 * (size_t)ts_.Nc);
+  d_fit1_.resize(1);
+  d_terms1_.resize(3);
+}
+
+// The tables of the population kernel's pair loops, built on the host from
+// the bond geometry.
+void Fitness::build_pair_tables()
+{
+  if (pair_tables_) return;
+  hipStream_t st = stream_;
+  const std::vector<int>& ptype = ptype_;
+  std::vector<Vec4> bond(ds_.bond.size());
+  static_assert(sizeof(Vec4) == sizeof(float4), "layout");
+  ds_.bond.download(reinterpret_cast<float4*>(bond.data()), bond.size(), st);
   GPUGA_HIP(hipStreamSynchronize(st));
   // the pairs a pair potential evaluates for atom i: all its bonds in force
   // configurations (forces need both directions), j > i elsewhere (energy
@@ -370,18 +433,6 @@ void Fitness::setup()
     return off;
   };
   if (spec_.type == POT_RI) {
-    // per-bond factors of src/ri.cu:80-101 that do not depend on parameters
-    std::vector<float4> tab(std::max(nl_.total, 1));
-    parallel_for(ts_.N, [&](int i) {
-      for (int b = nl_.start[i]; b < nl_.start[i] + nl_.NN[i]; ++b) {
-        const double d = geo_.bond[b].w;
-        const double dinv = 1.0 / d;
-        const double e = std::erfc(0.2 * d) * dinv;
-        const double g = e * dinv + 0.225675833419103 * std::exp(-0.04 * d * d) * dinv;
-        tab[b] = make_float4((float)std::pow(dinv, 6), (float)e, (float)g, (float)dinv);
-      }
-    });
-    ds_.ri_tab.upload(tab, st);
     // population form: per atom the pairs it evaluates (all bonds for force
     // configurations, those with j > i for the others), grouped by pair type
     // t_i + t_j.  A force configuration's pair: unit vector and d (one
@@ -413,7 +464,7 @@ void Fitness::setup()
         for (int u = 0; u < nn; ++u) {
           const int b = b0 + u;
           if (ptype[b] != t || !evaluates(i, b)) continue;
-          const Vec4 r = geo_.bond[b];
+          const Vec4 r = bond[b];
           const double dinv = 1.0 / r.w;
           if (force) {
             *out++ = make_float4((float)(r.x * dinv), (float)(r.y * dinv), (float)(r.z * dinv), r.w);
@@ -445,7 +496,7 @@ void Fitness::setup()
       for (int i = ts_.Na_sum[c]; i < ts_.Na_sum[c] + ts_.Na[c]; ++i)
         for (int b = nl_.start[i]; b < nl_.start[i] + nl_.NN[i]; ++b) {
           if (!evaluates(i, b)) continue;
-          const Vec4 r = geo_.bond[b];
+          const Vec4 r = bond[b];
           const double d = r.w;
           double d6, f6, fc, h;
           factors(d, d6, f6, fc, h);
@@ -468,7 +519,7 @@ void Fitness::setup()
     parallel_for(ts_.N_force, [&](int i) {
       double o[kRiAtomConst] = {};
       for (int b = nl_.start[i]; b < nl_.start[i] + nl_.NN[i]; ++b) {
-        const Vec4 r = geo_.bond[b];
+        const Vec4 r = bond[b];
         const double d = r.w;
         double d6, f6, fc, h;
         factors(d, d6, f6, fc, h);
@@ -483,6 +534,7 @@ void Fitness::setup()
       for (int k = 0; k < kRiAtomConst; ++k) fcon[(size_t)i * kRiAtomConst + k] = (float)o[k];
     });
     ds_.ri_fconst.upload(fcon, st);
+    GPUGA_HIP(hipStreamSynchronize(st));
   }
   if (spec_.nn2b()) {
     // population form: per atom the pairs it evaluates (all bonds for force
@@ -513,12 +565,12 @@ void Fitness::setup()
       for (int u = 0; u < nn; ++u)
         if (evaluates(i, b0 + u)) order.push_back(b0 + u);
       std::stable_sort(order.begin(), order.end(),
-                       [&](int a, int b) { return geo_.bond[a].w < geo_.bond[b].w; });
+                       [&](int a, int b) { return bond[a].w < bond[b].w; });
       const long first = rows_before(i);
       hdr[i] = make_int4((int)first, (int)order.size(), 0, 0);
       float4* out = &pt[(size_t)first];
       for (int b : order) {
-        const Vec4 r = geo_.bond[b];
+        const Vec4 r = bond[b];
         const double d = r.w, dinv = 1.0 / d;
         const double u = (d - (double)grid.d0) / (double)grid.h;
         const int g = std::max(0, std::min((int)u, grid.G - 2));
@@ -550,51 +602,233 @@ void Fitness::setup()
     });
     ds_.pair_tab.upload(pt, st);
     ds_.pair_hdr.upload(hdr, st);
+    GPUGA_HIP(hipStreamSynchronize(st));
   }
-  ds_.pe_ref.upload(ts_.pe_ref, st);
-  ds_.virial_ref.upload(ts_.virial_ref, st);
-  ds_.force_ref.upload(ts_.force_ref, st);
-  GPUGA_HIP(hipStreamSynchronize(st));
-
   DevSet& v = ds_.view;
-  v.Nc = ts_.Nc;
-  v.Nc_force = ts_.Nc_force;
-  v.N = ts_.N;
-  v.N_force = ts_.N_force;
-  v.Na = ds_.Na.get();
-  v.Na_sum = ds_.Na_sum.get();
-  v.type = ds_.type.get();
-  v.nn = ds_.nn.get();
-  v.bond0 = ds_.bond0.get();
-  v.nl = ds_.nl.get();
-  v.rev = ds_.rev.get();
-  v.ptype = ds_.ptype.get();
-  v.bond = ds_.bond.get();
-  v.tri0 = ds_.tri0.get();
-  v.tri = ds_.tri.get();
-  v.rec = ds_.rec.get();
   v.pair_hdr = ds_.pair_hdr.get();
   v.pair_tab = ds_.pair_tab.get();
   v.ri_cconst = ds_.ri_cconst.get();
   v.ri_fconst = ds_.ri_fconst.get();
-  v.pe_ref = ds_.pe_ref.get();
-  v.virial_ref = ds_.virial_ref.get();
-  v.force_ref = ds_.force_ref.get();
+  pair_tables_ = true;
+}
 
-  potential_ = make_potential(spec_, ds_);
-  potential_->initialize(ts_.N, ts_.max_Na);
-  // this device's fixed workspace of the allocation-free path, looked up
-  // here (set-up) so that the path's calls only use the kept address
-  ws_static_ = static_workspace();
-  d_pmin_.upload(spec_.pmin, st);
-  d_pmax_.upload(spec_.pmax, st);
+int Fitness::quad_elements() const
+{
+  if (nl_.total == 0 || !(dmin_ > 0.0f) || !std::isfinite(dmax_)) return 0;
+  // (a label that is no number makes the sums so by itself: left to the pair
+  // loop, whose terms then are what they were)
+  for (const std::vector<float>* v : {&ts_.pe_ref, &ts_.virial_ref, &ts_.force_ref})
+    for (float x : *v)
+      if (!std::isfinite(x)) return 0;
+  if (spec_.nn2b()) {
+    // half as many nodes as the grid has points, in elements of 32: more
+    // accurate than the cubic interpolation on the whole grid from 256
+    // points on (fewer than 4 elements resolve a network worse than the
+    // grid's three values per point); the forms grow with the square of the
+    // nodes, so a grid finer than 2048 points (all codes together) stays with
+    // the pair loop
+    const int G = std::max(opt_.nn2b_grid, 16), codes = spec_.pair_codes();
+    if (G < 256 || G > 2048) return 0;
+    return codes * G > 4096 ? 0 : G / (2 * QB);
+  }
+  // Rigid ion: exponentials of known largest rate over genes in [0, 1].  An
+  // element of half length s / rate interpolates one to 2e-12 of its largest
+  // value at s = 16.
+  double rate = 0.0;
+  auto lo = [&](int v) { return (double)std::min(spec_.pmin[v], spec_.pmax[v]); };
+  auto hi = [&](int v) { return (double)std::max(spec_.pmin[v], spec_.pmax[v]); };
+  for (int v = 0; v < spec_.V; ++v)
+    if (!std::isfinite(lo(v)) || !std::isfinite(hi(v))) return 0;
+  for (int t = 0; t < 3; ++t) {
+    if (lo(1 + 3 * t) == 0.0 && hi(1 + 3 * t) == 0.0) continue;
+    if (!(lo(2 + 3 * t) > 0.0)) return 0;
+    rate = std::max(rate, 1.0 / lo(2 + 3 * t));
+  }
+  if (lo(11) != 0.0 || hi(11) != 0.0) {
+    const double alpha = std::max(std::fabs(lo(12)), std::fabs(hi(12)));
+    if (!(lo(14) > 0.0)) return 0;
+    rate = std::max({rate, std::sqrt(2.0 * hi(14)) * alpha, std::sqrt(2.0 / lo(14)) * alpha});
+  }
+  const double e = std::ceil(0.5 * (dmax_ - dmin_) * rate / 16.0);
+  return e <= 8.0 ? std::max(1, (int)e) : 0;
+}
+
+void Fitness::setup_quad()
+{
+  const int E = quad_elements();
+  if (E == 0) return;
+  hipStream_t st = stream_;
+  QuadBasis b;
+  b.rigid = spec_.type == POT_RI ? 1 : 0;
+  b.codes = b.rigid ? 3 : spec_.pair_codes();
+  b.E = E;
+  b.d0 = dmin_;
+  b.len = std::max((double)dmax_ - (double)dmin_, 1e-3) / E;
+  const int CE = b.CE();
+  // the elements that the pairs of energy and of force configurations use
+  DeviceBuffer<int> d_used;
+  std::vector<int> used((size_t)4 * CE, 0);
+  d_used.upload(used, st);
+  launch_quad_used(ds_.view, b, d_used.get(), st);
+  d_used.download(used.data(), used.size(), st);
   GPUGA_HIP(hipStreamSynchronize(st));
-  d_f_.resize(3 * (size_t)ts_.N);
-  d_virial_.resize(6 * (size_t)ts_.N);
-  d_pe_.resize(ts_.N);
-  d_cerr_.resize(3 * (size_t)ts_.Nc);
-  d_fit1_.resize(1);
-  d_terms1_.resize(3);
+  // column blocks of each form and their value blocks; U' enters the virials
+  // and forces (U only inside NN2B's taper), U the energies
+  std::vector<int> col((size_t)6 * CE, -1), act;
+  std::vector<int2> vblk[3];
+  int nb[3];
+  // (the columns of the species codes above 0 hold differences from code 0's)
+  auto value = [&](int first, int ce) {
+    return make_int2(first + ce, b.species() && ce >= E ? first + ce % E : -1);
+  };
+  for (int f = 0; f < 3; ++f) {
+    const int* u = &used[f == 2 ? (size_t)2 * CE : 0];
+    vblk[f].push_back(make_int2(2 * CE, -1));
+    auto add = [&](int map, int first, const int* used, int ce0, int ce1) {
+      for (int ce = ce0; ce < ce1; ++ce)
+        if (used[ce]) {
+          col[(size_t)map * CE + ce] = (int)vblk[f].size();
+          vblk[f].push_back(value(first, ce));
+        }
+    };
+    // code 0's columns before the differences (rigid ion: no differences)
+    const int n0 = b.species() ? E : CE;
+    for (int part = 0; part < 2; ++part) {
+      const int ce0 = part ? n0 : 0, ce1 = part ? CE : n0;
+      add(f == 0 ? 0 : 3 + f, f == 0 ? 0 : CE, u, ce0, ce1);
+      if (f > 0) add(f, 0, u + CE, ce0, ce1);
+    }
+    nb[f] = (int)vblk[f].size();
+  }
+  for (int ce = 0; ce < CE; ++ce)
+    if (used[ce] || used[2 * CE + ce]) act.push_back(ce);
+  QuadRows rows;
+  DeviceBuffer<int> d_col;
+  d_col.upload(col, st);
+  rows.b = b;
+  rows.col = d_col.get();
+  for (int f = 0; f < 3; ++f) rows.nb[f] = nb[f];
+  if (quad_energy_lds(rows) > 156u * 1024u) return;
+  quad_prepare(rows);
+  quad_.basis = b;
+  quad_.n_act = (int)act.size();
+  quad_.act.upload(act, st);
+  // Rows in chunks of configurations and force atoms, the Gram products
+  // accumulated over the chunks.  Chunks and the split of a chunk's rows over
+  // waves do not depend on the columns, so a column's sums do not depend on
+  // which others the form has.
+  constexpr int kConfigs = 512, kAtoms = 2048, kSplits = 16;
+  DeviceBuffer<double> R, part;
+  auto finish = [&](int f, const double* p) {
+    quad_.nb[f] = nb[f];
+    quad_.q[f].resize((size_t)quad_tiles(nb[f]) * QB * QB);
+    quad_.vblk[f].upload(vblk[f], st);
+    launch_quad_finish(p, nb[f], kSplits, quad_.q[f].get(), st);
+  };
+  auto part_size = [&](int f) { return (size_t)kSplits * quad_tiles(nb[f]) * QB * QB; };
+  auto pad4 = [](int n) { return (std::max(n, 1) + 3) / 4 * 4; };
+  { // energy and virial rows
+    const int ne = ts_.Nc - ts_.Nc_force, step = std::min(kConfigs, pad4(ne));
+    const size_t D0 = rows.D(0), D1 = rows.D(1);
+    R.resize(step * (D0 + 6 * D1));
+    part.resize(part_size(0) + part_size(1));
+    double *re = R.get(), *rw = re + step * D0, *pw = part.get() + part_size(0);
+    for (int c0 = 0; c0 < std::max(ne, 1); c0 += step) {
+      const int n = std::min(step, ne - c0), n4 = pad4(n), c = ts_.Nc_force + c0;
+      R.zero(st);
+      if (n > 0) launch_quad_energy_rows(ds_.view, rows, c, c + n, re, rw, st);
+      launch_quad_gram(re, n4, nb[0], kSplits, c0 == 0, part.get(), st);
+      launch_quad_gram(rw, 6 * n4, nb[1], kSplits, c0 == 0, pw, st);
+    }
+    finish(0, part.get());
+    finish(1, pw);
+  }
+  GPUGA_HIP(hipStreamSynchronize(st));
+  { // force rows
+    const int na = ts_.N_force, step = std::min(kAtoms, pad4(na));
+    R.resize((size_t)step * 3 * rows.D(2));
+    part.resize(part_size(2));
+    for (int i0 = 0; i0 < std::max(na, 1); i0 += step) {
+      const int n = std::min(step, na - i0);
+      R.zero(st);
+      if (n > 0) launch_quad_force_rows(ds_.view, rows, i0, i0 + n, R.get(), st);
+      launch_quad_gram(R.get(), 3 * pad4(n), nb[2], kSplits, i0 == 0, part.get(), st);
+    }
+    finish(2, part.get());
+  }
+  GPUGA_HIP(hipStreamSynchronize(st));
+  quad_.on = true;
+}
+
+bool Fitness::quad_for(int P, const float* genes) const
+{
+  if (!quad_.on) return false;
+  if (spec_.nn2b()) return true; // (the distances alone set its elements)
+  for (size_t k = 0; k < (size_t)P * spec_.V; ++k)
+    if (!(genes[k] >= 0.0f && genes[k] <= 1.0f)) return false;
+  return true;
+}
+
+void Fitness::build_quad_plan(PopPlan& pl, int P)
+{
+  hipStream_t st = stream_;
+  pl.P = P;
+  pl.K = (P + WAVE - 1) / WAVE;
+  const size_t out_doubles = 3 * (size_t)P + ((size_t)P + 1 + 1) / 2;
+  pl.out.resize(out_doubles);
+  pl.out.zero(st);
+  pl.genes.resize((size_t)P * spec_.V);
+  pl.h_genes.resize((size_t)P * spec_.V);
+  pl.h_out.resize(out_doubles);
+  std::memset(pl.h_out.get(), 0, sizeof(double) * out_doubles);
+  PopCtl& c = pl.ctl;
+  c.K = pl.K;
+  c.P = P;
+  c.V = spec_.V;
+  c.genes = pl.genes.get();
+  c.pmin = d_pmin_.get();
+  c.pmax = d_pmax_.get();
+  c.terms = pl.out.get();
+  c.fitness = reinterpret_cast<float*>(c.terms + 3 * (size_t)P);
+  c.status = reinterpret_cast<unsigned*>(c.fitness + P);
+  c.norm = norm();
+  const int ld = (P + QP - 1) / QP * QP;
+  // (the linear block: zeros and the constant 1, the parameters written by
+  // each launch)
+  const size_t block = (size_t)QB * ld, lin = (size_t)2 * quad_.basis.CE() * block;
+  std::vector<double> ones(ld, 1.0);
+  pl.qvalues.resize(lin + block);
+  pl.qvalues.zero(st);
+  GPUGA_HIP(hipMemcpyAsync(pl.qvalues.get() + lin + (size_t)kQuadOne * ld, ones.data(),
+                           sizeof(double) * ld, hipMemcpyHostToDevice, st));
+  pl.qpart.resize((size_t)quad_.units() * ld);
+  pl.qdone.resize(ld / QP);
+  pl.qdone.zero(st);
+  QuadEval& q = pl.qeval;
+  for (int f = 0; f < 3; ++f)
+    q.form[f] = QuadForm{quad_.nb[f], quad_.vblk[f].get(), quad_.q[f].get()};
+  q.values = pl.qvalues.get();
+  q.ld = ld;
+  q.part = pl.qpart.get();
+  q.done = pl.qdone.get();
+  pl.qnodes = NodeTable{quad_.basis, quad_.act.get(), quad_.n_act, pl.qvalues.get(), ld};
+  GPUGA_HIP(hipStreamSynchronize(st));
+}
+
+void Fitness::ensure_items(PopPlan& pl)
+{
+  if (pl.items_built) return;
+  build_pair_tables();
+  build_plan(pl, pl.P, launch_shape(pl.P));
+}
+
+void Fitness::launch_quad(PopPlan& pl, hipStream_t st, const float* genes)
+{
+  PopCtl ctl = pl.ctl;
+  if (genes) ctl.genes = genes;
+  if (quad_.basis.rigid) launch_ri_values(ctl, pl.qnodes, st);
+  else launch_nn2b_nodes(ctl, nn2b_grid_desc(), pl.qnodes, st);
+  launch_quad_eval(ctl, pl.qeval, st);
 }
 
 NN2BGrid Fitness::nn2b_grid_desc() const
@@ -625,9 +859,10 @@ FitnessNorm Fitness::norm() const
 
 size_t Fitness::device_bytes() const
 {
-  size_t b = ds_.bytes() + d_f_.bytes() + d_virial_.bytes() + d_pe_.bytes() + d_cerr_.bytes();
+  size_t b = ds_.bytes() + quad_.bytes() + d_f_.bytes() + d_virial_.bytes() + d_pe_.bytes() + d_cerr_.bytes();
   for (auto& kv : plans_) {
     const PopPlan& p = *kv.second;
+    b += p.qvalues.bytes() + p.qpart.bytes();
     b += p.items.bytes() + p.part.bytes() + p.err.bytes() + p.bondf.bytes() + p.genes.bytes() +
          p.out.bytes() + p.gpart.bytes() + p.counters.bytes() + p.nn2b_table.bytes();
   }
@@ -990,6 +1225,7 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   c.spin_limit = spin_limit_;
   c.norm = norm();
   GPUGA_HIP(hipStreamSynchronize(st));
+  pl.items_built = true;
 }
 
 } // namespace gpuga
@@ -1001,7 +1237,8 @@ PopPlan& Fitness::plan(int P)
   auto it = plans_.find(P);
   if (it != plans_.end()) return *it->second;
   auto pl = std::make_unique<PopPlan>();
-  build_plan(*pl, P, launch_shape(P));
+  if (quad_.on) build_quad_plan(*pl, P);
+  else build_plan(*pl, P, launch_shape(P));
   PopPlan& ref = *pl;
   plans_[P] = std::move(pl);
   return ref;
@@ -1056,8 +1293,13 @@ void Fitness::compute_async(int P, const float* genes, int share)
   std::memcpy(pl.h_genes.get(), genes, sizeof(float) * (size_t)P * spec_.V);
   GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), pl.h_genes.get(), sizeof(float) * (size_t)P * spec_.V,
                            hipMemcpyHostToDevice, st));
+  // (a set with quadratic forms, genes outside their range: the pair loop,
+  // launched directly)
+  const bool direct = quad_.on && !quad_for(P, genes);
+  if (direct) ensure_items(pl);
   if (timing_) GPUGA_HIP(hipEventRecord(ev0_, st));
-  launch_generation(pl, st, share);
+  if (direct) launch_population(pl, st);
+  else launch_generation(pl, st, share);
   if (timing_) GPUGA_HIP(hipEventRecord(ev1_, st));
   GPUGA_HIP(hipMemcpyAsync(pl.h_out.get(), pl.out.get(),
                            sizeof(double) * 3 * P + sizeof(float) * P + sizeof(unsigned),
@@ -1093,9 +1335,15 @@ void captured(hipStream_t st, F&& body, hipGraph_t* graph, hipGraphExec_t* exec)
 
 void Fitness::launch_generation(PopPlan& pl, hipStream_t st, int share)
 {
-  // share 1, 2, 4 or 8 (rounded up, at most 8): 1/share of the grid
+  // share 1, 2, 4 or 8 (rounded up, at most 8): 1/share of the grid (the
+  // quadratic forms' launches are short and fill a part of the GPU by
+  // themselves)
   int j = 0;
-  while (j < PopPlan::kShares && (1 << j) < share) ++j;
+  while (!quad_.on && j < PopPlan::kShares && (1 << j) < share) ++j;
+  if (quad_.on && !opt_.use_graph) {
+    launch_quad(pl, st);
+    return;
+  }
   const int grid = std::max(1, (pl.grid + (1 << j) - 1) >> j);
   if (!opt_.use_graph) {
     launch_population(pl, st, nullptr, grid);
@@ -1115,7 +1363,10 @@ void Fitness::launch_generation(PopPlan& pl, hipStream_t st, int share)
 void Fitness::capture(PopPlan& pl, hipStream_t st)
 {
   if (pl.exec) return;
-  captured(st, [&] { launch_population(pl, st); }, &pl.graph, &pl.exec);
+  captured(st, [&] {
+    if (quad_.on) launch_quad(pl, st);
+    else launch_population(pl, st);
+  }, &pl.graph, &pl.exec);
 }
 
 void Fitness::prepare(int P)
@@ -1134,7 +1385,8 @@ void Fitness::capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph,
   captured(st, [&] {
     for (int i = 0; i < n; ++i) {
       const int b = (k + i) & 1;
-      launch_population(pl, st, pl.dga->genes(b));
+      if (pl.ga_quad) launch_quad(pl, st, pl.dga->genes(b));
+      else launch_population(pl, st, pl.dga->genes(b));
       pl.dga->step(b, pl.ctl.fitness, st);
     }
   }, graph, exec);
@@ -1154,6 +1406,11 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
   check_genes(P, ga.population().data());
   PopPlan& pl = plan(P);
   hipStream_t st = stream_;
+  // (crossover and mutation keep genes in [0, 1]: one look at the start)
+  const bool quad = quad_for(P, ga.population().data());
+  if (!quad) ensure_items(pl);
+  if (pl.ga_quad != quad) pl.drop_ga_graphs();
+  pl.ga_quad = quad;
   // the GA as it was before this call: staging draws advances its random
   // stream, so a failed run restores it
   const GA before = ga;
@@ -1190,7 +1447,8 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
       for (int i = 0; i < nb;) {
         const int k = (g + b + i) & 1;
         if (!opt_.use_graph) {
-          launch_population(pl, st, dga.genes(k));
+          if (quad) launch_quad(pl, st, dga.genes(k));
+          else launch_population(pl, st, dga.genes(k));
           dga.step(k, pl.ctl.fitness, st);
           ++i;
           continue;
@@ -1472,6 +1730,13 @@ size_t Fitness::estimate_bytes(const PotentialSpec& s, const TrainSet& ts, int P
   b += K * 3 * Nc * WAVE * sizeof(double) + 2 * Nc * K * 8 * WAVE * sizeof(double);
   if (tersoff) b += K * (B_force + ts.N_force) * 3 * WAVE * sizeof(float);
   if (s.nn2b()) b += (size_t)3 * s.pair_codes() * opt.nn2b_grid * K * WAVE * sizeof(float);
+  if (!tersoff) {
+    // quadratic forms: value blocks of the population and the three forms
+    // (rigid ion: at most 8 elements per type)
+    const size_t ce = s.nn2b() ? s.pair_codes() * (size_t)std::max(opt.nn2b_grid, 64) / (2 * QB) : 24;
+    b += (2 * ce + 1) * QB * sizeof(double) * (size_t)(P + QP);
+    b += 3 * quad_tiles(s.nn2b() ? 2 * ce + 1 : ce + 1) * QB * QB * sizeof(double);
+  }
   b += (size_t)P * s.V * sizeof(float) + (size_t)P * 4 * sizeof(double);
   return b;
 }
@@ -1480,6 +1745,7 @@ std::vector<double> Fitness::trace(int P, const float* genes)
 {
   check_genes(P, genes);
   PopPlan& pl = plan(P);
+  ensure_items(pl);
   hipStream_t st = stream_;
   const size_t n = pl.n_items;
   const size_t F = kTraceFields;
@@ -1552,7 +1818,8 @@ void Fitness::plan_shape(int P, int& chunk_cost, int& queues, int& blocks_per_cu
                          int& groups_last)
 {
   if (P < 1) fail("population size must be positive");
-  const PopPlan& pl = plan(P);
+  PopPlan& pl = plan(P);
+  ensure_items(pl);
   chunk_cost = pl.chunk_cost;
   queues = pl.nq;
   blocks_per_cu = pl.occ;
@@ -1570,6 +1837,14 @@ int Fitness::autotune(int P)
   // lane block qualifies, packing it or not.  Each choice is kept only if
   // its launch is faster.
   const bool tersoff = spec_.type == POT_TERSOFF1 || spec_.type == POT_TERSOFF2;
+  if (quad_.on) {
+    // nothing to tune: the population kernel only serves a trace, or genes
+    // outside [0, 1]
+    LaunchShape sh = option_shape();
+    sh.chunk_cost = heuristic_chunk_cost(P);
+    tuned_[P] = sh;
+    return sh.chunk_cost;
+  }
   const std::vector<int>& pnn = tersoff ? population_neighbors().NN : nl_.NN;
   long long total = 0, maxcfg = 0;
   for (int c = 0; c < ts_.Nc; ++c) {

@@ -11,6 +11,7 @@
 #include "ga.h"
 #include "ga_device.h"
 #include "kernels.h"
+#include "quadform.h"
 #include "trainset.h"
 
 namespace gpuga {
@@ -76,8 +77,30 @@ public:
 
 std::unique_ptr<Potential> make_potential(const PotentialSpec& spec, const DeviceSet& ds);
 
+// A pair potential's training set as quadratic forms (quadform.h).
+struct QuadSet {
+  bool on = false;
+  QuadBasis basis{};
+  int nb[3] = {0, 0, 0}; // column blocks of the energy, virial and force form
+  int n_act = 0;
+  DeviceBuffer<double> q[3];
+  DeviceBuffer<int2> vblk[3];
+  DeviceBuffer<int> act;
+  size_t bytes() const
+  {
+    return q[0].bytes() + q[1].bytes() + q[2].bytes() + act.bytes();
+  }
+  int units() const { return nb[0] + nb[1] + nb[2]; }
+};
+
 // One population plan (work items, scratch) for a population size P.
 struct PopPlan {
+  bool items_built = false; // the work items of the population kernel are there
+  DeviceBuffer<double> qvalues, qpart; // quadratic forms: values, row-block sums
+  DeviceBuffer<unsigned> qdone;
+  QuadEval qeval{};
+  NodeTable qnodes{};
+  bool ga_quad = false; // the GA graphs run the quadratic forms
   int P = 0, K = 0, n_items = 0, grid = 0, block = 256, chunk_cost = 0;
   int occ = 0;         // resident workgroups per CU the grid is sized for
   int groups_last = 1; // lane groups of the last lane block's items
@@ -193,6 +216,19 @@ public:
 
 private:
   void setup();
+  // Quadratic forms of a pair potential's set, when the rule of
+  // quad_elements() takes it.
+  void setup_quad();
+  // Elements of the distance range per pair code for the quadratic forms; 0
+  // when the population kernel's pair loop serves the set.
+  int quad_elements() const;
+  // the population kernel's pair tables (built with the set, or when a call
+  // of a set with quadratic forms first needs them)
+  void build_pair_tables();
+  void ensure_items(PopPlan& pl);
+  void build_quad_plan(PopPlan& pl, int P);
+  // whether genes [P][V] are evaluated by the quadratic forms
+  bool quad_for(int P, const float* genes) const;
   PopPlan& plan(int P);
   void build_plan(PopPlan& pl, int P, const LaunchShape& sh);
   // the shape the options fix (chunk cost > 0: no tuning)
@@ -200,6 +236,8 @@ private:
   // the population launch on genes (default: the plan's buffer)
   void launch_population(PopPlan& pl, hipStream_t st, const float* genes = nullptr,
                          int grid = 0);
+  // the same by the quadratic forms
+  void launch_quad(PopPlan& pl, hipStream_t st, const float* genes = nullptr);
   // n generations of the device GA from population buffer k, captured
   void capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph, hipGraphExec_t* exec);
   void launch_generation(PopPlan& pl, hipStream_t st, int share = 1); // graph or direct
@@ -231,7 +269,9 @@ private:
   bool pruned_ = false; // pnl_ holds fewer bonds than nl_
   bool loop_path_ = false; // Tersoff: more than 16 neighbours within R2
   LoopTab loop_{};         // the looped kernel's tables
-  Geometry geo_; // host bond geometry of the pair potentials' set-up
+  std::vector<int> ptype_; // pair type per bond
+  bool pair_tables_ = false;
+  QuadSet quad_;
   DeviceSet ds_;
   std::unique_ptr<Potential> potential_;
   std::map<int, std::unique_ptr<PopPlan>> plans_;

@@ -208,14 +208,13 @@ __device__ inline void sum_rows(const double* const (&a)[NA], long stride, int n
   for (int x = 0; x < NA; ++x) out[x] = (s[x][0] + s[x][1]) + (s[x][2] + s[x][3]);
 }
 
-// Fitness and terms of the lane block's individuals from the sums of the
-// three error terms over all configurations.
-__device__ inline void write_fitness(const PopCtl& ctl, int k, int lane, const double (&s)[3])
+// Fitness and terms of individual p (nothing past the population) from the
+// sums of the three error terms over all configurations.
+__device__ inline void write_fitness(const PopCtl& ctl, int p, const double (&s)[3])
 {
   const double tE = sqrt(s[0] * ctl.norm.inv_pss);
   const double tW = sqrt(s[1] * ctl.norm.inv_vss);
   const double tF = sqrt(s[2] * ctl.norm.inv_fss);
-  const int p = k * WAVE + lane;
   if (p < ctl.P) {
     ctl.fitness[p] =
       (float)(ctl.norm.w_energy * tE + ctl.norm.w_stress * tW + ctl.norm.w_force * tF);
@@ -261,7 +260,7 @@ __device__ inline bool config_done(const PopCtl& ctl, int Nc, int Nc_force, int 
   sum_rows<2, VALS>(ee, WAVE, g0 + gn - fe, s);
   s[2] = f[0];
   if (groups == 1) {
-    write_fitness(ctl, k, lane, s);
+    write_fitness(ctl, k * WAVE + lane, s);
     return true;
   }
   double* gp = ctl.gpart + ((long)k * groups + g) * 3 * WAVE + lane;
@@ -276,7 +275,7 @@ __device__ inline bool config_done(const PopCtl& ctl, int Nc, int Nc_force, int 
   const double* gb = ctl.gpart + (long)k * groups * 3 * WAVE + lane;
   const double* const eg[3] = {gb, gb + WAVE, gb + 2 * WAVE};
   sum_rows<3, VALS>(eg, 3 * WAVE, groups, s);
-  write_fitness(ctl, k, lane, s);
+  write_fitness(ctl, k * WAVE + lane, s);
   return true;
 }
 
