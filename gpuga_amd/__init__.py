@@ -75,8 +75,8 @@ def lib():
             "gpuga_fitness_bounds": (C.c_int, [vp, fp, fp]),
             "gpuga_fitness_info": (C.c_int, [vp, ip]),
             "gpuga_fitness_compute": (C.c_int, [vp, C.c_int, fp, fp]),
-            "gpuga_fitness_compute_terms": (C.c_int, [vp, C.c_int, fp, fp, dp]),
-            "gpuga_fitness_compute_plain": (C.c_int, [vp, C.c_int, fp, fp, dp]),
+            "gpuga_fitness_compute_terms": (C.c_int, [vp, C.c_int, vp, vp, vp]),
+            "gpuga_fitness_compute_plain": (C.c_int, [vp, C.c_int, vp, vp, vp]),
             "gpuga_fitness_compute_plain_noalloc": (C.c_int, [vp, C.c_int, fp, fp, dp]),
             "gpuga_fitness_predict": (C.c_int, [vp, C.c_char_p, fp]),
             "gpuga_fitness_find_force": (C.c_int, [vp, fp, fp, fp, fp]),
@@ -194,14 +194,10 @@ class Fitness:
     def compute(self, genes, *, terms=False, plain=False):
         g = _f32(genes).reshape(-1, self.V)
         P = g.shape[0]
-        fit = np.zeros(P, np.float32)
-        t = np.zeros((P, 3), np.float64)
-        if plain:
-            _check(lib().gpuga_fitness_compute_plain(self._h, P, _ptr(g), _ptr(fit),
-                                                     _ptr(t, C.c_double)))
-        else:
-            _check(lib().gpuga_fitness_compute_terms(self._h, P, _ptr(g), _ptr(fit),
-                                                     _ptr(t, C.c_double)))
+        fit = np.empty(P, np.float32)
+        t = np.empty((P, 3), np.float64) if terms else None
+        fn = lib().gpuga_fitness_compute_plain if plain else lib().gpuga_fitness_compute_terms
+        _check(fn(self._h, P, g.ctypes.data, fit.ctypes.data, t.ctypes.data if terms else None))
         return (fit, t) if terms else fit
 
     def denormalise(self, genes):
@@ -212,9 +208,9 @@ class Fitness:
 
     def find_force(self, params):
         p = _f32(params)
-        f = np.zeros(3 * self.N, np.float32)
-        w = np.zeros(6 * self.N, np.float32)
-        e = np.zeros(self.N, np.float32)
+        f = np.empty(3 * self.N, np.float32)
+        w = np.empty(6 * self.N, np.float32)
+        e = np.empty(self.N, np.float32)
         _check(lib().gpuga_fitness_find_force(self._h, _ptr(p), _ptr(f), _ptr(w), _ptr(e)))
         return f, w, e
 

@@ -152,23 +152,7 @@ void PopPlan::drop_ga_graphs()
     }
 }
 
-void PopPlan::drop_share_graphs()
-{
-  for (int j = 0; j < kShares; ++j) {
-    if (share_exec[j]) (void)hipGraphExecDestroy(share_exec[j]);
-    if (share_graph[j]) (void)hipGraphDestroy(share_graph[j]);
-    share_exec[j] = nullptr;
-    share_graph[j] = nullptr;
-  }
-}
-
-PopPlan::~PopPlan()
-{
-  drop_share_graphs();
-  drop_ga_graphs();
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-}
+PopPlan::~PopPlan() { drop_ga_graphs(); }
 
 // ------------------------------------------------------------ set-up
 
@@ -190,6 +174,7 @@ Fitness::~Fitness()
   plans_.clear();
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
+  if (ev_copy_) (void)hipEventDestroy(ev_copy_);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -217,6 +202,7 @@ void Fitness::setup()
   GPUGA_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
   GPUGA_HIP(hipEventCreate(&ev0_));
   GPUGA_HIP(hipEventCreate(&ev1_));
+  GPUGA_HIP(hipEventCreateWithFlags(&ev_copy_, hipEventDisableTiming));
 
   const bool tersoff = spec_.type == POT_TERSOFF1 || spec_.type == POT_TERSOFF2;
   if (spec_.type == POT_RI || spec_.type == POT_NN2B_SPECIES)
@@ -822,10 +808,8 @@ void Fitness::ensure_items(PopPlan& pl)
   build_plan(pl, pl.P, launch_shape(pl.P));
 }
 
-void Fitness::launch_quad(PopPlan& pl, hipStream_t st, const float* genes)
+void Fitness::launch_quad(PopPlan& pl, const PopCtl& ctl, hipStream_t st)
 {
-  PopCtl ctl = pl.ctl;
-  if (genes) ctl.genes = genes;
   if (quad_.basis.rigid) launch_ri_values(ctl, pl.qnodes, st);
   else launch_nn2b_nodes(ctl, nn2b_grid_desc(), pl.qnodes, st);
   launch_quad_eval(ctl, pl.qeval, st);
@@ -1244,10 +1228,8 @@ PopPlan& Fitness::plan(int P)
   return ref;
 }
 
-void Fitness::launch_population(PopPlan& pl, hipStream_t st, const float* genes, int grid)
+void Fitness::launch_population(PopPlan& pl, const PopCtl& ctl, hipStream_t st, int grid)
 {
-  PopCtl ctl = pl.ctl;
-  if (genes) ctl.genes = genes;
   // (a persistent grid of any size drains the same queues; the results do
   // not depend on it)
   const int G = grid > 0 ? grid : pl.grid;
@@ -1290,20 +1272,40 @@ void Fitness::compute_async(int P, const float* genes, int share)
   check_genes(P, genes);
   PopPlan& pl = plan(P);
   hipStream_t st = stream_;
-  std::memcpy(pl.h_genes.get(), genes, sizeof(float) * (size_t)P * spec_.V);
-  GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), pl.h_genes.get(), sizeof(float) * (size_t)P * spec_.V,
-                           hipMemcpyHostToDevice, st));
-  // (a set with quadratic forms, genes outside their range: the pair loop,
-  // launched directly)
-  const bool direct = quad_.on && !quad_for(P, genes);
-  if (direct) ensure_items(pl);
+  // (a set with quadratic forms, genes outside their range: the pair loop)
+  const bool quad = quad_for(P, genes);
+  if (!quad) ensure_items(pl);
+  const size_t bytes = sizeof(float) * (size_t)P * spec_.V;
+  std::memcpy(pl.h_genes.get(), genes, bytes);
+  // The generation is launched directly (a graph of one or two kernels takes
+  // 14 us longer to launch and wait for), and its last kernel writes the
+  // results to the pinned block: a copy back would be one more operation on
+  // the stream.
+  PopCtl ctl = pl.ctl;
+  ctl.terms = pl.h_out.get();
+  ctl.fitness = reinterpret_cast<float*>(ctl.terms + 3 * (size_t)P);
+  ctl.status = reinterpret_cast<unsigned*>(ctl.fitness + P);
+  *ctl.status = 0u;
+  if (quad && quad_.basis.rigid) {
+    ctl.genes = pl.h_genes.get(); // (each value is read a few times)
+  } else {
+    // up to 64 KiB by a kernel: its launch costs less than a copy's
+    if (bytes <= 64u * 1024u) launch_copy_in(pl.h_genes.get(), pl.genes.get(), P * spec_.V, st);
+    else
+      GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), pl.h_genes.get(), bytes, hipMemcpyHostToDevice, st));
+  }
   if (timing_) GPUGA_HIP(hipEventRecord(ev0_, st));
-  if (direct) launch_population(pl, st);
-  else launch_generation(pl, st, share);
+  if (quad) {
+    launch_quad(pl, ctl, st);
+  } else {
+    // share 1, 2, 4 or 8 (rounded up, at most 8): 1/share of the grid (the
+    // quadratic forms' launches are short and fill a part of the GPU by
+    // themselves)
+    int j = 0;
+    while (j < 3 && (1 << j) < share) ++j;
+    launch_population(pl, ctl, st, std::max(1, (pl.grid + (1 << j) - 1) >> j));
+  }
   if (timing_) GPUGA_HIP(hipEventRecord(ev1_, st));
-  GPUGA_HIP(hipMemcpyAsync(pl.h_out.get(), pl.out.get(),
-                           sizeof(double) * 3 * P + sizeof(float) * P + sizeof(unsigned),
-                           hipMemcpyDeviceToHost, st));
   pending_P_ = P;
 }
 
@@ -1333,47 +1335,9 @@ void captured(hipStream_t st, F&& body, hipGraph_t* graph, hipGraphExec_t* exec)
 
 } // namespace
 
-void Fitness::launch_generation(PopPlan& pl, hipStream_t st, int share)
-{
-  // share 1, 2, 4 or 8 (rounded up, at most 8): 1/share of the grid (the
-  // quadratic forms' launches are short and fill a part of the GPU by
-  // themselves)
-  int j = 0;
-  while (!quad_.on && j < PopPlan::kShares && (1 << j) < share) ++j;
-  if (quad_.on && !opt_.use_graph) {
-    launch_quad(pl, st);
-    return;
-  }
-  const int grid = std::max(1, (pl.grid + (1 << j) - 1) >> j);
-  if (!opt_.use_graph) {
-    launch_population(pl, st, nullptr, grid);
-    return;
-  }
-  if (j == 0) {
-    capture(pl, st);
-    GPUGA_HIP(hipGraphLaunch(pl.exec, st));
-    return;
-  }
-  if (!pl.share_exec[j - 1])
-    captured(st, [&] { launch_population(pl, st, nullptr, grid); }, &pl.share_graph[j - 1],
-             &pl.share_exec[j - 1]);
-  GPUGA_HIP(hipGraphLaunch(pl.share_exec[j - 1], st));
-}
-
-void Fitness::capture(PopPlan& pl, hipStream_t st)
-{
-  if (pl.exec) return;
-  captured(st, [&] {
-    if (quad_.on) launch_quad(pl, st);
-    else launch_population(pl, st);
-  }, &pl.graph, &pl.exec);
-}
-
 void Fitness::prepare(int P)
 {
-  if (opt_.backend == 1) return;
-  PopPlan& pl = plan(P);
-  if (opt_.use_graph) capture(pl, stream_);
+  if (opt_.backend != 1) plan(P);
 }
 
 static_assert((1 << (PopPlan::kGaGraphs - 1)) >= kGaMaxBatch, "a batch fits the largest graph");
@@ -1385,8 +1349,10 @@ void Fitness::capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph,
   captured(st, [&] {
     for (int i = 0; i < n; ++i) {
       const int b = (k + i) & 1;
-      if (pl.ga_quad) launch_quad(pl, st, pl.dga->genes(b));
-      else launch_population(pl, st, pl.dga->genes(b));
+      PopCtl ctl = pl.ctl;
+      ctl.genes = pl.dga->genes(b);
+      if (pl.ga_quad) launch_quad(pl, ctl, st);
+      else launch_population(pl, ctl, st);
       pl.dga->step(b, pl.ctl.fitness, st);
     }
   }, graph, exec);
@@ -1447,8 +1413,10 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
       for (int i = 0; i < nb;) {
         const int k = (g + b + i) & 1;
         if (!opt_.use_graph) {
-          if (quad) launch_quad(pl, st, dga.genes(k));
-          else launch_population(pl, st, dga.genes(k));
+          PopCtl ctl = pl.ctl;
+          ctl.genes = dga.genes(k);
+          if (quad) launch_quad(pl, ctl, st);
+          else launch_population(pl, ctl, st);
           dga.step(k, pl.ctl.fitness, st);
           ++i;
           continue;
@@ -1512,11 +1480,6 @@ void Fitness::set_spin_limit(int spins)
     pl.ctl.spin_limit = spins;
     // the captured launches hold the old control block
     pl.drop_ga_graphs();
-    pl.drop_share_graphs();
-    if (pl.exec) (void)hipGraphExecDestroy(pl.exec);
-    if (pl.graph) (void)hipGraphDestroy(pl.graph);
-    pl.exec = nullptr;
-    pl.graph = nullptr;
   }
 }
 
@@ -1636,10 +1599,21 @@ void Fitness::find_force(const float* physical, float* f, float* virial, float* 
   hipStream_t st = stream_;
   potential_->find_force(ds_.view, d_f_.get(), d_virial_.get(), d_pe_.get(), st);
   GPUGA_HIP(hipGetLastError());
-  if (f) d_f_.download(f, 3 * (size_t)ts_.N, st);
-  if (virial) d_virial_.download(virial, 6 * (size_t)ts_.N, st);
-  if (pe) d_pe_.download(pe, ts_.N, st);
+  // through a pinned block, energy and force to the caller while the virial
+  // is still on its way (a copy into pageable memory runs at a sixth of the
+  // pinned rate)
+  const size_t N = ts_.N;
+  h_atoms_.resize(10 * N);
+  float *he = h_atoms_.get(), *hf = he + N, *hw = hf + 3 * N;
+  if (pe) d_pe_.download(he, N, st);
+  if (f) d_f_.download(hf, 3 * N, st);
+  GPUGA_HIP(hipEventRecord(ev_copy_, st));
+  if (virial) d_virial_.download(hw, 6 * N, st);
+  GPUGA_HIP(hipEventSynchronize(ev_copy_));
+  if (pe) std::memcpy(pe, he, sizeof(float) * N);
+  if (f) std::memcpy(f, hf, sizeof(float) * 3 * N);
   GPUGA_HIP(hipStreamSynchronize(st));
+  if (virial) std::memcpy(virial, hw, sizeof(float) * 6 * N);
 }
 
 void Fitness::predict(const std::string& dir, const float* elite)
@@ -1756,7 +1730,7 @@ std::vector<double> Fitness::trace(int P, const float* genes)
   GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), genes, sizeof(float) * (size_t)P * spec_.V,
                            hipMemcpyHostToDevice, st));
   pl.ctl.trace = buf.get();
-  launch_population(pl, st);
+  launch_population(pl, pl.ctl, st);
   pl.ctl.trace = nullptr;
   std::vector<unsigned long long> t(F * n);
   buf.download(t.data(), t.size(), st);
@@ -1793,9 +1767,9 @@ double Fitness::time_plan(int P, const LaunchShape& sh, int reps, int* occ)
   hipStream_t st = stream_;
   GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), genes.data(), sizeof(float) * genes.size(),
                            hipMemcpyHostToDevice, st));
-  launch_population(pl, st); // warm-up
+  launch_population(pl, pl.ctl, st); // warm-up
   GPUGA_HIP(hipEventRecord(ev0_, st));
-  for (int r = 0; r < reps; ++r) launch_population(pl, st);
+  for (int r = 0; r < reps; ++r) launch_population(pl, pl.ctl, st);
   GPUGA_HIP(hipEventRecord(ev1_, st));
   GPUGA_HIP(hipStreamSynchronize(st));
   float ms = 0.0f;

@@ -19,7 +19,7 @@ namespace gpuga {
 struct FitnessOptions {
   int backend = 0;        // 0: population kernel, 1: per-individual launches
   int chunk_cost = 0;     // work-item cost target; 0 = autotune on first use
-  int use_graph = 1;      // replay each generation from a captured HIP graph
+  int use_graph = 1;      // run_ga: replay its generations from captured HIP graphs
   int nn2b_bf16 = 1;      // NN2B hidden layer 2 on BF16 MFMA (else FP32)
   int nn2b_grid = 1024;   // NN2B tabulation points
   int verbose = 0;
@@ -116,14 +116,6 @@ struct PopPlan {
   PinnedBuffer<float> h_genes;
   PinnedBuffer<double> h_out;
   PopCtl ctl{};
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  // the launch on 1/2, 1/4, 1/8 of the grid (a served job sharing the GPU),
-  // captured when first used
-  static constexpr int kShares = 3;
-  hipGraph_t share_graph[kShares] = {};
-  hipGraphExec_t share_exec[kShares] = {};
-  void drop_share_graphs();
   // device GA of this population size; runs of generations (population
   // launch + GA step each) as graphs: ga_exec[k][j] is 2^j generations
   // starting on population buffer k (a generation on buffer b writes the
@@ -170,7 +162,7 @@ public:
   // What the plan for P was built with: work-item cost, queues, resident
   // workgroups per CU, lane groups of the last lane block.
   void plan_shape(int P, int& chunk_cost, int& queues, int& blocks_per_cu, int& groups_last);
-  // Build the work plan (and its graph) for population size P now, so the
+  // Build the work plan for population size P now, so the
   // first generation does not pay for it.
   void prepare(int P);
   // `generations` GA generations (fitness, sort, crossover, mutation) with
@@ -233,15 +225,13 @@ private:
   void build_plan(PopPlan& pl, int P, const LaunchShape& sh);
   // the shape the options fix (chunk cost > 0: no tuning)
   LaunchShape option_shape() const;
-  // the population launch on genes (default: the plan's buffer)
-  void launch_population(PopPlan& pl, hipStream_t st, const float* genes = nullptr,
-                         int grid = 0);
+  // the population launch of ctl (the plan's, or a copy with other genes or
+  // results); grid 0: the plan's
+  void launch_population(PopPlan& pl, const PopCtl& ctl, hipStream_t st, int grid = 0);
   // the same by the quadratic forms
-  void launch_quad(PopPlan& pl, hipStream_t st, const float* genes = nullptr);
+  void launch_quad(PopPlan& pl, const PopCtl& ctl, hipStream_t st);
   // n generations of the device GA from population buffer k, captured
   void capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph, hipGraphExec_t* exec);
-  void launch_generation(PopPlan& pl, hipStream_t st, int share = 1); // graph or direct
-  void capture(PopPlan& pl, hipStream_t st);           // the plan's graph, once
   double time_plan(int P, const LaunchShape& sh, int reps, int* occ = nullptr);
   // after a launch whose status word is set: clear the plan's counters and
   // results, then fail
@@ -284,6 +274,8 @@ private:
   // per-atom outputs and plain-path scratch
   DeviceBuffer<float> d_f_, d_virial_, d_pe_, d_params_, d_fit1_, d_pmin_, d_pmax_;
   DeviceBuffer<double> d_cerr_, d_terms1_;
+  PinnedBuffer<float> h_atoms_; // find_force's results on their way to the caller
+  hipEvent_t ev_copy_ = nullptr;
   void* ws_static_ = nullptr; // this device's fixed workspace (noalloc.h)
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
   bool timing_ = false;

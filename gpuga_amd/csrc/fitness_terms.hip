@@ -100,7 +100,20 @@ __global__ void __launch_bounds__(RB) finish_terms(int Nc, FitnessNorm nrm,
   }
 }
 
+__global__ void __launch_bounds__(RB) copy_in(const float* __restrict__ from,
+                                              float* __restrict__ to, int n)
+{
+  const int i = blockIdx.x * RB + threadIdx.x;
+  if (i < n) to[i] = from[i];
+}
+
 } // namespace
+
+void launch_copy_in(const float* from, float* to, int n, hipStream_t st)
+{
+  copy_in<<<(n + RB - 1) / RB, RB, 0, st>>>(from, to, n);
+  GPUGA_HIP(hipGetLastError());
+}
 
 void launch_fitness_terms(const DevSet& s, const FitnessNorm& nrm, const float* f,
                           const float* virial, const float* pe, double* cerr, float* fitness,

@@ -18,6 +18,9 @@ void launch_ri_plain(const DevSet& s, const RIParams& q, const float4* tab, floa
 void launch_nn2b_plain(const DevSet& s, int n, bool species, const float* w, float* f,
                        float* virial, float* pe, hipStream_t st);
 
+// n floats from pinned host memory to device memory
+void launch_copy_in(const float* from, float* to, int n, hipStream_t st);
+
 // ---- fitness of one parameter set from per-atom outputs
 // cerr: [Nc][3] scratch; out: fitness (float) and terms[3] (double)
 void launch_fitness_terms(const DevSet& s, const FitnessNorm& nrm, const float* f,

@@ -114,7 +114,7 @@ struct PopCtl {
   unsigned* status;       // [1] non-zero: a dependency wait timed out
   int spin_limit;         // polls of a dependency wait before it gives up
                           // (about 1 us each); < 0: give up at once
-  float* fitness;         // [P]
+  float* fitness;         // [P] (with terms and status in device or pinned host memory)
   double* terms;          // [P][3]
   FitnessNorm norm;
   // optional item timeline: [n_items][kTraceFields] = wave slot, start,
@@ -567,7 +567,8 @@ __global__ void __launch_bounds__(256) population_kernel(PopCtl ctl, DevSet set,
       }
     } else {
       if (!wave_wait_count(cnt, (unsigned)nch, ctl.spin_limit)) {
-        if (lane == 0) atomicOr(ctl.status, 1u);
+        if (lane == 0)
+          __hip_atomic_store(ctl.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
       mark(4);
       if (packed) {

@@ -80,7 +80,7 @@ void Server::admit(Job& j)
     w.fit = std::make_unique<Fitness>(w.spec, std::move(w.ts), o);
     // deterministic work-item size: the same chunking alone or co-scheduled
     if (o.chunk_cost <= 0) w.fit->options().chunk_cost = w.fit->heuristic_chunk_cost(w.gp.population_size);
-    // plan and graph now: generation latencies then measure generations only
+    // plan now: generation latencies then measure generations only
     w.fit->prepare(w.gp.population_size);
     w.ga = std::make_unique<GA>(w.gp, w.fit->number_of_variables(), w.fit->spec().pmin,
                                 w.fit->spec().pmax);
