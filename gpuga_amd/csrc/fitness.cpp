@@ -2,6 +2,9 @@
 #include "fitness.h"
 #include "noalloc.h"
 
+#include <sys/mman.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -10,7 +13,7 @@
 
 namespace gpuga {
 
-int tersoff_population_occupancy(int cls, bool two, bool pack, int block);
+int tersoff_population_occupancy(bool two, bool pack, int block);
 
 // Neighbours within R2 the looped Tersoff population kernel takes (its LDS
 // rows: 4 x 64 lanes x 4 B per neighbour and wave, 64 KiB at this bound).
@@ -135,7 +138,7 @@ size_t DeviceSet::bytes() const
 {
   return Na.bytes() + Na_sum.bytes() + type.bytes() + nn.bytes() + bond0.bytes() + nl.bytes() +
          rev.bytes() + ptype.bytes() + tri0.bytes() + bond.bytes() + tri.bytes() +
-         ri_tab.bytes() + rec.bytes() + pair_hdr.bytes() + pair_tab.bytes() + pe_ref.bytes() +
+         ri_tab.bytes() + rec.bytes() + shell_rec.bytes() + pair_hdr.bytes() + pair_tab.bytes() + pe_ref.bytes() +
          virial_ref.bytes() + force_ref.bytes() + p_nn.bytes() + p_b0.bytes() + p_nl.bytes() +
          p_rev.bytes() + p_ptype.bytes() + p_tri0.bytes() + p_bond.bytes() + p_tri.bytes() +
          ri_cconst.bytes() + ri_fconst.bytes();
@@ -174,7 +177,8 @@ Fitness::~Fitness()
   plans_.clear();
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
-  if (ev_copy_) (void)hipEventDestroy(ev_copy_);
+  for (auto e : ev_half_)
+    if (e) (void)hipEventDestroy(e);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -202,7 +206,7 @@ void Fitness::setup()
   GPUGA_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
   GPUGA_HIP(hipEventCreate(&ev0_));
   GPUGA_HIP(hipEventCreate(&ev1_));
-  GPUGA_HIP(hipEventCreateWithFlags(&ev_copy_, hipEventDisableTiming));
+  for (auto& e : ev_half_) GPUGA_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 
   const bool tersoff = spec_.type == POT_TERSOFF1 || spec_.type == POT_TERSOFF2;
   if (spec_.type == POT_RI || spec_.type == POT_NN2B_SPECIES)
@@ -262,7 +266,8 @@ void Fitness::setup()
     }
     const NeighborList& pn = population_neighbors();
     const int M = record_slots(pn.max_nn);
-    loop_path_ = M == 0;
+    shell_M_ = pn.max_nn > 4 ? tersoff_shell_slots(pn.max_nn) : 0;
+    loop_path_ = M == 0 && shell_M_ == 0;
     if (loop_path_ && pn.max_nn > kLoopMaxNeighbors)
       fail(strfmt("the population kernel supports at most %d neighbours per atom within the "
                   "largest R2 (found %d); use the per-individual backend",
@@ -298,26 +303,32 @@ void Fitness::setup()
       // (the host vectors above are read before this scope ends)
       GPUGA_HIP(hipStreamSynchronize(st));
     }
+    loop_.nn = pd.NN;
+    loop_.b0 = pd.start;
+    loop_.tri0 = pd.tri0;
+    loop_.rev = pd.rev;
+    loop_.ptype = pptype;
+    loop_.bond = pbond;
+    loop_.tri = ptri;
+    loop_.max_nn = pn.max_nn;
+    if (shell_M_ > 0) {
+      ds_.shell_rec.resize(tersoff_shell_floats4(ts_.N, shell_M_));
+      build_shell_records(ts_.N, shell_M_, loop_, ds_.shell_rec.get(), st);
+    }
     if (M > 0) {
       const size_t RS = 1 + M + (size_t)M * M + M / 2;
       ds_.rec.resize((size_t)ts_.N * RS);
       build_records_device(ts_.N, M, pd, pptype, pbond, ptri, ds_.rec.get(), st);
       ds_.view.rec_nmax = M;
+    }
+    if (!loop_path_) {
       GPUGA_HIP(hipStreamSynchronize(st));
       // the records hold everything the kernel reads of the pruned list
       for (auto* b : {&ds_.p_nn, &ds_.p_b0, &ds_.p_nl, &ds_.p_rev, &ds_.p_ptype, &ds_.p_tri0})
         b->resize(0);
       ds_.p_bond.resize(0);
       ds_.p_tri.resize(0);
-    } else {
-      loop_.nn = pd.NN;
-      loop_.b0 = pd.start;
-      loop_.tri0 = pd.tri0;
-      loop_.rev = pd.rev;
-      loop_.ptype = pptype;
-      loop_.bond = pbond;
-      loop_.tri = ptri;
-      loop_.max_nn = pn.max_nn;
+      loop_ = LoopTab{};
     }
     ds_.view.bond_force =
       ts_.N_force > 0 ? pn.start[ts_.N_force - 1] + pn.NN[ts_.N_force - 1] : 0;
@@ -387,6 +398,7 @@ void Fitness::setup()
   d_f_.resize(3 * (size_t)ts_.N);
   d_virial_.resize(6 * (size_t)ts_.N);
   d_pe_.resize(ts_.N);
+  if (10 * (size_t)ts_.N > 3 * kHalf) h_atoms_.resize(2 * kHalf);
   d_cerr_.resize(3 * (size_t)ts_.Nc);
   d_fit1_.resize(1);
   d_terms1_.resize(3);
@@ -863,13 +875,6 @@ long long atom_cost(int type, int nn, bool force_cfg)
   return (force_cfg ? nn : nn / 2 + 1) + 4;
 }
 
-int nn_class(int max_nn)
-{
-  if (max_nn <= 4) return 0;
-  if (max_nn <= 8) return 1;
-  return 2;
-}
-
 } // namespace
 
 size_t Fitness::plan_bytes(int P) const
@@ -914,7 +919,7 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   const int K = pl.K;
 
   struct Chunk {
-    int c, chunk, a0, a1, cls;
+    int c, chunk, a0, a1;
     long long cost;
   };
   std::vector<Chunk> chunks;
@@ -968,23 +973,21 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
     slot0[c] = slots;
     slots += n;
     long long acc = 0;
-    int start = a0, k = 0, mx = 0;
+    int start = a0, k = 0;
     long long cacc = 0;
     for (int i = a0; i < a1; ++i) {
       const long long ci = atom_cost(spec_.type, pn.NN[i], fc);
       acc += ci;
       cacc += ci;
-      mx = std::max(mx, pn.NN[i]);
       // cut at the k-th cost quantile, or when the atoms left are exactly
       // the chunks still to make
       const int left_atoms = a1 - (i + 1), left_chunks = n - 1 - k;
       const bool must = left_chunks > 0 && left_atoms == left_chunks;
       const bool want = left_chunks > 0 && left_atoms >= left_chunks && acc * n >= total * (k + 1);
       if (must || want || i == a1 - 1) {
-        chunks.push_back(Chunk{c, k, start, i + 1, nn_class(mx), cacc});
+        chunks.push_back(Chunk{c, k, start, i + 1, cacc});
         start = i + 1;
         ++k;
-        mx = 0;
         cacc = 0;
       }
     }
@@ -1007,7 +1010,7 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   // G = 2, P = 216, the launch took 0.607 ms packed against 0.521 ms
   // unpacked; with G = 4, P = 208, 0.458 against 0.523 ms.)
   int G_last = 1;
-  if (tersoff && sh.pack && !loop_path_) {
+  if (tersoff && sh.pack && !loop_path_ && shell_M_ == 0) {
     const int Pr = P - (K - 1) * WAVE;
     int W = 1;
     while (W < Pr) W <<= 1;
@@ -1026,7 +1029,7 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
       const int n = ch.a1 - ch.a0, steps = (n + G - 1) / G;
       // (with the assembly of a one-chunk three-body force configuration)
       const long long asm_cost = tersoff && ch.c < ts_.Nc_force && nch[ch.c] == 1 ? 8LL * steps : 0;
-      eval.push_back(Costed{WorkItem{ch.c, k, ch.chunk, ch.a0, ch.a1, ch.cls, 0, G},
+      eval.push_back(Costed{WorkItem{ch.c, k, ch.chunk, ch.a0, ch.a1, 0, G, 0},
                             ch.cost * steps / n + asm_cost});
     }
   // three-body force configurations of several chunks: one force-assembly
@@ -1040,7 +1043,7 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
           const int G = k == K - 1 ? G_last : 1;
           const int n = ch.a1 - ch.a0, steps = (n + G - 1) / G;
           assemble.push_back(
-            Costed{WorkItem{ch.c, k, ch.chunk, ch.a0, ch.a1, ch.cls, 1, G}, 8LL * steps});
+            Costed{WorkItem{ch.c, k, ch.chunk, ch.a0, ch.a1, 1, G, 0}, 8LL * steps});
         }
   pl.n_items = (int)(eval.size() + assemble.size());
   const int waves_per_block = pl.block / WAVE;
@@ -1052,10 +1055,9 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
       case POT_NN2B:
       case POT_NN2B_SPECIES: occ = nn2b_population_occupancy(pl.block); break;
       default:
-        occ = loop_path_ ? tersoff_loop_occupancy(spec_.type == POT_TERSOFF2, pn.max_nn, pl.block)
-                         : tersoff_population_occupancy(nn_class(pn.max_nn),
-                                                        spec_.type == POT_TERSOFF2, G_last > 1,
-                                                        pl.block);
+        occ = shell_M_ > 0 ? tersoff_shell_occupancy(shell_M_, spec_.type == POT_TERSOFF2, pl.block)
+              : loop_path_ ? tersoff_loop_occupancy(spec_.type == POT_TERSOFF2, pn.max_nn, pl.block)
+                           : tersoff_population_occupancy(spec_.type == POT_TERSOFF2, G_last > 1, pl.block);
         break;
       }
       occ = std::max(occ, 1);
@@ -1243,14 +1245,17 @@ void Fitness::launch_population(PopPlan& pl, const PopCtl& ctl, hipStream_t st, 
     break;
   }
   default: {
+    if (shell_M_ > 0) {
+      launch_tersoff_shell_population(ctl, ds_.view, shell_M_, ds_.shell_rec.get(), G, pl.block, st);
+      break;
+    }
     if (loop_path_) {
       launch_tersoff_loop_population(ctl, ds_.view, loop_, G, pl.block, st);
       break;
     }
     // the instantiation with the packed path only when the plan has packed
     // items; the one for lone waves when there is at most a workgroup per CU
-    launch_tersoff_population(ctl, ds_.view, nn_class(population_neighbors().max_nn), G,
-                              pl.block, pl.groups_last > 1, G <= num_cu_, st);
+    launch_tersoff_population(ctl, ds_.view, G, pl.block, pl.groups_last > 1, G <= num_cu_, st);
     break;
   }
   }
@@ -1592,6 +1597,23 @@ void Fitness::plain_loop(int P, const float* genes, float* fitness, double* term
   }
 }
 
+namespace {
+
+// Maps the whole pages of [p, p + n) for writing, where the system can.
+void populate(void* p, size_t n)
+{
+#ifdef MADV_POPULATE_WRITE
+  constexpr int advice = MADV_POPULATE_WRITE;
+#else
+  constexpr int advice = 23; // its value on Linux (since 5.14)
+#endif
+  const size_t page = (size_t)sysconf(_SC_PAGESIZE);
+  const size_t a = ((size_t)p + page - 1) / page * page, b = ((size_t)p + n) / page * page;
+  if (b > a) (void)madvise(reinterpret_cast<void*>(a), b - a, advice);
+}
+
+} // namespace
+
 void Fitness::find_force(const float* physical, float* f, float* virial, float* pe)
 {
   std::vector<float> params(physical, physical + spec_.V);
@@ -1599,21 +1621,49 @@ void Fitness::find_force(const float* physical, float* f, float* virial, float* 
   hipStream_t st = stream_;
   potential_->find_force(ds_.view, d_f_.get(), d_virial_.get(), d_pe_.get(), st);
   GPUGA_HIP(hipGetLastError());
-  // through a pinned block, energy and force to the caller while the virial
-  // is still on its way (a copy into pageable memory runs at a sixth of the
-  // pinned rate)
   const size_t N = ts_.N;
-  h_atoms_.resize(10 * N);
-  float *he = h_atoms_.get(), *hf = he + N, *hw = hf + 3 * N;
-  if (pe) d_pe_.download(he, N, st);
-  if (f) d_f_.download(hf, 3 * N, st);
-  GPUGA_HIP(hipEventRecord(ev_copy_, st));
-  if (virial) d_virial_.download(hw, 6 * N, st);
-  GPUGA_HIP(hipEventSynchronize(ev_copy_));
-  if (pe) std::memcpy(pe, he, sizeof(float) * N);
-  if (f) std::memcpy(f, hf, sizeof(float) * 3 * N);
-  GPUGA_HIP(hipStreamSynchronize(st));
-  if (virial) std::memcpy(virial, hw, sizeof(float) * 6 * N);
+  // Results of more than 1.5 MiB through the pinned halves of h_atoms_, one
+  // filled while the other is copied to the caller: a copy into pageable
+  // memory runs at a third of the pinned rate (4 MB: a call of 357 -> 267 us;
+  // 1 MB takes 113 us either way).
+  const struct {
+    const float* from;
+    float* to;
+    size_t n;
+  } part[3] = {{d_pe_.get(), pe, N}, {d_f_.get(), f, 3 * N}, {d_virial_.get(), virial, 6 * N}};
+  if (h_atoms_.size() == 0) {
+    for (const auto& p : part)
+      if (p.to)
+        GPUGA_HIP(hipMemcpyAsync(p.to, p.from, sizeof(float) * p.n, hipMemcpyDeviceToHost, st));
+    GPUGA_HIP(hipStreamSynchronize(st));
+    return;
+  }
+  struct Piece {
+    float* to = nullptr;
+    size_t n = 0;
+  } piece[2];
+  // the caller's pages, while the GPU works: a copy into memory that has not
+  // been touched yet would fault on each of them (4.8 MB: 300 us)
+  for (const auto& p : part)
+    if (p.to) populate(p.to, sizeof(float) * p.n);
+  int k = 0;
+  auto take = [&](int h) { // wait for half h and hand it to the caller
+    if (!piece[h].to) return;
+    GPUGA_HIP(hipEventSynchronize(ev_half_[h]));
+    std::memcpy(piece[h].to, h_atoms_.get() + h * kHalf, sizeof(float) * piece[h].n);
+    piece[h].to = nullptr;
+  };
+  for (const auto& p : part)
+    for (size_t at = 0; p.to && at < p.n; at += kHalf, k ^= 1) {
+      take(k);
+      const size_t n = std::min(kHalf, p.n - at);
+      GPUGA_HIP(hipMemcpyAsync(h_atoms_.get() + k * kHalf, p.from + at, sizeof(float) * n,
+                               hipMemcpyDeviceToHost, st));
+      GPUGA_HIP(hipEventRecord(ev_half_[k], st));
+      piece[k] = Piece{p.to + at, n};
+    }
+  take(k);
+  take(k ^ 1);
 }
 
 void Fitness::predict(const std::string& dir, const float* elite)
@@ -1893,7 +1943,7 @@ int Fitness::autotune(int P)
     consider(sh, 6);
   }
   // the packed last lane block against plain lanes
-  if (opt_.pack_lanes && tersoff && !loop_path_) {
+  if (opt_.pack_lanes && tersoff && !loop_path_ && shell_M_ == 0) {
     const int Pr = P - (K - 1) * WAVE;
     if (Pr <= 16) {
       LaunchShape sh = best;

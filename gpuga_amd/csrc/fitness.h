@@ -47,7 +47,7 @@ struct LaunchShape {
 // Device-resident copy of one training set and its geometry tables.
 struct DeviceSet {
   DeviceBuffer<int> Na, Na_sum, type, nn, bond0, nl, rev, ptype, tri0;
-  DeviceBuffer<float4> bond, tri, ri_tab, rec, pair_tab;
+  DeviceBuffer<float4> bond, tri, ri_tab, rec, shell_rec, pair_tab;
   // the Tersoff population kernel's pruned list and its tables, kept when
   // the looped kernel reads them (more than 16 neighbours within R2)
   DeviceBuffer<int> p_nn, p_b0, p_nl, p_rev, p_ptype, p_tri0;
@@ -257,7 +257,8 @@ private:
   NeighborList nl_;
   NeighborList pnl_;    // pruned list of the Tersoff population kernel
   bool pruned_ = false; // pnl_ holds fewer bonds than nl_
-  bool loop_path_ = false; // Tersoff: more than 16 neighbours within R2
+  int shell_M_ = 0;        // Tersoff: bond slots of the unordered-pair kernel (0: another)
+  bool loop_path_ = false; // Tersoff: the looped kernel
   LoopTab loop_{};         // the looped kernel's tables
   std::vector<int> ptype_; // pair type per bond
   bool pair_tables_ = false;
@@ -274,8 +275,10 @@ private:
   // per-atom outputs and plain-path scratch
   DeviceBuffer<float> d_f_, d_virial_, d_pe_, d_params_, d_fit1_, d_pmin_, d_pmax_;
   DeviceBuffer<double> d_cerr_, d_terms1_;
-  PinnedBuffer<float> h_atoms_; // find_force's results on their way to the caller
-  hipEvent_t ev_copy_ = nullptr;
+  // find_force's results on their way to the caller: two halves
+  static constexpr size_t kHalf = 128 * 1024; // floats
+  PinnedBuffer<float> h_atoms_;
+  hipEvent_t ev_half_[2] = {};
   void* ws_static_ = nullptr; // this device's fixed workspace (noalloc.h)
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
   bool timing_ = false;

@@ -28,12 +28,12 @@ void launch_fitness_terms(const DevSet& s, const FitnessNorm& nrm, const float* 
                           double* terms, hipStream_t st);
 
 // ---- population kernels (one persistent launch per generation)
-// cls: neighbour-count class of the training set (0: <= 4, 1: <= 8, 2: <= 16);
-// pack: serve the packed-item queue (several atoms per wave); lone: a launch
-// of at most one wave per SIMD (the form that trades registers for latency)
-void launch_tersoff_population(const PopCtl& ctl, const DevSet& s, int cls, int grid, int block,
+// At most four neighbours within R2.  pack: serve the packed-item queue
+// (several atoms per wave); lone: a launch of at most one wave per SIMD (the
+// form that trades registers for latency)
+void launch_tersoff_population(const PopCtl& ctl, const DevSet& s, int grid, int block,
                                bool pack, bool lone, hipStream_t st);
-// Tersoff sets with more than 16 neighbours within R2: per-bond lane values
+// Tersoff sets with more than 20 neighbours within R2: per-bond lane values
 // in LDS (dynamic, tersoff_loop_lds_bytes per workgroup), geometry from the
 // bond and triplet tables of the list in t.
 struct LoopTab {
@@ -41,6 +41,14 @@ struct LoopTab {
   const float4 *bond, *tri;                // its bond and triplet tables
   int max_nn;
 };
+// 5 to 20 neighbours within R2: per-bond values in registers, one cosine per
+// pair of bonds (records built from the list's tables)
+int tersoff_shell_slots(int max_nn);
+size_t tersoff_shell_floats4(int N, int M);
+void build_shell_records(int N, int M, const LoopTab& t, float4* rec, hipStream_t st);
+void launch_tersoff_shell_population(const PopCtl& ctl, const DevSet& s, int M, const float4* rec,
+                                     int grid, int block, hipStream_t st);
+int tersoff_shell_occupancy(int M, bool two, int block);
 size_t tersoff_loop_lds_bytes(int max_nn, int block);
 void launch_tersoff_loop_population(const PopCtl& ctl, const DevSet& s, const LoopTab& t,
                                     int grid, int block, hipStream_t st);

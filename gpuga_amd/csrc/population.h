@@ -79,9 +79,9 @@ struct WorkItem {
   int k;      // lane block
   int chunk;  // chunk index inside the configuration
   int a0, a1; // global atom range of the chunk
-  int cls;    // neighbour-count class of the chunk
   int phase;  // 0: evaluate, 1: assemble forces of a three-body force configuration
   int groups; // 1: lane = individual; G > 1: packed lane block (see below)
+  int pad;    // (32 bytes)
 };
 
 struct PopCtl {

@@ -12,91 +12,11 @@
 // order), :250-307 (partial force f_ij), :355-392 (force and virial).
 #include <type_traits>
 
-#include "fastmath.h"
 #include "kernels.h"
 #include "population.h"
+#include "tersoff_math.h"
 
 namespace gpuga {
-
-// ------------------------------------------------------------ scalar pieces
-
-// Per-parameter-set constants in the form the kernels use: exponent
-// prefactors scaled by log2(e) for the exp2 instruction, 1/(R2-R1) and
-// 0.5 pi/(R2-R1) for the taper.
-struct TLane {
-  float cR[2], kR[2], kR2[2], cA[2], kA[2], kA2[2], r0[2];
-  float en, mhon, en1, mhon1, beta, beta2, h, r1, r2, inv_span, pif_half;
-  float r1min; // population kernels: the smallest R1 of the wave's lanes
-};
-
-__host__ __device__ inline TLane tersoff_lane(const TersoffParams& p)
-{
-  TLane q;
-  for (int k = 0; k < 2; ++k) {
-    q.cR[k] = p.cR[k];
-    q.kR[k] = p.kR[k];
-    q.kR2[k] = p.kR[k] * LOG2E;
-    q.cA[k] = p.cA[k];
-    q.kA[k] = p.kA[k];
-    q.kA2[k] = p.kA[k] * LOG2E;
-    q.r0[k] = p.r0[k];
-  }
-  q.en = p.en;
-  q.mhon = p.minus_half_over_n;
-  q.en1 = p.en - 1.0f;
-  q.mhon1 = p.minus_half_over_n - 1.0f;
-  q.beta = p.beta;
-  q.beta2 = 2.0f * p.beta;
-  q.h = p.h;
-  q.r1 = p.r1;
-  q.r2 = p.r2;
-  q.inv_span = 1.0f / (p.r2 - p.r1);
-  q.pif_half = 0.5f * p.pi_factor;
-  q.r1min = p.r1;
-  return q;
-}
-
-// fc and dfc/dr (src/minimal_tersoff.cu:77-90)
-__device__ __forceinline__ void tersoff_fc(const TLane& q, float d, float& fc, float& fcp)
-{
-  // 1 below r1, 0 from r2 on (a select), the taper between them under one
-  // branch that the wave skips when no lane needs it
-  const bool below = d < q.r1;
-  fc = below ? 1.0f : 0.0f;
-  fcp = 0.0f;
-  if (!below && d < q.r2) {
-    float sn, cs;
-    sincospi01((d - q.r1) * q.inv_span, sn, cs);
-    fc = 0.5f * cs + 0.5f;
-    fcp = -q.pif_half * sn;
-  }
-}
-
-// b = (1 + zeta^n)^(-1/2n) and db/dzeta = -1/2 (1 + zeta^n)^(-1/2n - 1)
-// zeta^(n - 1), the latter as one exp2 of the summed logarithms (no
-// reciprocal); b = 1, b' = 0 below zeta = 1e-16 (src/minimal_tersoff.cu:174-185)
-__device__ __forceinline__ void tersoff_bond_order(const TLane& q, float zeta, float& b, float& bp)
-{
-  const float lz = flog2(zeta);
-  const float bzn = fexp2(q.en * lz);
-  const float l1 = flog2(1.0f + bzn);
-  // the cut-off as selects of the exponents (exp2(0) = 1, exp2(-inf) = 0),
-  // so that no branch forms around the exp2 instructions
-  const bool tiny = zeta < 1.0e-16f;
-  b = fexp2(tiny ? 0.0f : q.mhon * l1);
-  bp = -fexp2(tiny ? -__builtin_inff() : fmaf(q.mhon1, l1, fmaf(q.en1, lz, -1.0f)));
-}
-
-// fR, fR', fA, fA' (src/minimal_tersoff.cu:62-75) of parameter set k
-__device__ __forceinline__ void tersoff_pair(const TLane& q, int k, float d, float& fr, float& frp,
-                                             float& fa, float& fap)
-{
-  const float x = d - q.r0[k];
-  fr = q.cR[k] * fexp2(q.kR2[k] * x);
-  frp = q.kR[k] * fr;
-  fa = q.cA[k] * fexp2(q.kA2[k] * x);
-  fap = q.kA[k] * fa;
-}
 
 // --------------------------------------- single-parameter-set kernels
 // Thread per atom; scratch per bond: b, b' then f_ij.
@@ -215,31 +135,18 @@ void launch_tersoff_plain(const DevSet& s, const TersoffParams& q, float* b, flo
 
 // ---------------------------------------------------------- population
 
-// NMAX bounds the neighbour count of the training set so the per-bond values
-// of an atom live in registers; TWO selects the two-species parameter sets.
-template <int NMAX, bool TWO>
+// Sets with at most four neighbours within R2, so the per-bond values of an
+// atom live in registers (five to twenty: tersoff_shell.hip); TWO selects the
+// two-species parameter sets.
+template <bool TWO>
 struct TersoffPop {
+  static constexpr int NMAX = 4;
   static constexpr bool kForcePass = true;
   static constexpr int kFoldValues = 24;
   using Lane = TLane;
   using Extra = int;
 
-  __device__ static Lane make(const PopCtl& ctl, int p)
-  {
-    constexpr int V = TWO ? 13 : 9;
-    float x[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v)
-      x[v] = denormalise(ldu(ctl.pmin, v), ldu(ctl.pmax, v), ctl.genes[(size_t)p * V + v]);
-    TLane q = tersoff_lane(tersoff_params(TWO ? 2 : 1, x));
-    // the wave's smallest R1 (every lane calls make): an atom whose bonds
-    // are all shorter has fc = 1, fc' = 0 on every lane
-    float m = q.r1;
-#pragma unroll
-    for (int o = WAVE / 2; o >= 1; o >>= 1) m = fminf(m, __shfl_xor(m, o));
-    q.r1min = m;
-    return q;
-  }
+  __device__ static Lane make(const PopCtl& ctl, int p) { return tersoff_make<TWO>(ctl, p); }
 
   // One atom for 64 individuals: the geometry is wave-uniform (scalar loads
   // from the atom's record), the parameters are per lane; all loop guards are
@@ -312,12 +219,10 @@ struct TersoffPop {
     // a body without neighbour-count guards: no selects, no guarded loads;
     // when its longest bond is also shorter than every lane's R1 (the usual
     // case), fc = 1 and fc' = 0 exactly and the taper terms drop out
-    // (four-bond records only: the larger bodies have no registers to spare
-    // for a third copy)
     if constexpr (U) {
       if (nn == NMAX) {
-        if (NMAX <= 4 && h.dmax < q.r1min)
-          atom_body<FORCE, U, true, NMAX <= 4, LR>(s, q, i, R, nn, unl, fblk, lane, acc);
+        if (h.dmax < q.r1min)
+          atom_body<FORCE, U, true, true, LR>(s, q, i, R, nn, unl, fblk, lane, acc);
         else
           atom_body<FORCE, U, true, false, LR>(s, q, i, R, nn, unl, fblk, lane, acc);
         return;
@@ -342,19 +247,12 @@ struct TersoffPop {
     // can afford: loaded at each use, inside the per-lane branches, every
     // load waited for on its own made a packed atom step cost five uniform
     // ones.
-    constexpr bool PRE = NMAX <= 8; // preload rows (register budget allows)
     float d[NMAX], dinv[NMAX];
-    if constexpr (PRE) {
 #pragma unroll
-      for (int u = 0; u < NMAX; ++u) {
-        d[u] = ldr<U, LR>(R, 1 + u).w;
-        dinv[u] = ldr<U, LR>(reinterpret_cast<const float*>(R + INV), u);
-      }
+    for (int u = 0; u < NMAX; ++u) {
+      d[u] = ldr<U, LR>(R, 1 + u).w;
+      dinv[u] = ldr<U, LR>(reinterpret_cast<const float*>(R + INV), u);
     }
-    auto dist = [&](int u) { return PRE ? d[u] : ldr<U, LR>(R, 1 + u).w; };
-    auto dist_inv = [&](int u) {
-      return PRE ? dinv[u] : ldr<U, LR>(reinterpret_cast<const float*>(R + INV), u);
-    };
     float fc[NMAX], fcp[NMAX], fcb[NMAX], A[NMAX], B[NMAX], pf[NMAX];
 #pragma unroll
     for (int u = 0; u < NMAX; ++u) {
@@ -364,60 +262,42 @@ struct TersoffPop {
           fcp[u] = 0.0f;
           fcb[u] = q.beta;
         } else {
-          tersoff_fc(q, dist(u), fc[u], fcp[u]);
+          tersoff_fc(q, d[u], fc[u], fcp[u]);
           fcb[u] = fc[u] * q.beta;
         }
       }
     }
-    // With four bonds, x = cos(theta_jk) - h and x^2 once per unordered pair:
-    // the record holds the same cosine, bit for bit, at (j, k) and (k, j)
+    // x = cos(theta_jk) - h and x^2 once per unordered pair: the record holds the same cosine, bit for bit, at (j, k) and (k, j)
     // (the set-up computes it with commuting products in one order).
-    constexpr bool SYM = NMAX <= 4;
     float xs[NMAX][NMAX], x2[NMAX][NMAX];
-    if constexpr (SYM) {
 #pragma unroll
-      for (int u = 0; u < NMAX; ++u)
+    for (int u = 0; u < NMAX; ++u)
 #pragma unroll
-        for (int v = u + 1; v < NMAX; ++v)
-          if (FULL || v < nn) {
-            xs[u][v] = ldr<U, LR>(R, 1 + NMAX + u * NMAX + v).x - q.h;
-            x2[u][v] = xs[u][v] * xs[u][v];
-          }
-    }
+      for (int v = u + 1; v < NMAX; ++v)
+        if (FULL || v < nn) {
+          xs[u][v] = ldr<U, LR>(R, 1 + NMAX + u * NMAX + v).x - q.h;
+          x2[u][v] = xs[u][v] * xs[u][v];
+        }
     auto xsym = [&](int u, int v) { return u < v ? xs[u][v] : xs[v][u]; };
     auto x2sym = [&](int u, int v) { return u < v ? x2[u][v] : x2[v][u]; };
     float e = 0.0f;
 #pragma unroll
     for (int u = 0; u < NMAX; ++u) {
       if (FULL || u < nn) {
-        float cs[NMAX];
-        if constexpr (PRE && !SYM) {
-#pragma unroll
-          for (int v = 0; v < NMAX; ++v)
-            if (v != u) cs[v] = ldr<U, LR>(R, 1 + NMAX + u * NMAX + v).x;
-        }
         float zeta = 0.0f;
 #pragma unroll
-        for (int v = 0; v < NMAX; ++v) {
-          if ((FULL || v < nn) && v != u) {
-            if constexpr (SYM) {
-              zeta = fmaf(fcb[v], x2sym(u, v), zeta);
-            } else {
-              const float x = (PRE ? cs[v] : ldr<U, LR>(R, 1 + NMAX + u * NMAX + v).x) - q.h;
-              zeta = fmaf(fcb[v], x * x, zeta);
-            }
-          }
-        }
+        for (int v = 0; v < NMAX; ++v)
+          if ((FULL || v < nn) && v != u) zeta = fmaf(fcb[v], x2sym(u, v), zeta);
         float b, bp;
         tersoff_bond_order(q, zeta, b, bp);
         // the parameter set as a branch on the (wave-uniform) bond type, so
         // the set is a compile-time index and the parameters stay in
         // registers (a run-time index puts them in scratch memory)
         float fr, frp, fa, fap;
-        if (TWO && ((unl >> u) & 1)) tersoff_pair(q, 1, dist(u), fr, frp, fa, fap);
-        else tersoff_pair(q, 0, dist(u), fr, frp, fa, fap);
+        if (TWO && ((unl >> u) & 1)) tersoff_pair(q, 1, d[u], fr, frp, fa, fap);
+        else tersoff_pair(q, 0, d[u], fr, frp, fa, fap);
         const float rep = fr - b * fa;
-        const float di = dist_inv(u);
+        const float di = dinv[u];
         A[u] = bp * fa;
         if constexpr (INNER) {
           e += rep;
@@ -440,25 +320,19 @@ struct TersoffPop {
         //   dsum = sum_k B_k (h - cos)^2                     (times beta)
         // where (A_j + A_k) fc_k = A_j fc_k + B_k
         float4 row[NMAX];
-        if constexpr (PRE) {
 #pragma unroll
-          for (int v = 0; v < NMAX; ++v)
-            if (v != u) row[v] = ldr<U, LR>(R, 1 + NMAX + u * NMAX + v);
-        }
+        for (int v = 0; v < NMAX; ++v)
+          if (v != u) row[v] = ldr<U, LR>(R, 1 + NMAX + u * NMAX + v);
         float cx = 0.0f, cy = 0.0f, cz = 0.0f, dsum = 0.0f;
 #pragma unroll
         for (int v = 0; v < NMAX; ++v) {
           if ((FULL || v < nn) && v != u) {
-            const float4 t = PRE ? row[v] : ldr<U, LR>(R, 1 + NMAX + u * NMAX + v);
-            const float x = SYM ? xsym(u, v) : t.x - q.h;
-            const float w = (INNER ? A[u] + A[v] : fmaf(A[u], fc[v], B[v])) * x;
+            const float4 t = row[v];
+            const float w = (INNER ? A[u] + A[v] : fmaf(A[u], fc[v], B[v])) * xsym(u, v);
             cx = fmaf(w, t.y, cx);
             cy = fmaf(w, t.z, cy);
             cz = fmaf(w, t.w, cz);
-            if constexpr (!INNER) {
-              if constexpr (SYM) dsum = fmaf(B[v], x2sym(u, v), dsum);
-              else dsum = fmaf(B[v] * x, x, dsum);
-            }
+            if constexpr (!INNER) dsum = fmaf(B[v], x2sym(u, v), dsum);
           }
         }
         const float4 r = ldr<U, LR>(R, 1 + u);
@@ -510,7 +384,7 @@ struct TersoffPop {
   // Lone-wave form: a record spread over the wave, word l in lane l and
   // word 64 + l in lane l (two vector loads).
   static constexpr int RW = RS * 4; // words per record
-  static_assert(NMAX > 4 || (RW >= WAVE && RW <= 2 * WAVE), "record layout of the lone-wave form");
+  static_assert(RW >= WAVE && RW <= 2 * WAVE, "record layout of the lone-wave form");
   struct Spread {
     int lo, hi;
   };
@@ -533,9 +407,9 @@ struct TersoffPop {
                __int_as_float(__builtin_amdgcn_readlane(v.lo, 3))};
   }
 
-  // HDR: load the next atom's header during the current atom (four-bond
-  // records; the kernel instantiation without the packed path, whose
-  // register budget has room for it).  LONE (launches of at most one wave
+  // HDR: load the next atom's header during the current atom (the kernel
+  // instantiation without the packed path, whose register budget has room for
+  // it).  LONE (launches of at most one wave
   // per SIMD, where a wave's time is the latency of its loads): the next
   // atom's whole record is loaded during the current atom, spread over the
   // wave, and written to the wave's LDS buffer at its end; the rows are read
@@ -547,7 +421,7 @@ struct TersoffPop {
   {
     const int lane = __lane_id();
     const unsigned r = dispatch_round();
-    if constexpr (LONE && NMAX <= 4) {
+    if constexpr (LONE) {
       // two records per wave of a 256-thread workgroup (the kernel's bound)
       __shared__ float4 buf[256 / WAVE][2][RS];
       const int w = wave_first((int)(threadIdx.x / WAVE));
@@ -568,7 +442,7 @@ struct TersoffPop {
       };
       if (it.c < s.Nc_force) run(std::true_type{});
       else run(std::false_type{});
-    } else if constexpr (NMAX > 4 || !HDR) {
+    } else if constexpr (!HDR) {
       if (it.c < s.Nc_force) {
         float* fblk = ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE;
         for (int i = it.a0; i < it.a1; ++i) {
@@ -694,7 +568,7 @@ struct TersoffPop {
   }
 };
 
-// Sets with more than 16 neighbours within R2: the reference's bond loops
+// Sets with more than 20 neighbours within R2: the reference's bond loops
 // (src/minimal_tersoff.cu:122-316) with run-time trip counts, the geometry
 // read from the bond and triplet tables (wave-uniform loads) and the per-bond
 // values of the 64 lanes (fc, fc'/d, b' fA, the pair part of f_ij) kept in
@@ -707,7 +581,7 @@ struct TersoffLoop {
   using Lane = TLane;
   using Extra = LoopTab;
 
-  __device__ static Lane make(const PopCtl& ctl, int p) { return TersoffPop<4, TWO>::make(ctl, p); }
+  __device__ static Lane make(const PopCtl& ctl, int p) { return tersoff_make<TWO>(ctl, p); }
 
   template <bool FORCE>
   __device__ static void atom(const DevSet& s, const LoopTab& t, const TLane& q, int i,
@@ -871,62 +745,38 @@ int tersoff_loop_occupancy(bool two, int max_nn, int block)
   return n;
 }
 
-template <int NMAX, bool TWO>
+template <bool TWO>
 static void launch_t(const PopCtl& ctl, const DevSet& s, int grid, int block, bool pack,
                      bool lone, hipStream_t st)
 {
-  if (pack) {
-    population_kernel<TersoffPop<NMAX, TWO>, true><<<grid, block, 0, st>>>(ctl, s, 0);
-    return;
-  }
-  if constexpr (NMAX == 4) {
-    if (lone) {
-      population_kernel<TersoffPop<NMAX, TWO>, false, true><<<grid, block, 0, st>>>(ctl, s, 0);
-      return;
-    }
-  }
-  population_kernel<TersoffPop<NMAX, TWO>, false><<<grid, block, 0, st>>>(ctl, s, 0);
+  if (pack) population_kernel<TersoffPop<TWO>, true><<<grid, block, 0, st>>>(ctl, s, 0);
+  else if (lone) population_kernel<TersoffPop<TWO>, false, true><<<grid, block, 0, st>>>(ctl, s, 0);
+  else population_kernel<TersoffPop<TWO>, false><<<grid, block, 0, st>>>(ctl, s, 0);
 }
 
-// cls: 0 for at most 4 neighbours per atom, 1 for 8, 2 for 16; pack: the
-// packed-item instantiation; lone: the instantiation for launches of one
-// wave per SIMD (four-bond records, no packed items)
-void launch_tersoff_population(const PopCtl& ctl, const DevSet& s, int cls, int grid, int block,
+// pack: the packed-item instantiation; lone: the instantiation for launches
+// of one wave per SIMD (no packed items)
+void launch_tersoff_population(const PopCtl& ctl, const DevSet& s, int grid, int block,
                                bool pack, bool lone, hipStream_t st)
 {
-  const bool two = ctl.V == 13;
-  switch (cls * 2 + (two ? 1 : 0)) {
-  case 0: launch_t<4, false>(ctl, s, grid, block, pack, lone, st); break;
-  case 1: launch_t<4, true>(ctl, s, grid, block, pack, lone, st); break;
-  case 2: launch_t<8, false>(ctl, s, grid, block, pack, lone, st); break;
-  case 3: launch_t<8, true>(ctl, s, grid, block, pack, lone, st); break;
-  case 4: launch_t<16, false>(ctl, s, grid, block, pack, lone, st); break;
-  default: launch_t<16, true>(ctl, s, grid, block, pack, lone, st); break;
-  }
+  if (ctl.V == 13) launch_t<true>(ctl, s, grid, block, pack, lone, st);
+  else launch_t<false>(ctl, s, grid, block, pack, lone, st);
   GPUGA_HIP(hipGetLastError());
 }
 
-template <int NMAX, bool TWO>
-static int occ_t(bool pack, int block)
+template <bool TWO>
+static const void* kernel_t(bool pack)
 {
-  int n = 0;
-  const void* f =
-    pack ? reinterpret_cast<const void*>(&population_kernel<TersoffPop<NMAX, TWO>, true>)
-         : reinterpret_cast<const void*>(&population_kernel<TersoffPop<NMAX, TWO>, false>);
-  GPUGA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, block, 0));
-  return n;
+  return pack ? reinterpret_cast<const void*>(&population_kernel<TersoffPop<TWO>, true>)
+              : reinterpret_cast<const void*>(&population_kernel<TersoffPop<TWO>, false>);
 }
 
-int tersoff_population_occupancy(int cls, bool two, bool pack, int block)
+int tersoff_population_occupancy(bool two, bool pack, int block)
 {
-  switch (cls * 2 + (two ? 1 : 0)) {
-  case 0: return occ_t<4, false>(pack, block);
-  case 1: return occ_t<4, true>(pack, block);
-  case 2: return occ_t<8, false>(pack, block);
-  case 3: return occ_t<8, true>(pack, block);
-  case 4: return occ_t<16, false>(pack, block);
-  default: return occ_t<16, true>(pack, block);
-  }
+  int n = 0;
+  GPUGA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+    &n, two ? kernel_t<true>(pack) : kernel_t<false>(pack), block, 0));
+  return n;
 }
 
 } // namespace gpuga
