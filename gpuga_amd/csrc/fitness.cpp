@@ -672,21 +672,17 @@ void Fitness::setup_quad()
   GPUGA_HIP(hipStreamSynchronize(st));
   // column blocks of each form and their value blocks; U' enters the virials
   // and forces (U only inside NN2B's taper), U the energies
-  std::vector<int> col((size_t)6 * CE, -1), act;
-  std::vector<int2> vblk[3];
+  std::vector<int> col((size_t)6 * CE, -1), vblk[3];
+  std::vector<int2> act;
   int nb[3];
-  // (the columns of the species codes above 0 hold differences from code 0's)
-  auto value = [&](int first, int ce) {
-    return make_int2(first + ce, b.species() && ce >= E ? first + ce % E : -1);
-  };
   for (int f = 0; f < 3; ++f) {
     const int* u = &used[f == 2 ? (size_t)2 * CE : 0];
-    vblk[f].push_back(make_int2(2 * CE, -1));
+    vblk[f].push_back(2 * CE);
     auto add = [&](int map, int first, const int* used, int ce0, int ce1) {
       for (int ce = ce0; ce < ce1; ++ce)
         if (used[ce]) {
           col[(size_t)map * CE + ce] = (int)vblk[f].size();
-          vblk[f].push_back(value(first, ce));
+          vblk[f].push_back(first + ce);
         }
     };
     // code 0's columns before the differences (rigid ion: no differences)
@@ -698,8 +694,12 @@ void Fitness::setup_quad()
     }
     nb[f] = (int)vblk[f].size();
   }
-  for (int ce = 0; ce < CE; ++ce)
-    if (used[ce] || used[2 * CE + ce]) act.push_back(ce);
+  auto in_use = [&](int ce) { return used[ce] || used[2 * CE + ce]; };
+  for (int k = 0; k < (b.rigid ? CE : E); ++k) {
+    int mask = 0;
+    for (int c = 0; c < (b.rigid ? 1 : b.codes); ++c) mask |= in_use(c * E + k) ? 1 << c : 0;
+    if (mask) act.push_back(make_int2(k, mask));
+  }
   QuadRows rows;
   DeviceBuffer<int> d_col;
   d_col.upload(col, st);
@@ -754,6 +754,11 @@ void Fitness::setup_quad()
     }
     finish(2, part.get());
   }
+  std::vector<int2> unit;
+  for (int I = std::max({nb[0], nb[1], nb[2]}) - 1; I >= 0; --I)
+    for (int f = 0; f < 3; ++f)
+      if (I < nb[f]) unit.push_back(make_int2(f, I));
+  quad_.unit.upload(unit, st);
   GPUGA_HIP(hipStreamSynchronize(st));
   quad_.on = true;
 }
@@ -805,6 +810,8 @@ void Fitness::build_quad_plan(PopPlan& pl, int P)
   QuadEval& q = pl.qeval;
   for (int f = 0; f < 3; ++f)
     q.form[f] = QuadForm{quad_.nb[f], quad_.vblk[f].get(), quad_.q[f].get()};
+  q.unit = quad_.unit.get();
+  q.units = quad_.units();
   q.values = pl.qvalues.get();
   q.ld = ld;
   q.part = pl.qpart.get();
@@ -822,9 +829,18 @@ void Fitness::ensure_items(PopPlan& pl)
 
 void Fitness::launch_quad(PopPlan& pl, const PopCtl& ctl, hipStream_t st)
 {
-  if (quad_.basis.rigid) launch_ri_values(ctl, pl.qnodes, st);
-  else launch_nn2b_nodes(ctl, nn2b_grid_desc(), pl.qnodes, st);
+  launch_quad_values(pl, ctl, 0, pl.P, st);
   launch_quad_eval(ctl, pl.qeval, st);
+}
+
+void Fitness::launch_quad_values(PopPlan& pl, const PopCtl& ctl, int first, int count,
+                                 hipStream_t st)
+{
+  if (quad_.basis.rigid) launch_ri_values(ctl, pl.qnodes, st);
+  // (with the last individuals, the padding of the values)
+  else
+    launch_nn2b_nodes(ctl, nn2b_grid_desc(), pl.qnodes, first,
+                      first + count == pl.P ? pl.qnodes.ld - first : count, st);
 }
 
 NN2BGrid Fitness::nn2b_grid_desc() const
@@ -1280,8 +1296,6 @@ void Fitness::compute_async(int P, const float* genes, int share)
   // (a set with quadratic forms, genes outside their range: the pair loop)
   const bool quad = quad_for(P, genes);
   if (!quad) ensure_items(pl);
-  const size_t bytes = sizeof(float) * (size_t)P * spec_.V;
-  std::memcpy(pl.h_genes.get(), genes, bytes);
   // The generation is launched directly (a graph of one or two kernels takes
   // 14 us longer to launch and wait for), and its last kernel writes the
   // results to the pinned block: a copy back would be one more operation on
@@ -1291,18 +1305,28 @@ void Fitness::compute_async(int P, const float* genes, int share)
   ctl.fitness = reinterpret_cast<float*>(ctl.terms + 3 * (size_t)P);
   ctl.status = reinterpret_cast<unsigned*>(ctl.fitness + P);
   *ctl.status = 0u;
-  if (quad && quad_.basis.rigid) {
-    ctl.genes = pl.h_genes.get(); // (each value is read a few times)
-  } else {
-    // up to 64 KiB by a kernel: its launch costs less than a copy's
-    if (bytes <= 64u * 1024u) launch_copy_in(pl.h_genes.get(), pl.genes.get(), P * spec_.V, st);
-    else
-      GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), pl.h_genes.get(), bytes, hipMemcpyHostToDevice, st));
-  }
-  if (timing_) GPUGA_HIP(hipEventRecord(ev0_, st));
+  float* h = pl.h_genes.get();
   if (quad) {
-    launch_quad(pl, ctl, st);
+    // The genes are read in place, each once or a few times.  From 64 Ki genes
+    // on in two halves, the second one's copied while the first one's values
+    // are computed (256 x 1153: a call of 77 us, 89 in one piece, 83 in three).
+    ctl.genes = h;
+    if (timing_) GPUGA_HIP(hipEventRecord(ev0_, st));
+    const int parts = quad_.basis.rigid || (long)P * spec_.V < 65536 ? 1 : 2;
+    for (int k = 0; k < parts; ++k) {
+      const int p0 = (int)((long)P * k / parts), p1 = (int)((long)P * (k + 1) / parts);
+      const size_t at = (size_t)p0 * spec_.V;
+      std::memcpy(h + at, genes + at, sizeof(float) * (size_t)(p1 - p0) * spec_.V);
+      launch_quad_values(pl, ctl, p0, p1 - p0, st);
+    }
+    launch_quad_eval(ctl, pl.qeval, st);
   } else {
+    const size_t bytes = sizeof(float) * (size_t)P * spec_.V;
+    std::memcpy(h, genes, bytes);
+    // up to 64 KiB by a kernel: its launch costs less than a copy's
+    if (bytes <= 64u * 1024u) launch_copy_in(h, pl.genes.get(), P * spec_.V, st);
+    else GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), h, bytes, hipMemcpyHostToDevice, st));
+    if (timing_) GPUGA_HIP(hipEventRecord(ev0_, st));
     // share 1, 2, 4 or 8 (rounded up, at most 8): 1/share of the grid (the
     // quadratic forms' launches are short and fill a part of the GPU by
     // themselves)

@@ -84,8 +84,8 @@ struct QuadSet {
   int nb[3] = {0, 0, 0}; // column blocks of the energy, virial and force form
   int n_act = 0;
   DeviceBuffer<double> q[3];
-  DeviceBuffer<int2> vblk[3];
-  DeviceBuffer<int> act;
+  DeviceBuffer<int> vblk[3];
+  DeviceBuffer<int2> unit, act;
   size_t bytes() const
   {
     return q[0].bytes() + q[1].bytes() + q[2].bytes() + act.bytes();
@@ -228,8 +228,9 @@ private:
   // the population launch of ctl (the plan's, or a copy with other genes or
   // results); grid 0: the plan's
   void launch_population(PopPlan& pl, const PopCtl& ctl, hipStream_t st, int grid = 0);
-  // the same by the quadratic forms
+  // the same by the quadratic forms (their values, then their evaluation)
   void launch_quad(PopPlan& pl, const PopCtl& ctl, hipStream_t st);
+  void launch_quad_values(PopPlan& pl, const PopCtl& ctl, int first, int count, hipStream_t st);
   // n generations of the device GA from population buffer k, captured
   void capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph, hipGraphExec_t* exec);
   double time_plan(int P, const LaunchShape& sh, int reps, int* occ = nullptr);

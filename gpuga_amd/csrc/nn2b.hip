@@ -12,7 +12,6 @@
 // (src/nn2b.cu:143-148).
 #include "kernels.h"
 #include "population.h"
-#include "quadform.h"
 
 namespace gpuga {
 
@@ -25,34 +24,42 @@ __device__ inline size_t tab_index(int code, int K, int k, int G, int g, int q, 
   return ((((size_t)code * K + k) * G + g) * 3 + q) * WAVE + lane;
 }
 
-// The network and its derivatives at distance d (FP32): p, p' and, with DD,
-// p''.  w: the parameters (LDS); code: the pair's species code.  NMAX bounds
-// the neuron count for register-resident layers.
-template <int NMAX, bool DD>
-__device__ __forceinline__ void network(const float* w, int n, bool species, int code, float d,
-                                        float& pv, float& pd, float& pdd)
+// FP32 tabulation: block per individual (weights staged in LDS), thread per
+// grid point.  NMAX bounds the neuron count for register-resident layers.
+template <int NMAX>
+__global__ void __launch_bounds__(256) nn2b_tabulate_f32(PopCtl ctl, NN2BGrid grid,
+                                                         float* __restrict__ table)
 {
+  extern __shared__ float w[];
+  const int p = blockIdx.y, code = blockIdx.z;
+  const int n = grid.n, V = ctl.V;
+  for (int v = threadIdx.x; v < V; v += blockDim.x)
+    w[v] = denormalise(ctl.pmin[v], ctl.pmax[v], ctl.genes[(size_t)p * V + v]);
+  __syncthreads();
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= grid.G) return;
   const float* w0 = w;
   const float* b0 = w + n;
   const float* w1 = w + 2 * n;
   const float* b1 = w + n * (n + 2);
   const float* w2 = w + n * (n + 3);
   const float b2 = w[n * (n + 4)];
-  const float* ws = w + n * (n + 4) + 1; // species-pair weights
+  const float* ws = w + n * (n + 4) + 1; // species-pair weights (codes > 1)
+  const float d = grid.d0 + grid.h * g;
   float x1[NMAX], y1[NMAX], y2[NMAX];
 #pragma unroll
   for (int m = 0; m < NMAX; ++m) {
     if (m < n) {
       // the species-pair input as a shift of the bias (none for one code)
-      const float bm = species ? b0[m] - ws[m] * (float)code : b0[m];
+      const float bm = grid.codes > 1 ? b0[m] - ws[m] * (float)code : b0[m];
       const float t = ftanh(w0[m] * d - bm);
       const float s = 1.0f - t * t;
       x1[m] = t;
-      y1[m] = s * w0[m]; // d x1 / dr
-      if (DD) y2[m] = -2.0f * t * s * w0[m] * w0[m]; // d2 x1 / dr2
+      y1[m] = s * w0[m];                      // d x1 / dr
+      y2[m] = -2.0f * t * s * w0[m] * w0[m];  // d2 x1 / dr2
     }
   }
-  pv = pd = pdd = 0.0f;
+  float pv = 0.0f, pd = 0.0f, pdd = 0.0f;
   for (int a = 0; a < n; ++a) {
     float z = 0.0f, zd = 0.0f, zdd = 0.0f;
 #pragma unroll
@@ -61,59 +68,19 @@ __device__ __forceinline__ void network(const float* w, int n, bool species, int
         const float wm = w1[a * n + m];
         z += wm * x1[m];
         zd += wm * y1[m];
-        if (DD) zdd += wm * y2[m];
+        zdd += wm * y2[m];
       }
     }
     const float x2 = ftanh(z - b1[a]);
     const float s = 1.0f - x2 * x2;
     pv += w2[a] * x2;
     pd += w2[a] * s * zd;
-    if (DD) pdd += w2[a] * (s * zdd - 2.0f * x2 * s * zd * zd);
+    pdd += w2[a] * (s * zdd - 2.0f * x2 * s * zd * zd);
   }
-  pv -= b2;
-}
-
-// FP32 tabulation: block per individual (weights staged in LDS), thread per
-// grid point.
-template <int NMAX>
-__global__ void __launch_bounds__(256) nn2b_tabulate_f32(PopCtl ctl, NN2BGrid grid,
-                                                         float* __restrict__ table)
-{
-  extern __shared__ float w[];
-  const int p = blockIdx.y, code = blockIdx.z;
-  const int V = ctl.V;
-  for (int v = threadIdx.x; v < V; v += blockDim.x)
-    w[v] = denormalise(ctl.pmin[v], ctl.pmax[v], ctl.genes[(size_t)p * V + v]);
-  __syncthreads();
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= grid.G) return;
-  float pv, pd, pdd;
-  network<NMAX, true>(w, grid.n, grid.codes > 1, code, grid.d0 + grid.h * g, pv, pd, pdd);
   const int k = p / WAVE, lane = p % WAVE;
-  table[tab_index(code, ctl.K, k, grid.G, g, 0, lane)] = pv;
+  table[tab_index(code, ctl.K, k, grid.G, g, 0, lane)] = pv - b2;
   table[tab_index(code, ctl.K, k, grid.G, g, 1, lane)] = pd;
   table[tab_index(code, ctl.K, k, grid.G, g, 2, lane)] = pdd;
-}
-
-// The same at the nodes of the quadratic forms (p and p' only): block per
-// individual and 256 nodes.
-template <int NMAX>
-__global__ void __launch_bounds__(256) nn2b_nodes_f32(PopCtl ctl, NN2BGrid grid, NodeTable tab)
-{
-  extern __shared__ float w[];
-  const int p = blockIdx.y, V = ctl.V;
-  for (int v = threadIdx.x; v < V; v += blockDim.x)
-    w[v] = denormalise(ctl.pmin[v], ctl.pmax[v], ctl.genes[(size_t)min(p, ctl.P - 1) * V + v]);
-  __syncthreads();
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= tab.n_act * QB) return;
-  const int ce = tab.act[g / QB], m = g % QB;
-  float pv, pd, pdd;
-  network<NMAX, false>(w, grid.n, grid.codes > 1, ce / tab.b.E, node_at(tab.b, ce % tab.b.E, m),
-                       pv, pd, pdd);
-  double* o = tab.values + ((long)ce * QB + m) * tab.ld + p;
-  o[0] = pv;
-  o[(long)tab.b.CE() * QB * tab.ld] = pd;
 }
 
 } // namespace
@@ -266,30 +233,6 @@ void launch_nn2b_tabulate_f32(const PopCtl& ctl, const NN2BGrid& g, float* table
     nn2b_tabulate_f32<32><<<grid, block, lds, st>>>(ctl, g, table);
   else if (g.n <= 64)
     nn2b_tabulate_f32<64><<<grid, block, lds, st>>>(ctl, g, table);
-  else
-    fail("NN2B supports at most 64 neurons");
-  GPUGA_HIP(hipGetLastError());
-}
-
-void launch_nn2b_nodes_bf16(const PopCtl& ctl, const NN2BGrid& g, const NodeTable& t,
-                            hipStream_t st);
-
-void launch_nn2b_nodes(const PopCtl& ctl, const NN2BGrid& g, const NodeTable& t, hipStream_t st)
-{
-  if (g.bf16 && g.n <= 32) {
-    launch_nn2b_nodes_bf16(ctl, g, t, st);
-    return;
-  }
-  const dim3 block(256), grid((t.n_act * QB + 255) / 256, t.ld);
-  const size_t lds = sizeof(float) * ctl.V;
-  if (g.n <= 8)
-    nn2b_nodes_f32<8><<<grid, block, lds, st>>>(ctl, g, t);
-  else if (g.n <= 16)
-    nn2b_nodes_f32<16><<<grid, block, lds, st>>>(ctl, g, t);
-  else if (g.n <= 32)
-    nn2b_nodes_f32<32><<<grid, block, lds, st>>>(ctl, g, t);
-  else if (g.n <= 64)
-    nn2b_nodes_f32<64><<<grid, block, lds, st>>>(ctl, g, t);
   else
     fail("NN2B supports at most 64 neurons");
   GPUGA_HIP(hipGetLastError());

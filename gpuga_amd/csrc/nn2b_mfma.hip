@@ -16,7 +16,6 @@
 // output layer (src/nn2b.cu:71-77) through LDS in a fixed order.  n <= 32
 // (zero padded).
 #include "kernels.h"
-#include "quadform.h"
 
 namespace gpuga {
 
@@ -44,23 +43,19 @@ __device__ inline f32x16 mfma3(const bf16x8& ah, const bf16x8& al, const bf16x8&
 
 constexpr int TILE = 32;
 
-// NODES: the elements of the quadratic forms (a tile is an element's 32 nodes,
-// p and p' only) instead of the uniform grid.
-template <bool NODES>
 __global__ void __launch_bounds__(64) nn2b_tabulate_bf16(PopCtl ctl, NN2BGrid grid, int tiles,
-                                                         float* __restrict__ table, NodeTable tab)
+                                                         float* __restrict__ table)
 {
-  constexpr int NQ = NODES ? 2 : 3;
-  __shared__ float red[NQ][TILE][TILE + 1];
-  const int p = blockIdx.y;
+  __shared__ float red[3][TILE][TILE + 1];
+  const int p = blockIdx.y, code = blockIdx.z;
   const int l = threadIdx.x, col = l & 31, kg = l >> 5;
   const int n = grid.n, V = ctl.V;
-  const float* gp = ctl.genes + (size_t)(NODES ? min(p, ctl.P - 1) : p) * V;
+  const float* gp = ctl.genes + (size_t)p * V;
   auto W = [&](int v) { return denormalise(ctl.pmin[v], ctl.pmax[v], gp[v]); };
 
   // input neurons of this lane, in its A and B operands alike:
   // m = 16 s + 8 kg + j (K step s, element j)
-  float w0m[16], b0m[16], wsm[16];
+  float w0m[16], b0m[16];
   bf16x8 Bh[2], Bl[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -69,8 +64,9 @@ __global__ void __launch_bounds__(64) nn2b_tabulate_bf16(PopCtl ctl, NN2BGrid gr
       const int m = 16 * s + 8 * kg + j;
       const bool ok = m < n;
       w0m[8 * s + j] = ok ? W(m) : 0.0f;
-      b0m[8 * s + j] = ok ? W(n + m) : 0.0f;
-      wsm[8 * s + j] = ok && grid.codes > 1 ? W(n * (n + 4) + 1 + m) : 0.0f;
+      // the species-pair input (codes > 1) enters as a shift of the bias
+      b0m[8 * s + j] =
+        ok ? W(n + m) - (grid.codes > 1 ? W(n * (n + 4) + 1 + m) * (float)code : 0.0f) : 0.0f;
       split_bf16(ok && col < n ? W(2 * n + col * n + m) : 0.0f, Bh[s], Bl[s], j);
     }
   }
@@ -80,18 +76,9 @@ __global__ void __launch_bounds__(64) nn2b_tabulate_bf16(PopCtl ctl, NN2BGrid gr
   const int k = p / WAVE, lp = p % WAVE;
 
   for (int tt = 0; tt < tiles; ++tt) {
-    const int ti = blockIdx.x * tiles + tt, g0 = ti * TILE;
-    int ce = 0, code = blockIdx.z;
-    float d;
-    if constexpr (NODES) {
-      if (ti >= tab.n_act) break;
-      ce = tab.act[ti];
-      code = ce / tab.b.E;
-      d = node_at(tab.b, ce % tab.b.E, col);
-    } else {
-      if (g0 >= grid.G) break;
-      d = grid.d0 + grid.h * (float)(g0 + col);
-    }
+    const int g0 = (blockIdx.x * tiles + tt) * TILE;
+    if (g0 >= grid.G) break;
+    const float d = grid.d0 + grid.h * (float)(g0 + col);
     f32x16 Z = {0}, Zd = {0}, Zdd = {0};
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -99,16 +86,15 @@ __global__ void __launch_bounds__(64) nn2b_tabulate_bf16(PopCtl ctl, NN2BGrid gr
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float w = w0m[8 * s + j];
-        // the species-pair input (codes > 1) enters as a shift of the bias
-        const float t = ftanh(w * d - (b0m[8 * s + j] - wsm[8 * s + j] * (float)code));
+        const float t = ftanh(w * d - b0m[8 * s + j]);
         const float sg = 1.0f - t * t;
         split_bf16(t, AXh, AXl, j);
         split_bf16(sg * w, AYh, AYl, j);
-        if constexpr (!NODES) split_bf16(-2.0f * t * sg * w * w, AZh, AZl, j);
+        split_bf16(-2.0f * t * sg * w * w, AZh, AZl, j);
       }
       Z = mfma3(AXh, AXl, Bh[s], Bl[s], Z);
       Zd = mfma3(AYh, AYl, Bh[s], Bl[s], Zd);
-      if constexpr (!NODES) Zdd = mfma3(AZh, AZl, Bh[s], Bl[s], Zdd);
+      Zdd = mfma3(AZh, AZl, Bh[s], Bl[s], Zdd);
     }
     // this lane holds output neuron `col` for grid rows 8 (r/4) + 4 kg + r%4
 #pragma unroll
@@ -118,21 +104,17 @@ __global__ void __launch_bounds__(64) nn2b_tabulate_bf16(PopCtl ctl, NN2BGrid gr
       const float s = 1.0f - x2 * x2;
       red[0][row][col] = w2c * x2;
       red[1][row][col] = w2c * s * Zd[r];
-      if constexpr (!NODES) red[2][row][col] = w2c * (s * Zdd[r] - 2.0f * x2 * s * Zd[r] * Zd[r]);
+      red[2][row][col] = w2c * (s * Zdd[r] - 2.0f * x2 * s * Zd[r] * Zd[r]);
     }
     __syncthreads();
-    for (int idx = l; idx < NQ * TILE; idx += WAVE) {
+    for (int idx = l; idx < 3 * TILE; idx += WAVE) {
       const int q = idx / TILE, row = idx % TILE;
       float sum = 0.0f;
       for (int c = 0; c < TILE; ++c) sum += red[q][row][c];
       if (q == 0) sum -= b2;
-      if constexpr (NODES) {
-        tab.values[(((long)q * tab.b.CE() + ce) * QB + row) * tab.ld + p] = sum;
-      } else {
-        const int g = g0 + row;
-        if (g < grid.G)
-          table[((((size_t)code * ctl.K + k) * grid.G + g) * 3 + q) * WAVE + lp] = sum;
-      }
+      const int g = g0 + row;
+      if (g < grid.G)
+        table[((((size_t)code * ctl.K + k) * grid.G + g) * 3 + q) * WAVE + lp] = sum;
     }
     __syncthreads();
   }
@@ -151,19 +133,7 @@ void launch_nn2b_tabulate_bf16(const PopCtl& ctl, const NN2BGrid& g, float* tabl
   const int ntiles = (g.G + TILE - 1) / TILE;
   const int tiles = 4;
   const dim3 grid((ntiles + tiles - 1) / tiles, ctl.P, g.codes), block(64);
-  nn2b_tabulate_bf16<false><<<grid, block, 0, st>>>(ctl, g, tiles, table, NodeTable{});
-  GPUGA_HIP(hipGetLastError());
-}
-
-// (an element per wave: more of them than of the grid's tiles are wanted in
-// flight, and loading the weights is a small part of a tile)
-void launch_nn2b_nodes_bf16(const PopCtl& ctl, const NN2BGrid& g, const NodeTable& t,
-                            hipStream_t st)
-{
-  static_assert(TILE == QB, "a tile is an element");
-  const int tiles = 4;
-  const dim3 grid((t.n_act + tiles - 1) / tiles, t.ld), block(64);
-  nn2b_tabulate_bf16<true><<<grid, block, 0, st>>>(ctl, g, tiles, nullptr, t);
+  nn2b_tabulate_bf16<<<grid, block, 0, st>>>(ctl, g, tiles, table);
   GPUGA_HIP(hipGetLastError());
 }
 

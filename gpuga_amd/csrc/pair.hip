@@ -313,17 +313,6 @@ constexpr int NN2B_MAX_PLAIN = 64;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// tanh x = sgn(x) (1 - e) / (1 + e) and 1 - tanh^2 x = 4 e / (1 + e)^2 with
-// e = exp(-2 |x|): about 1e-7 absolute, the derivative without a difference
-// of nearly equal numbers.
-__device__ __forceinline__ void tanh_sech2(float x, float& t, float& s)
-{
-  const float e = fexp2(-2.0f * LOG2E * __builtin_fabsf(x));
-  const float r = frcp(1.0f + e);
-  t = __builtin_copysignf((1.0f - e) * r, x);
-  s = 4.0f * e * r * r;
-}
-
 // A wave takes NN2B_ATOMS consecutive atoms, whose bonds are consecutive, and
 // evaluates the network (src/nn2b.cu:49-78) for 32 bonds at a time: lane l
 // computes the first hidden layer and its derivative of bond l % 32 for the

@@ -51,8 +51,7 @@ __device__ inline float node_at(const QuadBasis& b, int e, int m)
 // (I, J <= I), the ones with J < I doubled, [column of J][row of I] each.
 struct QuadForm {
   int nb;
-  const int2* vblk; // [nb] value block of each column block, and the block
-                    // subtracted from it (-1: none)
+  const int* vblk; // [nb] value block of each column block
   const double* q;
 };
 constexpr long quad_tiles(long nb) { return nb * (nb + 1) / 2; }
@@ -60,6 +59,8 @@ constexpr long quad_tiles(long nb) { return nb * (nb + 1) / 2; }
 // Evaluation of all forms for a population: values [blocks][QB][ld].
 struct QuadEval {
   QuadForm form[3]; // energy, virial, force
+  const int2* unit; // [units] (form, row block), the longest rows first
+  int units;
   const double* values;
   int ld;           // individuals, padded to a multiple of QP
   double* part;     // [units][ld] row-block sums
@@ -69,7 +70,9 @@ struct QuadEval {
 // Where the tabulation kernels put U and U' of the nodes.
 struct NodeTable {
   QuadBasis b;
-  const int* act; // [n_act] elements (code E + e) some row uses
+  const int2* act; // [n_act] rigid ion: (code E + e, 1) that some row uses;
+                   // NN2B: element, mask of the codes that use it (code 0's
+                   // always, with the differences of the others)
   int n_act;
   double* values;
   int ld;
@@ -108,7 +111,9 @@ void launch_quad_gram(const double* R, int rows, int nb, int splits, bool first,
 void launch_quad_finish(const double* part, int nb, int splits, double* q, hipStream_t st);
 
 void launch_ri_values(const PopCtl& ctl, const NodeTable& t, hipStream_t st);
-void launch_nn2b_nodes(const PopCtl& ctl, const NN2BGrid& g, const NodeTable& t, hipStream_t st);
+// the individuals [first, first + count)
+void launch_nn2b_nodes(const PopCtl& ctl, const NN2BGrid& g, const NodeTable& t, int first,
+                       int count, hipStream_t st);
 void launch_quad_eval(const PopCtl& ctl, const QuadEval& q, hipStream_t st);
 
 } // namespace gpuga

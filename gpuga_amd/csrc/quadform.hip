@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(256) ri_values(PopCtl ctl, NodeTable tab)
     }
     return;
   }
-  const int ce = ldu(tab.act, blockIdx.x), t = ce / tab.b.E, el = ce % tab.b.E;
+  const int ce = ldu(tab.act, blockIdx.x).x, t = ce / tab.b.E, el = ce % tab.b.E;
   const double a = X(1 + 3 * t), rate = -1.0 / X(2 + 3 * t);
   double mR = 0.0, kR = 0.0, mA = 0.0, kA = 0.0, r0 = 0.0;
   if (t == 1) {
@@ -429,35 +429,36 @@ __global__ void __launch_bounds__(256) ri_values(PopCtl ctl, NodeTable tab)
 // blocks J <= I spread over its four waves: y = sum_J Q_IJ v_J on
 // v_mfma_f64_16x16x4_f64 (two products of 16 rows share the values'
 // operand), then v_I . y, which is linear in the waves' parts of y.  The last
-// workgroup of the QP individuals to finish sums the row blocks in order and
-// writes fitness and terms.
+// workgroup of the QP individuals to finish sums the row blocks in a fixed
+// order and writes fitness and terms.
 //
-// Bound by the latency of a wave's operand loads and of the hand-over to the
-// last workgroup, so a wave has few column blocks, and loads the next one's
-// operands before the products of one.  256 individuals on forms of 17
-// blocks: 18.3 us with a wave for all column blocks of 16 rows, 16.2 us so.
-__global__ void __launch_bounds__(256) quad_eval(PopCtl ctl, QuadEval q)
+// Bound by latency: launching (about 3 us), a wave's operand loads (about 5 us
+// here) and the hand-over to the last workgroup (two memory round trips, then
+// one for the sums, whose loads are spread over the workgroup; 6 us).  256
+// individuals on forms of 17 blocks: 18.3 us with one wave for all column
+// blocks of 16 rows, 16.2 us so; with eight waves, whose registers leave one
+// workgroup a CU, 21.8 us.  100 individuals on forms of about 46 blocks: 36.2
+// us with a unit's workgroups on all XCDs, each fetching the form, 21.8 us so.
+constexpr int EVAL_WAVES = 4;
+
+__global__ void __launch_bounds__(EVAL_WAVES * WAVE, 4) quad_eval(PopCtl ctl, QuadEval q)
 {
-  __shared__ double sh[4][QP], sums[3][QP];
+  constexpr int SLICES = EVAL_WAVES * WAVE / QP;
+  __shared__ double sh[EVAL_WAVES][QP], fold[3][SLICES][QP], sums[3][QP];
   __shared__ int last;
   const int lane = __lane_id(), w = wave_first((int)(threadIdx.x / WAVE));
-  // unit -> form and row block, the longest rows first
-  int f = 0, I = 0;
-  {
-    const int most = max(q.form[0].nb, max(q.form[1].nb, q.form[2].nb));
-    int u = blockIdx.x;
-    for (I = most - 1; I > 0; --I) {
-      int here = 0;
-      for (int s = 0; s < 3; ++s) here += I < q.form[s].nb;
-      if (u < here) break;
-      u -= here;
-    }
-    for (f = 0; f < 2; ++f)
-      if (I < q.form[f].nb && u-- == 0) break;
-  }
+  // workgroup -> unit (form and row block) and individuals: the workgroups of
+  // a unit run on one XCD (workgroup b on XCD b % 8), one after another, so a
+  // tile of Q comes from memory to one L2 once
+  const int groups = q.ld / QP;
+  const int unit = (int)blockIdx.x / kXcds / groups * kXcds + (int)blockIdx.x % kXcds;
+  const int pb = (int)blockIdx.x / kXcds % groups;
+  if (unit >= q.units) return;
+  const int2 fi = ldu(q.unit, unit);
+  const int f = fi.x, I = fi.y;
   const QuadForm F = f == 0 ? q.form[0] : f == 1 ? q.form[1] : q.form[2];
   const long ld = q.ld;
-  const int p0 = blockIdx.y * QP;
+  const int p0 = pb * QP;
   const double* A0 = F.q + quad_tiles(I) * QB * QB + (lane / 16) * QB + lane % 16;
   const double* V = q.values + p0 + lane % 16 + (lane / 16) * ld;
   struct Operands {
@@ -465,27 +466,21 @@ __global__ void __launch_bounds__(256) quad_eval(PopCtl ctl, QuadEval q)
   };
   auto load = [&](int J) {
     Operands o;
-    const int2 v = ldu(F.vblk, J);
     const double* A = A0 + (long)J * QB * QB;
-    const double* B = V + (long)v.x * QB * ld;
+    const double* B = V + (long)ldu(F.vblk, J) * QB * ld;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       o.a[0][k] = A[4 * k * QB];
       o.a[1][k] = A[4 * k * QB + 16];
       o.b[k] = B[4 * k * ld];
     }
-    if (v.y >= 0) {
-      const double* C = V + (long)v.y * QB * ld;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) o.b[k] -= C[4 * k * ld];
-    }
     return o;
   };
   f64x4 y[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
   if (w <= I) {
     Operands o = load(w);
-    for (int J = w; J <= I; J += 4) {
-      const Operands n = load(min(J + 4, I));
+    for (int J = w; J <= I; J += EVAL_WAVES) {
+      const Operands n = load(min(J + EVAL_WAVES, I));
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         y[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[0][k], o.b[k], y[0], 0, 0, 0);
@@ -495,49 +490,51 @@ __global__ void __launch_bounds__(256) quad_eval(PopCtl ctl, QuadEval q)
     }
   }
   // rows 16 h + 4 x + lane / 16, individual lane % 16
-  const int2 v = ldu(F.vblk, I);
-  const double* B = V + (long)v.x * QB * ld;
-  const double* C = V + (long)max(v.y, 0) * QB * ld;
+  const double* B = V + (long)ldu(F.vblk, I) * QB * ld;
   double sum = 0.0;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const long r = (16 * h + 4 * x) * ld;
-      sum = fma(v.y >= 0 ? B[r] - C[r] : B[r], y[h][x], sum);
-    }
+    for (int x = 0; x < 4; ++x) sum = fma(B[(16 * h + 4 * x) * ld], y[h][x], sum);
   sum += __shfl_xor(sum, 16);
   sum += __shfl_xor(sum, 32);
   if (lane < QP) sh[w][lane] = sum;
   __syncthreads();
   const int t = threadIdx.x;
-  const int nb0 = q.form[0].nb, nb1 = q.form[1].nb;
-  const int row = f == 0 ? I : f == 1 ? nb0 + I : nb0 + nb1 + I;
+  const int r0 = f == 0 ? 0 : f == 1 ? q.form[0].nb : q.form[0].nb + q.form[1].nb;
   double* part = q.part + p0;
   if (w == 0) {
-    if (lane < QP) cstore(part + row * ld + lane, (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]));
+    if (lane < QP) {
+      double x = 0.0;
+#pragma unroll
+      for (int u = 0; u < EVAL_WAVES; ++u) x += sh[u][lane];
+      cstore(part + (r0 + I) * ld + lane, x);
+    }
     publish();
-    const unsigned done = wave_atomic_add(&q.done[blockIdx.y], 1u);
-    if (lane == 0) last = done == gridDim.x - 1u;
+    const unsigned done = wave_atomic_add(&q.done[pb], 1u);
+    if (lane == 0) last = done == (unsigned)q.units - 1u;
   }
   __syncthreads();
   if (!last) return;
   observe();
-  if (t < 3 * QP) {
-    const int s = t / QP, l = t % QP;
-    const int r0 = s == 0 ? 0 : s == 1 ? nb0 : nb0 + nb1, n = q.form[s].nb;
+  // row block r of a form in slice r % SLICES, then the slices in order
+  const int l = t % QP, sl = t / QP;
+  int first = 0;
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
     double x = 0.0;
-    for (int r = 0; r < n; r += 16) {
-      double v[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = r + u < n ? cload(part + (r0 + r + u) * ld + l) : 0.0;
-#pragma unroll
-      for (int u = 0; u < 16; ++u) x += v[u];
-    }
-    // (a sum of squares; rounding may leave it just below zero)
-    sums[s][l] = x < 0.0 ? 0.0 : x;
+    for (int r = sl; r < q.form[s].nb; r += SLICES) x += cload(part + (first + r) * ld + l);
+    fold[s][sl][l] = x;
+    first += q.form[s].nb;
   }
-  if (t == 0) q.done[blockIdx.y] = 0u;
+  if (t == 0) q.done[pb] = 0u;
+  __syncthreads();
+  if (t < 3 * QP) {
+    double x = 0.0;
+    for (int u = 0; u < SLICES; ++u) x += fold[t / QP][u][l];
+    // (a sum of squares; rounding may leave it just below zero)
+    sums[t / QP][l] = x < 0.0 ? 0.0 : x;
+  }
   __syncthreads();
   if (t < QP) {
     const double s[3] = {sums[0][t], sums[1][t], sums[2][t]};
@@ -623,8 +620,8 @@ void launch_ri_values(const PopCtl& ctl, const NodeTable& t, hipStream_t st)
 
 void launch_quad_eval(const PopCtl& ctl, const QuadEval& q, hipStream_t st)
 {
-  const int units = q.form[0].nb + q.form[1].nb + q.form[2].nb;
-  quad_eval<<<dim3(units, q.ld / QP), 256, 0, st>>>(ctl, q);
+  const int blocks = (q.units + kXcds - 1) / kXcds * kXcds * (q.ld / QP);
+  quad_eval<<<blocks, EVAL_WAVES * WAVE, 0, st>>>(ctl, q);
   GPUGA_HIP(hipGetLastError());
 }
 
