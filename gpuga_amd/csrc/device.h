@@ -20,6 +20,7 @@ constexpr int kRiAtomConst = 27;
 
 struct DevSet {
   int Nc, Nc_force, N, N_force;
+  int max_nn;             // most neighbours of an atom
   const int* Na;          // [Nc]
   const int* Na_sum;      // [Nc]
   const int* type;        // [N]

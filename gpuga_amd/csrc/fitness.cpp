@@ -366,6 +366,7 @@ void Fitness::setup()
   v.Nc_force = ts_.Nc_force;
   v.N = ts_.N;
   v.N_force = ts_.N_force;
+  v.max_nn = nl_.max_nn;
   v.Na = ds_.Na.get();
   v.Na_sum = ds_.Na_sum.get();
   v.type = ds_.type.get();

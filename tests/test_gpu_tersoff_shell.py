@@ -57,3 +57,37 @@ def test_neighbour_bounds_match_oracle(k, two):
     ref, _ = O.Case(potential=pot, arrays=d).fitness(genes, threads=16)
     np.testing.assert_allclose(f, ref, rtol=1e-5)
     np.testing.assert_allclose(terms, plain, rtol=2e-5)
+
+
+@pytest.mark.parametrize("k,two", [(3, False), (4, True), (5, False)])
+def test_per_atom_outputs_of_few_neighbours(k, two):
+    """find_force of the one-pass kernel (at most four neighbours) and of the
+    two-kernel form above it, with atoms of 0 to k neighbours, the last atom of
+    the set among those without; 2e-5 of the largest magnitude, the bound of
+    every per-atom FP32 output."""
+    import gpuga_amd as G
+    from gpuga_amd import synth
+    from oracle import oracle as O
+    print_case("tersoff per-atom outputs", k, two)
+    rng = np.random.default_rng(k)
+    cells = []
+    for n in (k, 1, 2, k, 0):  # a centre with n neighbours, and one atom out of reach
+        th = np.arccos(np.linspace(0.9, -0.9, max(n, 1)))[:n]
+        ph = 2.4 * np.arange(n)
+        p = 2.4 * np.stack([np.cos(ph) * np.sin(th), np.sin(ph) * np.sin(th), np.cos(th)], 1)
+        p = np.concatenate([[[0, 0, 0]], p + rng.normal(0, 0.03, p.shape), [[9, 9, 9]]]) + 5.0
+        cells.append((np.diag([20.0] * 3), p, (np.arange(n + 2) % 2 if two else
+                                               np.zeros(n + 2)).astype(np.int32)))
+    d = synth._assemble(cells, 0.4, rng)
+    lo, hi = TWO if two else ONE
+    d.update(potential_type=2 if two else 1, cutoff=2.75, weights=(0.3, 0.3, 0.4), pmin=lo, pmax=hi,
+             pe_ref=np.ones(5, np.float32), virial_ref=np.ones(30, np.float32),
+             force_ref=np.ones(d["r"].size, np.float32))
+    pot = {x: d[x] for x in ("potential_type", "cutoff", "weights", "pmin", "pmax")}
+    params = (lo + (hi - lo) * rng.random(len(lo))).astype(np.float32)
+    with G.Fitness(arrays=d) as fit:
+        NN, _, _ = fit.neighbors()
+        got = fit.find_force(params)
+    assert NN.max() == k and NN[-1] == 0
+    for a, b in zip(got, O.Case(potential=pot, arrays=d).find_force(params)):
+        np.testing.assert_allclose(a, b, rtol=0, atol=2e-5 * np.abs(b).max())
