@@ -146,13 +146,12 @@ size_t DeviceSet::bytes() const
 
 void PopPlan::drop_ga_graphs()
 {
-  for (int k = 0; k < 2; ++k)
-    for (int j = 0; j < kGaGraphs; ++j) {
-      if (ga_exec[k][j]) (void)hipGraphExecDestroy(ga_exec[k][j]);
-      if (ga_graph[k][j]) (void)hipGraphDestroy(ga_graph[k][j]);
-      ga_exec[k][j] = nullptr;
-      ga_graph[k][j] = nullptr;
-    }
+  for (int k = 0; k < 2; ++k) {
+    if (ga_exec[k]) (void)hipGraphExecDestroy(ga_exec[k]);
+    if (ga_graph[k]) (void)hipGraphDestroy(ga_graph[k]);
+    ga_exec[k] = nullptr;
+    ga_graph[k] = nullptr;
+  }
 }
 
 PopPlan::~PopPlan() { drop_ga_graphs(); }
@@ -1370,8 +1369,6 @@ void Fitness::prepare(int P)
   if (opt_.backend != 1) plan(P);
 }
 
-static_assert((1 << (PopPlan::kGaGraphs - 1)) >= kGaMaxBatch, "a batch fits the largest graph");
-
 void Fitness::capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph,
                                   hipGraphExec_t* exec)
 {
@@ -1420,14 +1417,16 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
   // device starts after one generation's draws and the host then draws each
   // batch while the device runs the one before
   const int B = dga.batch();
-  // Every graph a batch can use (runs of 2^j generations on either
-  // population buffer) is captured before the first launch, on the first
-  // call: captured on first use, they cost the call that met them about
-  // 1-3 ms of host time with the device idle.
-  if (opt_.use_graph)
+  // Generations are launched directly, whole batches of a long run as graphs.
+  // A graph of few generations takes 14 us longer to launch than its kernels
+  // (ten generations of 50 individuals: 391 us in graphs of 1, 2, 4 and 2 + 1,
+  // 357 us launched directly), and capturing it costs the first call 1-3 ms;
+  // whole batches run equally fast either way and leave the host free to draw.
+  // Captured before the first launch: later, the device would wait idle.
+  const bool graphs = opt_.use_graph && B >= 8 && generations >= 3 * B;
+  if (graphs)
     for (int k = 0; k < 2; ++k)
-      for (int j = 0; j < PopPlan::kGaGraphs && (1 << j) <= B; ++j)
-        if (!pl.ga_exec[k][j]) capture_generations(pl, k, 1 << j, &pl.ga_graph[k][j], &pl.ga_exec[k][j]);
+      if (!pl.ga_exec[k]) capture_generations(pl, k, B, &pl.ga_graph[k], &pl.ga_exec[k]);
   const int H = dga.history_cap();
   std::vector<float> h((size_t)H * (1 + V));
   int g = 0; // generations queued
@@ -1438,30 +1437,22 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
     for (int b = 0, ramp = 1, nb = 0; b < n; b += nb, ramp = std::min(2 * ramp, B)) {
       nb = std::min({ramp, B, n - b});
       dga.stage(ga, first_generation + g + b, nb, st);
-      // the batch as runs of 2^j generations, each one graph (no launch
-      // gap between the generations inside a graph)
-      for (int i = 0; i < nb;) {
-        const int k = (g + b + i) & 1;
-        if (!opt_.use_graph) {
-          PopCtl ctl = pl.ctl;
-          ctl.genes = dga.genes(k);
-          if (quad) launch_quad(pl, ctl, st);
-          else launch_population(pl, ctl, st);
-          dga.step(k, pl.ctl.fitness, st);
-          ++i;
-          continue;
-        }
-        int j = 0;
-        while (j + 1 < PopPlan::kGaGraphs && (2 << j) <= nb - i) ++j;
-        if (!pl.ga_exec[k][j]) capture_generations(pl, k, 1 << j, &pl.ga_graph[k][j], &pl.ga_exec[k][j]);
-        GPUGA_HIP(hipGraphLaunch(pl.ga_exec[k][j], st));
-        i += 1 << j;
+      const int k0 = (g + b) & 1;
+      if (graphs && nb == B) {
+        GPUGA_HIP(hipGraphLaunch(pl.ga_exec[k0], st));
+        continue;
+      }
+      for (int i = 0; i < nb; ++i) {
+        const int k = k0 ^ (i & 1);
+        PopCtl ctl = pl.ctl;
+        ctl.genes = dga.genes(k);
+        if (quad) launch_quad(pl, ctl, st);
+        else launch_population(pl, ctl, st);
+        dga.step(k, pl.ctl.fitness, st);
       }
     }
     if (timing_) GPUGA_HIP(hipEventRecord(ev1_, st));
-    unsigned status = 0;
-    GPUGA_HIP(hipMemcpyAsync(&status, pl.ctl.status, sizeof status, hipMemcpyDeviceToHost, st));
-    GPUGA_HIP(hipStreamSynchronize(st));
+    const unsigned status = dga.collect((g + n) & 1, n, pl.ctl.status, st);
     if (timing_) {
       float ms = 0.0f;
       GPUGA_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));

@@ -19,7 +19,7 @@ namespace gpuga {
 struct FitnessOptions {
   int backend = 0;        // 0: population kernel, 1: per-individual launches
   int chunk_cost = 0;     // work-item cost target; 0 = autotune on first use
-  int use_graph = 1;      // run_ga: replay its generations from captured HIP graphs
+  int use_graph = 1;      // run_ga: replay whole batches of generations from HIP graphs
   int nn2b_bf16 = 1;      // NN2B hidden layer 2 on BF16 MFMA (else FP32)
   int nn2b_grid = 1024;   // NN2B tabulation points
   int verbose = 0;
@@ -116,14 +116,13 @@ struct PopPlan {
   PinnedBuffer<float> h_genes;
   PinnedBuffer<double> h_out;
   PopCtl ctl{};
-  // device GA of this population size; runs of generations (population
-  // launch + GA step each) as graphs: ga_exec[k][j] is 2^j generations
-  // starting on population buffer k (a generation on buffer b writes the
-  // next into buffer 1 - b)
-  static constexpr int kGaGraphs = 6; // runs of 1, 2, 4, ..., 32 generations
+  // device GA of this population size; a whole staged batch of generations
+  // (population launch + GA step each) as a graph: ga_exec[k] starts on
+  // population buffer k (a generation on buffer b writes the next into buffer
+  // 1 - b)
   std::unique_ptr<DeviceGA> dga;
-  hipGraph_t ga_graph[2][kGaGraphs] = {};
-  hipGraphExec_t ga_exec[2][kGaGraphs] = {};
+  hipGraph_t ga_graph[2] = {};
+  hipGraphExec_t ga_exec[2] = {};
   void drop_ga_graphs();
   ~PopPlan();
 };

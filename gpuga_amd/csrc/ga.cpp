@@ -377,6 +377,17 @@ void DeviceGA::upload(const GA& ga, int generation, hipStream_t st)
 {
   if (generation < 0) fail("generation numbers start at 0");
   const size_t PV = (size_t)d_.P * d_.V;
+  collected_ = false;
+  staged_ = 0;
+  if (PV <= kBlockWords) {
+    // (a run that ended early may not have been waited for)
+    if (begun_) GPUGA_HIP(hipStreamSynchronize(st));
+    in_.resize(PV);
+    std::memcpy(in_.get(), ga.population().data(), sizeof(float) * PV);
+    begun_ = true;
+    launch_ga_begin(d_, genes0_, in_.get(), generation, st);
+    return;
+  }
   GPUGA_HIP(hipMemcpyAsync(genes0_, ga.population().data(), sizeof(float) * PV,
                            hipMemcpyHostToDevice, st));
   const unsigned zero[2] = {0u, 0u};
@@ -384,7 +395,6 @@ void DeviceGA::upload(const GA& ga, int generation, hipStream_t st)
   GPUGA_HIP(hipMemcpyAsync(d_.generation, &generation, sizeof(int), hipMemcpyHostToDevice, st));
   GPUGA_HIP(hipMemcpyAsync(d_.history_gen0, &generation, sizeof(int), hipMemcpyHostToDevice, st));
   GPUGA_HIP(hipStreamSynchronize(st)); // the host values are stack/host memory
-  staged_ = 0;
 }
 
 void DeviceGA::restart_history(int generation, hipStream_t st)
@@ -447,9 +457,34 @@ void DeviceGA::step(int k, const float* fitness, hipStream_t st) const
   launch_ga_step(d, st);
 }
 
+unsigned DeviceGA::collect(int k, int n, const unsigned* status, hipStream_t st)
+{
+  if (n > d_.history_cap) fail("history beyond its capacity");
+  const size_t words = 1 + d_.P + (size_t)d_.P * d_.V + (size_t)n * (1 + d_.V);
+  collected_ = words <= kBlockWords;
+  if (collected_) {
+    out_.resize(words);
+    launch_ga_end(d_, genes(k), n, status, out_.get(), st);
+    GPUGA_HIP(hipStreamSynchronize(st));
+    begun_ = false;
+    return out_[0];
+  }
+  unsigned s = 0;
+  GPUGA_HIP(hipMemcpyAsync(&s, status, sizeof s, hipMemcpyDeviceToHost, st));
+  GPUGA_HIP(hipStreamSynchronize(st));
+  begun_ = false;
+  return s;
+}
+
 void DeviceGA::download(GA& ga, int k, hipStream_t st) const
 {
   const size_t PV = (size_t)d_.P * d_.V;
+  if (collected_) {
+    const float* sorted = reinterpret_cast<const float*>(out_.get() + 1);
+    std::memcpy(ga.fitness().data(), sorted, sizeof(float) * d_.P);
+    std::memcpy(ga.population().data(), sorted + d_.P, sizeof(float) * PV);
+    return;
+  }
   GPUGA_HIP(hipMemcpyAsync(ga.population().data(), genes(k), sizeof(float) * PV,
                            hipMemcpyDeviceToHost, st));
   GPUGA_HIP(hipMemcpyAsync(ga.fitness().data(), d_.sorted, sizeof(float) * d_.P,
@@ -460,6 +495,11 @@ void DeviceGA::download(GA& ga, int k, hipStream_t st) const
 void DeviceGA::history(float* out, int n, hipStream_t st) const
 {
   if (n > d_.history_cap) fail("history beyond its capacity");
+  if (collected_) {
+    std::memcpy(out, out_.get() + 1 + d_.P + (size_t)d_.P * d_.V,
+                sizeof(float) * (size_t)n * (1 + d_.V));
+    return;
+  }
   GPUGA_HIP(hipMemcpyAsync(out, d_.history, sizeof(float) * (size_t)n * (1 + d_.V),
                            hipMemcpyDeviceToHost, st));
   GPUGA_HIP(hipStreamSynchronize(st));

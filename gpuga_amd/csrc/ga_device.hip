@@ -226,7 +226,53 @@ __global__ void __launch_bounds__(GA_THREADS) ga_step(GaDev d)
   }
 }
 
+// The start of a run: population from the pinned block, counters and
+// generation number.
+__global__ void __launch_bounds__(256) ga_begin(GaDev d, float* __restrict__ genes,
+                                                const float* __restrict__ from, int generation)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < d.P * d.V) genes[i] = from[i];
+  if (i == 0) {
+    d.step[0] = 0u;
+    *d.done = 0u;
+    *d.generation = generation;
+    *d.history_gen0 = generation;
+  }
+}
+
+// The end of a run into the pinned block: status | sorted fitness | population
+// | n history rows.
+__global__ void __launch_bounds__(256) ga_end(GaDev d, const float* __restrict__ genes, int n,
+                                              const unsigned* __restrict__ status,
+                                              unsigned* __restrict__ to)
+{
+  const int i = blockIdx.x * 256 + threadIdx.x, PV = d.P * d.V;
+  float* sorted = reinterpret_cast<float*>(to + 1);
+  float* pop = sorted + d.P;
+  float* hist = pop + PV;
+  if (i == 0) to[0] = *status;
+  if (i < d.P) sorted[i] = d.sorted[i];
+  if (i < PV) pop[i] = genes[i];
+  if (i < n * (1 + d.V)) hist[i] = d.history[i];
+}
+
 } // namespace
+
+void launch_ga_begin(const GaDev& d, float* genes, const float* from, int generation,
+                     hipStream_t st)
+{
+  ga_begin<<<(d.P * d.V + 255) / 256, 256, 0, st>>>(d, genes, from, generation);
+  GPUGA_HIP(hipGetLastError());
+}
+
+void launch_ga_end(const GaDev& d, const float* genes, int n, const unsigned* status,
+                   unsigned* to, hipStream_t st)
+{
+  const int most = std::max({d.P, d.P * d.V, n * (1 + d.V)});
+  ga_end<<<(most + 255) / 256, 256, 0, st>>>(d, genes, n, status, to);
+  GPUGA_HIP(hipGetLastError());
+}
 
 // rows per workgroup and LDS bytes of a step of shape (P, V)
 void ga_step_shape(int P, int V, int* rows, size_t* lds)

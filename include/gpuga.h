@@ -26,8 +26,9 @@ typedef struct gpuga_options {
   int chunk_cost; /* work-item size of the population launch; 0 = autotune
                      the launch shape (this and the fields below left at 0
                      or, for pack_lanes, at 1) */
-  int use_graph;  /* 1: gpuga_fitness_run_ga replays its generations from HIP
-                     graphs; 0: it launches them one by one */
+  int use_graph;  /* 1: gpuga_fitness_run_ga replays whole batches of a long
+                     run's generations from HIP graphs; 0: it launches every
+                     generation by itself */
   int nn2b_bf16;  /* 1: NN2B hidden layer on BF16 MFMA; 0: FP32 */
   int nn2b_grid;  /* NN2B tabulation points (default 1024) */
   int verbose;

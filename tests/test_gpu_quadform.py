@@ -123,15 +123,16 @@ def test_genes_outside_the_bounds_take_the_pair_loop():
     np.testing.assert_allclose(f, ref, rtol=1e-5)
 
 
-@pytest.mark.parametrize("kind", ["ri", "dimers"])
-def test_device_generations_equal_the_host_loop(kind):
+@pytest.mark.parametrize("kind,P", [("ri", 30), ("dimers", 30), ("large", 64)])
+def test_device_generations_equal_the_host_loop(kind, P):
+    """large: 64 x 1021 genes, which start from one pinned block but, with the
+    history, do not return in one."""
     import gpuga_amd as G
     print_case("quadratic forms, device GA", kind)
-    d = _ri() if kind == "ri" else _dimers(40, 20, 6, 6)
-    P = 30
+    d = _ri() if kind == "ri" else _dimers(40, 20, 30 if kind == "large" else 6, 6)
     with G.Fitness(arrays=d, nn2b_bf16=0) as fit:
-        host = G.GA(P, 16, fit.V, maximum_generation=40, seed=3)
-        dev = G.GA(P, 16, fit.V, maximum_generation=40, seed=3)
+        host = G.GA(P, P // 2 + P // 2 % 2, fit.V, maximum_generation=40, seed=3)
+        dev = G.GA(P, P // 2 + P // 2 % 2, fit.V, maximum_generation=40, seed=3)
         best = []
         for k in range(5):
             f = fit.compute(host.population)
