@@ -439,8 +439,10 @@ __device__ inline double group_sum(double x, int W)
 // loads each next atom's record during the current one and reads its rows
 // from the wave's LDS copy (Pot::chunk<true, true>; only with kHeaderAhead
 // and without PACK).
+// (at least two waves per SIMD: the widest instantiations would take registers
+// past the 256 that allows)
 template <class Pot, bool PACK = false, bool LONE = false>
-__global__ void __launch_bounds__(256) population_kernel(PopCtl ctl, DevSet set,
+__global__ void __launch_bounds__(256, 2) population_kernel(PopCtl ctl, DevSet set,
                                                          typename Pot::Extra ex)
 {
   const int lane = __lane_id();

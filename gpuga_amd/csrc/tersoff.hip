@@ -103,6 +103,7 @@ __global__ void __launch_bounds__(128) tersoff_plain_forces(DevSet s, TLane q,
   if (i >= s.N) return;
   const int nn = s.nn[i], b0 = s.bond0[i];
   const float4* T = s.tri + (nn > 0 ? s.tri0[i] : 0);
+  const TSets sets = tersoff_sets(q);
   float4 r[M], t[M][M];
   int type[M];
   // (loads past the last neighbour repeat it, so that all are in flight
@@ -135,7 +136,7 @@ __global__ void __launch_bounds__(128) tersoff_plain_forces(DevSet s, TLane q,
       }
       float b, bp, fr, frp, fa, fap;
       tersoff_bond_order(q, zeta, b, bp);
-      tersoff_pair_sel(q, type[u] & 1, r[u].w, fr, frp, fa, fap);
+      tersoff_pair_sel(sets, type[u] & 1, r[u].w, fr, frp, fa, fap);
       A[u] = bp * fa;
       e += fc[u] * (fr - b * fa) * 0.5f;
       pf[u] = (fcp[u] * (fr - b * fa) + fc[u] * (frp - b * fap)) * dinv[u];

@@ -89,16 +89,40 @@ __device__ __forceinline__ void tersoff_pair(const TLane& q, int k, float d, flo
   fap = q.kA[k] * fa;
 }
 
-// The same of set 1 where `second` (wave-uniform), else 0, as selects (a
-// run-time index, which a branch may become, puts the sets in scratch memory).
-__device__ __forceinline__ void tersoff_pair_sel(const TLane& q, bool second, float d, float& fr,
+// Both sets' constants as plain values, for a choice between them by selects:
+// a select between members of a TLane in memory becomes a load from a selected
+// address, and the sets stay in scratch memory (the empty asm keeps the
+// compiler from seeing where the values come from).
+struct TSets {
+  float v[2][7]; // cR, kR, kR2, cA, kA, kA2, r0
+};
+__device__ __forceinline__ TSets tersoff_sets(const TLane& q)
+{
+  TSets t;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const float v[7] = {q.cR[k], q.kR[k], q.kR2[k], q.cA[k], q.kA[k], q.kA2[k], q.r0[k]};
+#pragma unroll
+    for (int m = 0; m < 7; ++m) {
+      t.v[k][m] = v[m];
+      asm volatile("" : "+v"(t.v[k][m]));
+    }
+  }
+  return t;
+}
+
+// tersoff_pair of set 1 where `second` (wave-uniform), else of set 0
+__device__ __forceinline__ void tersoff_pair_sel(const TSets& t, bool second, float d, float& fr,
                                                  float& frp, float& fa, float& fap)
 {
-  const float x = d - (second ? q.r0[1] : q.r0[0]);
-  fr = (second ? q.cR[1] : q.cR[0]) * fexp2((second ? q.kR2[1] : q.kR2[0]) * x);
-  frp = (second ? q.kR[1] : q.kR[0]) * fr;
-  fa = (second ? q.cA[1] : q.cA[0]) * fexp2((second ? q.kA2[1] : q.kA2[0]) * x);
-  fap = (second ? q.kA[1] : q.kA[0]) * fa;
+  float c[7];
+#pragma unroll
+  for (int m = 0; m < 7; ++m) c[m] = second ? t.v[1][m] : t.v[0][m];
+  const float x = d - c[6];
+  fr = c[0] * fexp2(c[2] * x);
+  frp = c[1] * fr;
+  fa = c[3] * fexp2(c[5] * x);
+  fap = c[4] * fa;
 }
 
 // Individual p's constants from its genes (every lane of a wave calls it).

@@ -45,16 +45,22 @@ __device__ __forceinline__ void upto(F&& f)
 
 // The per-bond values of an atom in registers, every loop unrolled, left by a
 // scalar branch after the atom's last bond: an atom with fewer neighbours
-// than M does no padded work.
+// than M does no padded work.  The record comes through LDS (the next atom's
+// loads in flight during this one): its broadcast reads return in order and
+// are waited for one by one, and the unit vectors do not fill the scalar
+// registers.  What the pair loops do not touch (fc' / d, the pair part) waits
+// in LDS rows, and a scheduling barrier every four pairs keeps their reads from
+// moving ahead of one another, so that two waves fit a SIMD.
 //
-// Bound by the VALU: 20 instructions a pair and about 60 a bond, at one or
-// two waves a SIMD (214 VGPRs for 16 neighbours, 251 for 20).  The looped
-// kernel, which takes any number of neighbours with its per-bond values in
-// LDS and every load waited for in turn, took 332 us on 6 400 atoms with up
-// to 18 neighbours (15.6 on average), two lane blocks; this form 129 us.  On
-// sets of 12, 14 and 16 neighbours it is 3.5 to 11 times as fast as bodies of
-// ordered pairs with guards, which spilled to scratch (5 400 atoms of 8.3
-// neighbours, 200 individuals: a call of 454 -> 124 us).
+// Bound by the VALU (20 instructions a pair, about 60 a bond) at two waves a
+// SIMD.  The looped kernel, which takes any number of neighbours with its
+// per-bond values in LDS and every load waited for in turn, took 332 us on
+// 6 400 atoms with up to 18 neighbours (15.6 on average), two lane blocks;
+// this form 112 us (129 us with the record in scalar registers; twice as many
+// registers, one wave a SIMD, without the barriers: 180 us).  On sets of 12, 14
+// and 16 neighbours it is 4 to 11 times as fast as bodies of ordered pairs
+// with guards, which spilled to scratch (5 400 atoms of 8.3 neighbours, 200
+// individuals: a call of 454 -> 113 us).
 template <int M, bool TWO>
 struct TersoffShell {
   static constexpr bool kForcePass = true;
@@ -67,20 +73,27 @@ struct TersoffShell {
 
   __device__ static Lane make(const PopCtl& ctl, int p) { return tersoff_make<TWO>(ctl, p); }
 
+  // R: the atom's record in LDS; FCP, PF: LDS rows of the wave's lanes for the
+  // values that the pair loops do not touch (fc' / d, the pair part of f_ij)
   template <bool FORCE>
-  __device__ static void atom(const DevSet& s, const float4* rec, const TLane& q, int i,
-                              float* fblk, int lane, Acc& acc)
+  __device__ static void atom(const DevSet& s, const float4* R, float* FCP, float* PF,
+                              const TLane& q, int i, int nn, int unl, float* fblk, int lane,
+                              Acc& acc)
   {
-    const float4* R = rec + (long)i * RS;
-    const int* H = reinterpret_cast<const int*>(R);
     const float* C = reinterpret_cast<const float*>(R + shell_first_cos(M));
-    const int nn = ldu(H, 0), unl = TWO ? ldu(H, 1) : 0;
-    float fc[M], fcp[M], z[M];
+    // (an empty asm between the passes: the compiler would keep the first
+    // pass's reads of the record for the second one)
+    constexpr int STEP = 4; // pairs between scheduling barriers
+    auto pass = [] { asm volatile("" ::: "memory"); };
+    TSets sets;
+    if constexpr (TWO) sets = tersoff_sets(q);
+    float fc[M], z[M];
     upto<M>([&](auto U) {
       constexpr int u = U;
       if (u < nn) {
-        tersoff_fc(q, ldu(R, 1 + u).w, fc[u], fcp[u]);
-        fcp[u] *= ldu(R, 1 + M + u).w;
+        float fcp;
+        tersoff_fc(q, R[1 + u].w, fc[u], fcp);
+        FCP[u * WAVE + lane] = fcp * R[1 + M + u].w;
         z[u] = 0.0f;
       }
     });
@@ -89,35 +102,38 @@ struct TersoffShell {
       if (v > 0 && v < nn)
         upto<v>([&](auto U) {
           constexpr int u = U;
-          const float x = ldu(C, shell_cos(v) + u) - q.h;
+          const float x = C[shell_cos(v) + u] - q.h;
           const float x2 = x * x;
           z[u] = fmaf(fc[v], x2, z[u]);
           z[v] = fmaf(fc[u], x2, z[v]);
         });
     });
-    float e = 0.0f, B[M], pf[M], cx[M], cy[M], cz[M], m[M], ds[M];
+    pass();
+    float e = 0.0f, B[M], cx[M], cy[M], cz[M], m[M], ds[M];
     upto<M>([&](auto U) {
       constexpr int u = U;
       if (u < nn) {
         float b, bp, fr, frp, fa, fap;
         tersoff_bond_order(q, q.beta * z[u], b, bp);
-        const float d = ldu(R, 1 + u).w;
-        tersoff_pair_sel(q, TWO && ((unl >> u) & 1), d, fr, frp, fa, fap);
+        const float d = R[1 + u].w;
+        if constexpr (TWO) tersoff_pair_sel(sets, (unl >> u) & 1, d, fr, frp, fa, fap);
+        else tersoff_pair(q, 0, d, fr, frp, fa, fap);
         const float rep = fr - b * fa;
         e = fmaf(fc[u], rep, e);
-        pf[u] = fmaf(fcp[u], rep, fc[u] * (frp - b * fap) * ldu(R, 1 + M + u).w);
+        PF[u * WAVE + lane] = fmaf(FCP[u * WAVE + lane], rep, fc[u] * (frp - b * fap) * R[1 + M + u].w);
         B[u] = bp * fa * fc[u];
         cx[u] = cy[u] = cz[u] = m[u] = ds[u] = 0.0f;
       }
     });
+    pass();
     upto<M>([&](auto V) {
       constexpr int v = V;
       if (v > 0 && v < nn) {
-        const float4 ev = ldu(R, 1 + M + v);
+        const float4 ev = R[1 + M + v];
         upto<v>([&](auto U) {
           constexpr int u = U;
-          const float c = ldu(C, shell_cos(v) + u), x = c - q.h, x2 = x * x;
-          const float4 eu = ldu(R, 1 + M + u);
+          const float c = C[shell_cos(v) + u], x = c - q.h, x2 = x * x;
+          const float4 eu = R[1 + M + u];
           const float S = fmaf(fc[v], B[u], fc[u] * B[v]) * x;
           const float Sc = S * c;
           cx[u] = fmaf(S, ev.x, cx[u]);
@@ -130,21 +146,23 @@ struct TersoffShell {
           m[v] += Sc;
           ds[u] = fmaf(B[v], x2, ds[u]);
           ds[v] = fmaf(B[u], x2, ds[v]);
+          if constexpr (u % STEP == STEP - 1) __builtin_amdgcn_sched_barrier(0);
         });
       }
     });
+    pass();
     float wxx = 0, wyy = 0, wzz = 0, wxy = 0, wyz = 0, wzx = 0;
     upto<M>([&](auto U) {
       constexpr int u = U;
       if (u < nn) {
-        const float4 r = ldu(R, 1 + u), eu = ldu(R, 1 + M + u);
-        const float coef = 0.5f * (pf[u] - fcp[u] * (q.beta * ds[u]));
+        const float4 r = R[1 + u], eu = R[1 + M + u];
+        const float coef = 0.5f * (PF[u * WAVE + lane] - FCP[u * WAVE + lane] * (q.beta * ds[u]));
         const float hc = q.beta * eu.w;
         const float fx = fmaf(coef, r.x, -hc * fmaf(-m[u], eu.x, cx[u]));
         const float fy = fmaf(coef, r.y, -hc * fmaf(-m[u], eu.y, cy[u]));
         const float fz = fmaf(coef, r.z, -hc * fmaf(-m[u], eu.z, cz[u]));
         if (FORCE) {
-          const int rb = ldu(reinterpret_cast<const int*>(R + 1 + 2 * M), u);
+          const int rb = wave_first(reinterpret_cast<const int*>(R + 1 + 2 * M)[u]);
           float* o = fblk + (size_t)rb * 3 * WAVE + lane;
           cstore(o, fx);
           cstore(o + WAVE, fy);
@@ -178,16 +196,48 @@ struct TersoffShell {
     }
   }
 
+  // A record spread over the wave, word 64 k + l in register k of lane l.
+  static constexpr int RW = RS * 4, NW = (RW + WAVE - 1) / WAVE;
+  struct Spread {
+    int w[NW];
+  };
+  __device__ static Spread spread_load(const float4* rec, int i)
+  {
+    const int* w = reinterpret_cast<const int*>(rec + (long)i * RS);
+    Spread v;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) v.w[k] = w[min(WAVE * k + (int)__lane_id(), RW - 1)];
+    return v;
+  }
+  __device__ static void spread_store(float4* buf, const Spread& v)
+  {
+    int* w = reinterpret_cast<int*>(buf);
+#pragma unroll
+    for (int k = 0; k < NW; ++k)
+      if (WAVE * k + (int)__lane_id() < RW) w[WAVE * k + __lane_id()] = v.w[k];
+  }
+
   __device__ static void chunk(const DevSet& s, const TLane& q, const WorkItem& it,
                                const PopCtl& ctl, const float4* rec, Acc& acc)
   {
-    const int lane = __lane_id();
-    if (it.c < s.Nc_force) {
-      float* fblk = ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE;
-      for (int i = it.a0; i < it.a1; ++i) atom<true>(s, rec, q, i, fblk, lane, acc);
-    } else {
-      for (int i = it.a0; i < it.a1; ++i) atom<false>(s, rec, q, i, nullptr, lane, acc);
-    }
+    __shared__ float4 buf[256 / WAVE][RS];
+    __shared__ float side[256 / WAVE][2][M * WAVE];
+    const int lane = __lane_id(), w = wave_first((int)(threadIdx.x / WAVE));
+    float4* R = buf[w];
+    Spread v = spread_load(rec, it.a0);
+    auto run = [&](auto force) {
+      constexpr bool F = decltype(force)::value;
+      float* fblk = F ? ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE : nullptr;
+      for (int i = it.a0; i < it.a1; ++i) {
+        const int nn = __builtin_amdgcn_readlane(v.w[0], 0);
+        const int unl = TWO ? __builtin_amdgcn_readlane(v.w[0], 1) : 0;
+        spread_store(R, v); // (LDS operations of a wave stay in order)
+        v = spread_load(rec, min(i + 1, it.a1 - 1));
+        atom<F>(s, R, side[w][0], side[w][1], q, i, nn, unl, fblk, lane, acc);
+      }
+    };
+    if (it.c < s.Nc_force) run(std::true_type{});
+    else run(std::false_type{});
   }
 
   // F_i = sum_j (f_ij - f_ji), then sum_i |F_i - F_ref,i|^2
