@@ -11,13 +11,20 @@ namespace gpuga {
 
 constexpr int WAVE = 64; // CDNA wavefront width
 
-// Read-only training set in HBM: per-atom SoA arrays, CSR neighbour list and
-// the parameter-independent geometry tables.
 // doubles per pair type of a configuration's RI sums (ri_cconst), floats
 // per force atom (ri_fconst)
 constexpr int kRiTypeConst = 22;
 constexpr int kRiAtomConst = 27;
 
+// words of a moment record, first word and words of a bond, and the cosine
+// that its moments are taken about (near the tetrahedral -1/3 and short in
+// binary, so that h less it is exact for the usual h)
+constexpr int kMomWords = 80;
+constexpr int kMomBond = 16;
+constexpr float kMomCos = -0.34375f;
+
+// Read-only training set in HBM: per-atom SoA arrays, CSR neighbour list and
+// the parameter-independent geometry tables.
 struct DevSet {
   int Nc, Nc_force, N, N_force;
   int max_nn;             // most neighbours of an atom
@@ -40,6 +47,16 @@ struct DevSet {
   // an atom is independent of the others, so they issue together.
   const float4* rec;
   int rec_nmax;
+  // Moment records of the energy configurations' atoms with four bonds (the
+  // Tersoff population kernel; atom N_force + i at i kMomWords floats).  With
+  // c'_uv = cos theta_uv - kMomCos and G_uv = r_u (x) d cos / d r_u + r_v (x)
+  // d cos / d r_v of bonds u, v: four distances; four sums over v of 2 c';
+  // four of c'^2; then the longest bond's length (+inf for an atom of fewer
+  // bonds, or with bonds of both kinds) and its unlike-type bit mask as int;
+  // two unused; then per bond u -r_a r_b / 2 d (xx, yy, zz, xy, yz, zx), the
+  // sums over v of c' G (xx, yy, xy, yz, zx; G is symmetric and traceless)
+  // and of G.  Null where the set has no use for them.
+  const float* mom;
   int bond_force;         // bonds of the force configurations (they come first)
   // Pair-potential population tables.  An atom's pairs are all its bonds in
   // a force configuration and those with j > i otherwise.

@@ -53,7 +53,7 @@ struct DeviceSet {
   DeviceBuffer<int> p_nn, p_b0, p_nl, p_rev, p_ptype, p_tri0;
   DeviceBuffer<float4> p_bond, p_tri;
   DeviceBuffer<int4> pair_hdr;
-  DeviceBuffer<float> pe_ref, virial_ref, force_ref;
+  DeviceBuffer<float> pe_ref, virial_ref, force_ref, mom;
   DeviceBuffer<double> ri_cconst;
   DeviceBuffer<float> ri_fconst;
   DevSet view{};

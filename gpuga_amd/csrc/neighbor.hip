@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "device.h"
 #include "trainset.h"
 
 namespace gpuga {
@@ -214,6 +215,68 @@ __global__ void __launch_bounds__(256) geo_records(int N, int M, const int* NN, 
   }
 }
 
+// Moment record (device.h) of atom i0 + blockIdx.x * 64 + threadIdx.x / 4,
+// bond threadIdx.x % 4 (and its share of the first words); *inside: atoms whose
+// record serves an R1 of r1.
+__global__ void __launch_bounds__(256) geo_moments(int i0, int N, const int* NN, const int* start,
+                                                   const int* ptype, const float4* bond, float r1,
+                                                   float* mom, int* inside)
+{
+  const int i = i0 + blockIdx.x * 64 + threadIdx.x / 4, u = threadIdx.x % 4;
+  if (i >= N) return;
+  float* M = mom + (long)(i - i0) * kMomWords;
+  float* B = M + kMomBond * (1 + u);
+  const int b0 = start[i];
+  if (NN[i] != 4) {
+    for (int k = 0; k < kMomBond; ++k) B[k] = 0.0f;
+    for (int k = 0; k < 4; ++k) M[4 * u + k] = 4 * u + k == 12 ? __builtin_inff() : 0.0f;
+    return;
+  }
+  double e[4][3];
+  float dmax = 0.0f;
+  int mask = 0;
+  for (int v = 0; v < 4; ++v) {
+    const float4 r = bond[b0 + v];
+    const double d2 = (double)r.x * r.x + (double)r.y * r.y + (double)r.z * r.z;
+    const double inv = 1.0 / sqrt(d2);
+    e[v][0] = r.x * inv;
+    e[v][1] = r.y * inv;
+    e[v][2] = r.z * inv;
+    dmax = fmaxf(dmax, r.w);
+    mask |= (ptype[b0 + v] & 1) << v;
+  }
+  const int A[6] = {0, 1, 2, 0, 1, 2}, C[6] = {0, 1, 2, 1, 2, 0}; // xx yy zz xy yz zx
+  double c1 = 0.0, c2 = 0.0, q1[6] = {0}, q0[6] = {0};
+  for (int v = 0; v < 4; ++v) {
+    if (v == u) continue;
+    const double c = e[u][0] * e[v][0] + e[u][1] * e[v][1] + e[u][2] * e[v][2];
+    const double cs = c - (double)kMomCos;
+    c1 += cs;
+    c2 += cs * cs;
+    for (int k = 0; k < 6; ++k) {
+      const double g = e[u][A[k]] * e[v][C[k]] + e[v][A[k]] * e[u][C[k]] -
+                       c * (e[u][A[k]] * e[u][C[k]] + e[v][A[k]] * e[v][C[k]]);
+      q0[k] += g;
+      q1[k] += cs * g;
+    }
+  }
+  const float4 r = bond[b0 + u];
+  M[u] = r.w;
+  M[4 + u] = (float)(2.0 * c1);
+  M[8 + u] = (float)c2;
+  const float reach = mask == 0 || mask == 15 ? dmax : __builtin_inff();
+  M[12 + u] = u == 0 ? reach : u == 1 ? __int_as_float(mask) : 0.0f;
+  if (u == 0 && reach < r1) atomicAdd(inside, 1);
+  const double x[3] = {r.x, r.y, r.z};
+  for (int k = 0; k < 6; ++k) B[k] = (float)(-0.5 * x[A[k]] * x[C[k]] / (double)r.w);
+  for (int k = 0, j = 0; k < 6; ++k) {
+    if (k == 2) continue; // zz = -xx - yy
+    B[6 + j] = (float)q1[k];
+    B[11 + j] = (float)q0[k];
+    ++j;
+  }
+}
+
 #pragma clang fp contract(on)
 
 // Device copies of the positions, boxes and configuration index.
@@ -290,6 +353,21 @@ void build_records_device(int N, int M, const DeviceNeighbors& d, const int* pty
   geo_records<<<(unsigned)blocks, 256, 0, st>>>(N, M, d.NN, d.start, d.rev, ptype, d.tri0, bond,
                                                 tri, rec);
   GPUGA_HIP(hipGetLastError());
+}
+
+int build_moments_device(int i0, int N, const DeviceNeighbors& d, const int* ptype,
+                         const float4* bond, float r1, float* mom, hipStream_t st)
+{
+  if (N <= i0) return 0;
+  DeviceBuffer<int> count;
+  int inside = 0;
+  count.upload(&inside, 1, st);
+  geo_moments<<<(N - i0 + 63) / 64, 256, 0, st>>>(i0, N, d.NN, d.start, ptype, bond, r1, mom,
+                                                  count.get());
+  GPUGA_HIP(hipGetLastError());
+  count.download(&inside, 1, st);
+  GPUGA_HIP(hipStreamSynchronize(st));
+  return inside;
 }
 
 NeighborList build_neighbors_device(const TrainSet& ts, float cutoff, hipStream_t st)

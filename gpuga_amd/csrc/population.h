@@ -150,6 +150,27 @@ __device__ __forceinline__ T cload(const T* p)
 __device__ __forceinline__ void publish() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void observe() { asm volatile("" ::: "memory"); }
 
+// The lane index as a value of this place: what is computed from it (addresses,
+// offsets) is computed here, not kept in registers from the kernel's entry on.
+__device__ __forceinline__ int lane_here()
+{
+  int l = __lane_id();
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
+// x of lane `lane ^ m`
+__device__ __forceinline__ float wave_xor(float x, int m, int lane)
+{
+  return __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ m) << 2, __float_as_int(x)));
+}
+__device__ __forceinline__ double wave_xor(double x, int m, int lane)
+{
+  const int at = (lane ^ m) << 2;
+  return __hiloint2double(__builtin_amdgcn_ds_bpermute(at, __double2hiint(x)),
+                          __builtin_amdgcn_ds_bpermute(at, __double2loint(x)));
+}
+
 __device__ inline unsigned wave_atomic_add(unsigned* p, unsigned x)
 {
   unsigned old = 0;
@@ -407,8 +428,35 @@ __device__ __forceinline__ unsigned dispatch_round()
 // (fixed order; every lane ends with its column's total).
 __device__ inline double group_sum(double x, int W)
 {
-  for (int m = W; m < WAVE; m <<= 1) x += __shfl_xor(x, m);
+  const int lane = lane_here();
+  for (int m = W; m < WAVE; m <<= 1) x += wave_xor(x, m, lane);
   return x;
+}
+
+// The kernel's arguments, read where they are used: taken as parameters, the
+// compiler loads all of them (about 120 scalar registers) at entry and keeps
+// them in lanes of vector registers, at an instruction per word and use (200
+// words; 40 now, and up to 17 vector registers fewer).  The empty asm makes
+// each call's loads its own.
+template <class Extra>
+struct KernelArgs {
+  const PopCtl& ctl;
+  const DevSet& set;
+  const Extra& ex;
+};
+template <class Extra>
+__device__ __forceinline__ KernelArgs<Extra> kernel_args()
+{
+  constexpr size_t set_at = (sizeof(PopCtl) + alignof(DevSet) - 1) / alignof(DevSet) * alignof(DevSet);
+  constexpr size_t ex_at =
+    (set_at + sizeof(DevSet) + alignof(Extra) - 1) / alignof(Extra) * alignof(Extra);
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto* p = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+#else
+  const char* p = nullptr;
+#endif
+  return {*(const PopCtl*)(p), *(const DevSet*)(p + set_at), *(const Extra*)(p + ex_at)};
 }
 
 // Pot must provide:
@@ -419,6 +467,9 @@ __device__ inline double group_sum(double x, int W)
 //                                                   a form that loads ahead
 //                                                   (used by the instantiations
 //                                                   without packed items)
+//   static constexpr int kWaves, kWavesPacked;      waves per SIMD that the
+//                                                   registers must allow (with
+//                                                   the packed code)
 //   static constexpr bool kForcePass;               three-body force assembly
 //   static double force_pass(set, ctl, ex, a0, a1, k, lane)
 //                                                   sum |F-F_ref|^2 over [a0, a1)
@@ -430,44 +481,46 @@ __device__ inline double group_sum(double x, int W)
 //                                                   the same for lane group g
 // PACK selects the instantiation that also serves packed items (chosen per
 // item); the other one never contains the packed code, so its register
-// budget is unaffected.  (Forcing the PACK one to the other's occupancy
-// makes it spill to scratch, and a launch that needs scratch memory costs
-// more than the wave it saves.)  LONE is the instantiation for launches of
+// budget is unaffected.  (Where its occupancy would need scratch memory it
+// gets a wave less: a launch that needs scratch costs more.)  LONE is the instantiation for launches of
 // at most one wave per SIMD, where a wave's time is the latency of its
 // dependent loads and registers are plentiful: with one lane block the
 // individuals' constants load while the fetch is in flight, and a chunk
 // loads each next atom's record during the current one and reads its rows
 // from the wave's LDS copy (Pot::chunk<true, true>; only with kHeaderAhead
 // and without PACK).
-// (at least two waves per SIMD: the widest instantiations would take registers
-// past the 256 that allows)
 template <class Pot, bool PACK = false, bool LONE = false>
-__global__ void __launch_bounds__(256, 2) population_kernel(PopCtl ctl, DevSet set,
-                                                         typename Pot::Extra ex)
+__global__ void __launch_bounds__(256, LONE ? 1 : PACK ? Pot::kWavesPacked : Pot::kWaves)
+  population_kernel(PopCtl, DevSet, typename Pot::Extra)
 {
-  const int lane = __lane_id();
+  using Extra = typename Pot::Extra;
   const unsigned total_waves = gridDim.x * (blockDim.x / WAVE);
   const unsigned wave_slot = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-  const int Nc = set.Nc;
   unsigned prev = 0xffffffffu;
-  const unsigned long long t_entry = ctl.trace ? wall_clock64() : 0ull;
+  const PopCtl& ctl0 = kernel_args<Extra>().ctl;
+  const unsigned long long t_entry = ctl0.trace ? wall_clock64() : 0ull;
   // home queue: one of the queues of this wave's XCD (workgroups of one XCD
   // spread over its queues)
-  const unsigned qpx = (unsigned)max(ctl.nq / kXcds, 1); // queues per XCD
-  int q = (int)((xcc_id() * qpx + (blockIdx.x / kXcds) % qpx) % (unsigned)ctl.nq);
+  const unsigned qpx = (unsigned)max(ctl0.nq / kXcds, 1); // queues per XCD
+  int q = (int)((xcc_id() * qpx + (blockIdx.x / kXcds) % qpx) % (unsigned)ctl0.nq);
   // a launch with a wave for every item: each queue has as many home waves
   // as items, so every first fetch finds one
   // (wave_slot is the same in every lane, but derived from threadIdx.x the
   // compiler cannot tell: taken through readfirstlane, the load is scalar
   // and q stays in an SGPR, as do the item and everything that follows)
   const int slot_u = wave_first((int)wave_slot);
-  if (slot_u < ctl.n_home) q = ldu(ctl.home, slot_u);
+  if (slot_u < ctl0.n_home) q = ldu(ctl0.home, slot_u);
   bool skip_fetch = false;
-  const bool early_lanes = LONE && ctl.K == 1;
+  const bool early_lanes = LONE && ctl0.K == 1;
   // values loaded per round trip by the reductions (more, in the lone-wave
   // form, made its launches slower: 48 values, 26.6 against 24.9 us)
   constexpr int FV = Pot::kFoldValues;
   for (;;) {
+    const KernelArgs<Extra> args = kernel_args<Extra>();
+    const PopCtl& ctl = args.ctl;
+    const DevSet& set = args.set;
+    const Extra& ex = args.ex;
+    const int lane = lane_here();
     // With one lane block, every item's individuals are known before the
     // fetch: their constants load while it is in flight.
     typename Pot::Lane lanes{};
@@ -543,6 +596,7 @@ __global__ void __launch_bounds__(256, 2) population_kernel(PopCtl ctl, DevSet s
           Pot::chunk(set, lanes, item, ctl, ex, acc);
         mark(5);
       }
+      const KernelArgs<Extra> after = kernel_args<Extra>();
       if (Pot::kForcePass && is_force) {
         publish(); // the per-bond forces of this chunk are complete
         if (nch > 1) {
@@ -555,15 +609,15 @@ __global__ void __launch_bounds__(256, 2) population_kernel(PopCtl ctl, DevSet s
         if (packed) {
           if constexpr (can_pack) {
             const int G = item.groups, W = WAVE / G;
-            acc.v[7] = group_sum(Pot::force_pass_packed(set, ctl, item.a0, item.a1, k,
+            acc.v[7] = group_sum(Pot::force_pass_packed(after.set, after.ctl, item.a0, item.a1, k,
                                                         lane & (W - 1), lane / W, G),
                                  W);
           }
         } else {
-          acc.v[7] = Pot::force_pass(set, ctl, ex, item.a0, item.a1, k, lane);
+          acc.v[7] = Pot::force_pass(after.set, after.ctl, after.ex, item.a0, item.a1, k, lane);
         }
       } else if (nch > 1) {
-        if (!fold_chunks<FV>(ctl, cnt, c, k, item.chunk, nch, lane, is_force, acc))
+        if (!fold_chunks<FV>(after.ctl, cnt, c, k, item.chunk, nch, lane, is_force, acc))
           continue;
         if (lane == 0) *cnt = 0u;
       }
@@ -584,9 +638,10 @@ __global__ void __launch_bounds__(256, 2) population_kernel(PopCtl ctl, DevSet s
         acc.v[7] = Pot::force_pass(set, ctl, ex, item.a0, item.a1, k, lane);
       }
       mark(5);
-      unsigned* cnt2 = &ctl.cnt2[(long)c * ctl.K + k];
+      const KernelArgs<Extra> after = kernel_args<Extra>();
+      unsigned* cnt2 = &after.ctl.cnt2[(long)c * after.ctl.K + k];
       if (nch > 1) {
-        if (!fold_chunks<FV>(ctl, cnt2, c, k, item.chunk, nch, lane, true, acc))
+        if (!fold_chunks<FV>(after.ctl, cnt2, c, k, item.chunk, nch, lane, true, acc))
           continue;
       }
       if (lane == 0) {
@@ -595,15 +650,16 @@ __global__ void __launch_bounds__(256, 2) population_kernel(PopCtl ctl, DevSet s
       }
     }
 
+    const KernelArgs<Extra> done = kernel_args<Extra>();
     double eE = 0.0, eW = 0.0, eF = 0.0;
     if (is_force) {
       eF = acc.v[7];
     } else {
-      const double dE = acc.v[0] - (double)ldu(set.pe_ref, c);
+      const double dE = acc.v[0] - (double)ldu(done.set.pe_ref, c);
       eE = dE * dE;
 #pragma unroll
       for (int u = 0; u < 6; ++u) {
-        const double dW = acc.v[1 + u] - (double)ldu(set.virial_ref, c + (long)Nc * u);
+        const double dW = acc.v[1 + u] - (double)ldu(done.set.virial_ref, c + (long)done.set.Nc * u);
         eW += dW * dW;
       }
     }
@@ -611,8 +667,8 @@ __global__ void __launch_bounds__(256, 2) population_kernel(PopCtl ctl, DevSet s
     // the launch has finished, so every queue is empty: this wave goes
     // straight to the exit (two memory round trips less at the end of the
     // launch's longest chain).
-    if (config_done<FV>(ctl, Nc, set.Nc_force, c, k, lane, eE, eW, eF) &&
-        ctl.K == 1)
+    if (config_done<FV>(done.ctl, done.set.Nc, done.set.Nc_force, c, k, lane, eE, eW, eF) &&
+        done.ctl.K == 1)
       skip_fetch = true;
   }
 }

@@ -224,6 +224,7 @@ void launch_tersoff_plain(const DevSet& s, const TersoffParams& q, float* b, flo
 template <bool TWO>
 struct TersoffPop {
   static constexpr int NMAX = 4;
+  static constexpr int kWaves = 4, kWavesPacked = TWO ? 3 : 4;
   static constexpr bool kForcePass = true;
   static constexpr int kFoldValues = 24;
   using Lane = TLane;
@@ -265,17 +266,18 @@ struct TersoffPop {
   // as they arrive).  Lanes 0-2 read the header words (count, longest bond,
   // bond types), lanes 3-5 one word in each later 128-byte line of the
   // record, which brings those lines into L2 for the row loads.
-  __device__ static int ahead_load(const DevSet& s, int i)
+  __device__ static unsigned ahead_offset(int lane)
   {
-    const char* base = reinterpret_cast<const char*>(s.rec + (long)i * RS);
-    const int lane = __lane_id();
-    const int off = lane == 1   ? 12
-                    : lane == 2 ? 4
-                    : lane == 3 ? min(128, RS * 16 - 4)
-                    : lane == 4 ? min(256, RS * 16 - 4)
-                    : lane == 5 ? RS * 16 - 4
-                                : 0;
-    return *reinterpret_cast<const int*>(base + off);
+    return lane == 1   ? 12
+           : lane == 2 ? 4
+           : lane == 3 ? min(128, RS * 16 - 4)
+           : lane == 4 ? min(256, RS * 16 - 4)
+           : lane == 5 ? RS * 16 - 4
+                       : 0;
+  }
+  __device__ static int ahead_load(const DevSet& s, int i, unsigned off)
+  {
+    return *reinterpret_cast<const int*>(reinterpret_cast<const char*>(s.rec + (long)i * RS) + off);
   }
   __device__ static Hdr header_of(int v)
   {
@@ -464,6 +466,152 @@ struct TersoffPop {
     }
   }
 
+  // An energy configuration's atom of four bonds, all of one kind and inside
+  // every lane's R1, from its moment record M (wave-uniform with U, in LDS
+  // with LR, else per lane).  An atom's energy and virial need the cosines
+  // only through sums that do not depend on the individual: with
+  // x = cos - h = c' - h',
+  //   zeta_u = beta sum_v x^2 = beta (sum c'^2 + h' (3 h' - sum 2 c'))
+  //   sum_uv A_u x r_u (x) dcos/dr_u, both ends of a pair together
+  //          = sum_u A_u (sum_v c' G_uv - h' sum_v G_uv)
+  // (products of two of the individual's constants are not rounded ahead: such
+  // an error is the same for every bond, and does not average out).  False,
+  // with nothing in `out`, where the first sum is a small difference (below 1/16
+  // of its first term), or zeta below the bond order's cut-off, or a NaN: such
+  // atoms take the general body.
+  //
+  // Bound by the VALU (200 instructions an atom, the general body 250) and, with
+  // the per-bond forces of the force configurations, memory.  120 200 atoms, a
+  // fifth of the configurations with forces, 200 individuals: the launch 284 ->
+  // 264 us, the error against 64 bits the same.
+  template <bool U, bool LR>
+  __device__ static bool moments(const TLane& q, const float* M, int unl, float (&out)[7])
+  {
+    const float hs = q.h - kMomCos;
+    float z[4], low = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float c2 = ldr<U, LR>(M, 8 + u);
+      z[u] = fmaf(hs, fmaf(3.0f, hs, -ldr<U, LR>(M, 4 + u)), c2);
+      const float l = fmaf(-1.0f / 16.0f, c2, z[u]);
+      low = u == 0 ? l : fminf(low, l);
+    }
+    if (__any(!(q.beta * low >= 1.0e-16f))) return false;
+    auto bonds = [&](const float (&c)[7]) {
+      float e = 0.0f, A[4], w[4], sum[kMomBond];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float x = ldr<U, LR>(M, u) - c[6];
+        const float lz = flog2(q.beta * z[u]);
+        const float l1 = flog2(1.0f + fexp2(q.en * lz));
+        const float fr = c[0] * fexp2(c[2] * x), fa = c[3] * fexp2(c[5] * x);
+        const float bfa = fexp2(q.mhon * l1) * fa;
+        A[u] = fexp2(fmaf(q.mhon1, l1, q.en1 * lz)) * fa; // -2 b' fA
+        w[u] = fmaf(-c[4], bfa, c[1] * fr);               // fR' - b fA'
+        const float rep = fr - bfa;
+        e = u == 0 ? rep : e + rep;
+      }
+      // sums over the bonds, four words of each at a time (per-lane records:
+      // loaded after the sums before, by the empty asm; the compiler would load
+      // the whole record at once, in 64 registers)
+#pragma unroll
+      for (int k = 0; k < kMomBond; k += 4) {
+        using v4 = __attribute__((ext_vector_type(4))) float;
+        auto* b = (const __attribute__((address_space(1))) v4*)(M + kMomBond + k);
+        v4 g4[4];
+        if constexpr (!U) {
+          asm volatile("" : "+v"(b) : "v"(k == 0 ? e : sum[k - 1]));
+#pragma unroll
+          for (int u = 0; u < 4; ++u) g4[u] = b[kMomBond / 4 * u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int j = k; j < k + 4; ++j) {
+            float g;
+            if constexpr (U) g = ldr<U, LR>(M, kMomBond * (1 + u) + j);
+            else g = g4[u][j - k];
+            const float f = j < 6 ? w[u] : A[u];
+            sum[j] = u == 0 ? f * g : fmaf(f, g, sum[j]);
+          }
+      }
+      const float *p = sum, *v1 = sum + 6, *v0 = sum + 11;
+      const float bh = -0.5f * q.beta;
+      float t[5];
+#pragma unroll
+      for (int j = 0; j < 5; ++j) t[j] = fmaf(-hs, v0[j], v1[j]);
+      out[0] = 0.5f * e;
+      out[1] = fmaf(bh, t[0], p[0]);
+      out[2] = fmaf(bh, t[1], p[1]);
+      out[3] = fmaf(-bh, t[0] + t[1], p[2]);
+      out[4] = fmaf(bh, t[2], p[3]);
+      out[5] = fmaf(bh, t[3], p[4]);
+      out[6] = fmaf(bh, t[4], p[5]);
+    };
+    float c[2][7];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      c[k][0] = q.cR[k];
+      c[k][1] = q.kR[k];
+      c[k][2] = q.kR2[k];
+      c[k][3] = q.cA[k];
+      c[k][4] = q.kA[k];
+      c[k][5] = q.kA2[k];
+      c[k][6] = q.r0[k];
+    }
+    if constexpr (!TWO) {
+      bonds(c[0]);
+    } else if constexpr (U) {
+      if (unl) bonds(c[1]);
+      else bonds(c[0]);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 7; ++m) c[0][m] = unl ? c[1][m] : c[0][m];
+      bonds(c[0]);
+    }
+    return true;
+  }
+
+  // The atoms [a0, a1) of an energy configuration, moment records first.  The
+  // next atom's moment record is touched by one vector load during this atom
+  // (see ahead_load): the words that the branch needs (lanes 0, 1) and one in
+  // each of its other lines; after an atom that its moment record did not
+  // serve, the next atom's general record too.
+  __device__ static void energy_chunk(const DevSet& s, const TLane& q, int a0, int a1, int lane,
+                                      unsigned r, Acc& acc)
+  {
+    const unsigned off = 4u * (lane == 0 ? 12u : lane == 1 ? 13u : lane == 2 ? 44u : 76u);
+    const unsigned goff = ahead_offset(lane);
+    const bool use = s.mom != nullptr;
+    auto record = [&](int i) {
+      return reinterpret_cast<const char*>(s.mom) + (long)(i - s.N_force) * (kMomWords * 4);
+    };
+    int hv = 0, gv = 0;
+    bool fast = use, have = false;
+    if (use) hv = *reinterpret_cast<const int*>(record(a0) + off);
+    for (int i = a0; i < a1; ++i) {
+      rotate_priority(r + (unsigned)i);
+      const float dmax = __int_as_float(__builtin_amdgcn_readlane(hv, 0));
+      const int munl = TWO ? __builtin_amdgcn_readlane(hv, 1) : 0;
+      const int j = min(i + 1, a1 - 1);
+      if (use) hv = *reinterpret_cast<const int*>(record(j) + off);
+      const bool had = have;
+      const Hdr h = header_of(gv);
+      have = !fast;
+      if (have) gv = ahead_load(s, j, goff);
+      float w[7];
+      fast = use && dmax < q.r1min &&
+             moments<true, false>(q, reinterpret_cast<const float*>(record(i)), munl, w);
+      if (fast) {
+#pragma unroll
+        for (int u = 0; u < 7; ++u) acc.v[u] += (double)w[u];
+      } else {
+        if (had) atom_h<false, true>(s, q, i, h, s.rec + (long)i * RS, nullptr, lane, acc);
+        else atom<false, true>(s, q, i, nullptr, lane, acc);
+      }
+    }
+  }
+
   // Lone-wave form: a record spread over the wave, word l in lane l and
   // word 64 + l in lane l (two vector loads).
   static constexpr int RW = RS * 4; // words per record
@@ -471,16 +619,14 @@ struct TersoffPop {
   struct Spread {
     int lo, hi;
   };
-  __device__ static Spread spread_load(const DevSet& s, int i)
+  __device__ static Spread spread_load(const DevSet& s, int i, int l)
   {
     const int* w = reinterpret_cast<const int*>(s.rec + (long)i * RS);
-    const int l = __lane_id();
     return Spread{w[l], w[min(WAVE + l, RW - 1)]};
   }
-  __device__ static void spread_store(float4* buf, const Spread& v)
+  __device__ static void spread_store(float4* buf, const Spread& v, int l)
   {
     int* w = reinterpret_cast<int*>(buf);
-    const int l = __lane_id();
     w[l] = v.lo;
     if (WAVE + l < RW) w[WAVE + l] = v.hi;
   }
@@ -488,6 +634,19 @@ struct TersoffPop {
   {
     return Hdr{__builtin_amdgcn_readlane(v.lo, 0), TWO ? __builtin_amdgcn_readlane(v.lo, 1) : 0,
                __int_as_float(__builtin_amdgcn_readlane(v.lo, 3))};
+  }
+
+  // the same of an atom's moment record
+  static_assert(kMomWords >= WAVE && kMomWords <= 2 * WAVE, "moment records of the lone-wave form");
+  __device__ static Spread mom_load(const DevSet& s, int i, int l)
+  {
+    const int* w = reinterpret_cast<const int*>(s.mom + (long)(i - s.N_force) * kMomWords);
+    return Spread{w[l], w[min(WAVE + l, kMomWords - 1)]};
+  }
+  __device__ static void mom_store(float* buf, const Spread& v, int l)
+  {
+    buf[l] = __int_as_float(v.lo);
+    if (WAVE + l < kMomWords) buf[WAVE + l] = __int_as_float(v.hi);
   }
 
   // HDR: load the next atom's header during the current atom (the kernel
@@ -502,29 +661,63 @@ struct TersoffPop {
   __device__ static void chunk(const DevSet& s, const TLane& q, const WorkItem& it,
                                const PopCtl& ctl, int, Acc& acc)
   {
-    const int lane = __lane_id();
+    const int lane = lane_here();
     const unsigned r = dispatch_round();
     if constexpr (LONE) {
       // two records per wave of a 256-thread workgroup (the kernel's bound)
       __shared__ float4 buf[256 / WAVE][2][RS];
+      __shared__ alignas(16) float mbuf[256 / WAVE][2][kMomWords];
       const int w = wave_first((int)(threadIdx.x / WAVE));
-      Spread cur = spread_load(s, it.a0);
-      spread_store(buf[w][0], cur);
-      auto run = [&](auto force) {
-        constexpr bool F = decltype(force)::value;
-        float* fblk = F ? ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE : nullptr;
+      if (it.c < s.Nc_force) {
+        Spread cur = spread_load(s, it.a0, lane);
+        spread_store(buf[w][0], cur, lane);
+        float* fblk = ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE;
         for (int i = it.a0; i < it.a1; ++i) {
           rotate_priority(r + (unsigned)i);
           const int b = (i - it.a0) & 1;
           const Hdr h = spread_header(cur);
-          const Spread nxt = spread_load(s, min(i + 1, it.a1 - 1));
-          atom_h<F, true, true>(s, q, i, h, buf[w][b], fblk, lane, acc);
-          spread_store(buf[w][b ^ 1], nxt);
+          const Spread nxt = spread_load(s, min(i + 1, it.a1 - 1), lane);
+          atom_h<true, true, true>(s, q, i, h, buf[w][b], fblk, lane, acc);
+          spread_store(buf[w][b ^ 1], nxt, lane);
           cur = nxt;
         }
-      };
-      if (it.c < s.Nc_force) run(std::true_type{});
-      else run(std::false_type{});
+      } else {
+        // (after an atom that its moment record does not serve, the next
+        // atom's general record is loaded too)
+        const bool use = s.mom != nullptr;
+        Spread cur{}, nxt{}, gen{};
+        bool fast = use, have = !use;
+        if (use) {
+          cur = mom_load(s, it.a0, lane);
+          mom_store(mbuf[w][0], cur, lane);
+        } else {
+          gen = spread_load(s, it.a0, lane);
+          spread_store(buf[w][0], gen, lane);
+        }
+        for (int i = it.a0; i < it.a1; ++i) {
+          rotate_priority(r + (unsigned)i);
+          const int b = (i - it.a0) & 1, j = min(i + 1, it.a1 - 1);
+          const float dmax = __int_as_float(__builtin_amdgcn_readlane(cur.lo, 12));
+          const int munl = TWO ? __builtin_amdgcn_readlane(cur.lo, 13) : 0;
+          const Hdr h = spread_header(gen);
+          const bool had = have;
+          if (use) nxt = mom_load(s, j, lane);
+          have = !fast;
+          if (have) gen = spread_load(s, j, lane);
+          float o[7];
+          fast = use && dmax < q.r1min && moments<true, true>(q, mbuf[w][b], munl, o);
+          if (fast) {
+#pragma unroll
+            for (int u = 0; u < 7; ++u) acc.v[u] += (double)o[u];
+          } else {
+            if (had) atom_h<false, true, true>(s, q, i, h, buf[w][b], nullptr, lane, acc);
+            else atom<false, true>(s, q, i, nullptr, lane, acc);
+          }
+          if (use) mom_store(mbuf[w][b ^ 1], nxt, lane);
+          if (have) spread_store(buf[w][b ^ 1], gen, lane);
+          cur = nxt;
+        }
+      }
     } else if constexpr (!HDR) {
       if (it.c < s.Nc_force) {
         float* fblk = ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE;
@@ -533,30 +726,23 @@ struct TersoffPop {
           atom<true, true>(s, q, i, fblk, lane, acc);
         }
       } else {
-        for (int i = it.a0; i < it.a1; ++i) {
-          rotate_priority(r + (unsigned)i);
-          atom<false, true>(s, q, i, nullptr, lane, acc);
-        }
+        energy_chunk(s, q, it.a0, it.a1, lane, r, acc);
       }
     } else {
       // the next atom's header is loaded during this atom, so its row loads
       // issue at once (one memory latency per atom, not two)
-      int hv = ahead_load(s, it.a0);
       if (it.c < s.Nc_force) {
+        const unsigned off = ahead_offset(lane);
+        int hv = ahead_load(s, it.a0, off);
         float* fblk = ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE;
         for (int i = it.a0; i < it.a1; ++i) {
           rotate_priority(r + (unsigned)i);
           const Hdr h = header_of(hv);
-          hv = ahead_load(s, min(i + 1, it.a1 - 1));
+          hv = ahead_load(s, min(i + 1, it.a1 - 1), off);
           atom_h<true, true>(s, q, i, h, s.rec + (long)i * RS, fblk, lane, acc);
         }
       } else {
-        for (int i = it.a0; i < it.a1; ++i) {
-          rotate_priority(r + (unsigned)i);
-          const Hdr h = header_of(hv);
-          hv = ahead_load(s, min(i + 1, it.a1 - 1));
-          atom_h<false, true>(s, q, i, h, s.rec + (long)i * RS, nullptr, lane, acc);
-        }
+        energy_chunk(s, q, it.a0, it.a1, lane, r, acc);
       }
     }
   }
@@ -571,7 +757,37 @@ struct TersoffPop {
       float* fblk = ctl.bondf + (size_t)it.k * ctl.B_force * 3 * WAVE;
       for (int i = it.a0 + g; i < it.a1; i += G) atom<true, false>(s, q, i, fblk, col, acc);
     } else {
-      for (int i = it.a0 + g; i < it.a1; i += G) atom<false, false>(s, q, i, nullptr, col, acc);
+      // Moment records first, then the atoms (steps of the wave, kept as bits of
+      // `left` in lane n % 64) that they do not serve: both bodies in one loop
+      // took 170 registers.  A step of eight atoms: 11.3 -> 6.0 us.
+      const int steps = (it.a1 - it.a0 + G - 1) / G;
+      const int kept = s.mom ? min(steps, 32 * WAVE) : 0;
+      const int lane = lane_here();
+      unsigned left = 0;
+      bool some = steps > kept;
+      for (int n = 0; n < kept; ++n) {
+        const int i = it.a0 + g + n * G;
+        bool ok = true;
+        float w[7] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        if (i < it.a1) {
+          const float* M = s.mom + (long)(i - s.N_force) * kMomWords;
+          ok = !__any(!(M[12] < q.r1min)) &&
+               moments<false, false>(q, M, TWO ? __float_as_int(M[13]) : 0, w);
+        }
+#pragma unroll
+        for (int u = 0; u < 7; ++u) acc.v[u] += (double)w[u];
+        if (__any(!ok)) {
+          some = true;
+          if (lane == n % WAVE) left |= 1u << (n / WAVE);
+        }
+      }
+      if (some)
+        for (int n = 0; n < steps; ++n) {
+          const unsigned w = (unsigned)__builtin_amdgcn_readlane((int)left, n % WAVE);
+          if (n < kept && !(w >> (n / WAVE) & 1u)) continue;
+          const int i = it.a0 + g + n * G;
+          if (i < it.a1) atom<false, false>(s, q, i, nullptr, col, acc);
+        }
     }
   }
 
@@ -658,6 +874,7 @@ struct TersoffPop {
 // LDS rows, lane-contiguous, one region per wave.
 template <bool TWO>
 struct TersoffLoop {
+  static constexpr int kWaves = 4, kWavesPacked = 4;
   static constexpr bool kForcePass = true;
   static constexpr int kFoldValues = 24;
   static constexpr bool kPacked = false;

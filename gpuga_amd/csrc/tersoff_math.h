@@ -138,8 +138,9 @@ __device__ inline TLane tersoff_make(const PopCtl& ctl, int p)
   // the wave's smallest R1: an atom whose bonds are all shorter has fc = 1,
   // fc' = 0 on every lane
   float m = q.r1;
+  const int lane = lane_here();
 #pragma unroll
-  for (int o = WAVE / 2; o >= 1; o >>= 1) m = fminf(m, __shfl_xor(m, o));
+  for (int o = WAVE / 2; o >= 1; o >>= 1) m = fminf(m, wave_xor(m, o, lane));
   q.r1min = m;
   return q;
 }

@@ -128,6 +128,10 @@ void build_geometry_device(const TrainSet& ts, const DeviceNeighbors& d, float4*
                            float4* tri, hipStream_t st);
 void build_records_device(int N, int M, const DeviceNeighbors& d, const int* ptype,
                           const float4* bond, const float4* tri, float4* rec, hipStream_t st);
+// Moment records (device.h) of the atoms [i0, N), lists of at most four
+// neighbours; returns how many of them serve an individual with this R1.
+int build_moments_device(int i0, int N, const DeviceNeighbors& d, const int* ptype,
+                         const float4* bond, float r1, float* mom, hipStream_t st);
 
 // Index of the configuration that holds atom i.
 int config_of(const TrainSet& ts, int i);
