@@ -144,18 +144,6 @@ size_t DeviceSet::bytes() const
          ri_cconst.bytes() + ri_fconst.bytes();
 }
 
-void PopPlan::drop_ga_graphs()
-{
-  for (int k = 0; k < 2; ++k) {
-    if (ga_exec[k]) (void)hipGraphExecDestroy(ga_exec[k]);
-    if (ga_graph[k]) (void)hipGraphDestroy(ga_graph[k]);
-    ga_exec[k] = nullptr;
-    ga_graph[k] = nullptr;
-  }
-}
-
-PopPlan::~PopPlan() { drop_ga_graphs(); }
-
 // ------------------------------------------------------------ set-up
 
 Fitness::Fitness(const std::string& dir, const FitnessOptions& opt) : opt_(opt)
@@ -1352,51 +1340,9 @@ void Fitness::compute_async(int P, const float* genes, int share)
   pending_P_ = P;
 }
 
-namespace {
-
-// The launches of `body` on st as a graph, instantiated.  A failure inside
-// ends the capture first, so the stream is usable again.
-template <class F>
-void captured(hipStream_t st, F&& body, hipGraph_t* graph, hipGraphExec_t* exec)
-{
-  GPUGA_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  try {
-    body();
-  } catch (...) {
-    hipGraph_t g = nullptr;
-    (void)hipStreamEndCapture(st, &g);
-    if (g) (void)hipGraphDestroy(g);
-    throw;
-  }
-  GPUGA_HIP(hipStreamEndCapture(st, graph));
-  GPUGA_HIP(hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0));
-  // the graph's upload to the device, now: left to its first launch, it
-  // held that launch back by up to 2 ms with the device idle (an 8-
-  // generation graph of the 384-individual Tersoff workload)
-  GPUGA_HIP(hipGraphUpload(*exec, st));
-}
-
-} // namespace
-
 void Fitness::prepare(int P)
 {
   if (opt_.backend != 1) plan(P);
-}
-
-void Fitness::capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph,
-                                  hipGraphExec_t* exec)
-{
-  hipStream_t st = stream_;
-  captured(st, [&] {
-    for (int i = 0; i < n; ++i) {
-      const int b = (k + i) & 1;
-      PopCtl ctl = pl.ctl;
-      ctl.genes = pl.dga->genes(b);
-      if (pl.ga_quad) launch_quad(pl, ctl, st);
-      else launch_population(pl, ctl, st);
-      pl.dga->step(b, pl.ctl.fitness, st);
-    }
-  }, graph, exec);
 }
 
 void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best, float* elite)
@@ -1416,31 +1362,21 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
   // (crossover and mutation keep genes in [0, 1]: one look at the start)
   const bool quad = quad_for(P, ga.population().data());
   if (!quad) ensure_items(pl);
-  if (pl.ga_quad != quad) pl.drop_ga_graphs();
-  pl.ga_quad = quad;
   // the GA as it was before this call: staging draws advances its random
   // stream, so a failed run restores it
   const GA before = ga;
-  if (!pl.dga || !pl.dga->matches(ga)) {
-    pl.drop_ga_graphs();
+  if (!pl.dga || !pl.dga->matches(ga))
     pl.dga = std::make_unique<DeviceGA>(ga, pl.genes.get(), 1024, st, opt_.ga_batch);
-  }
   DeviceGA& dga = *pl.dga;
   dga.upload(ga, first_generation, st);
   // batches double from one generation up to the staging capacity, so the
   // device starts after one generation's draws and the host then draws each
   // batch while the device runs the one before
   const int B = dga.batch();
-  // Generations are launched directly, whole batches of a long run as graphs.
-  // A graph of few generations takes 14 us longer to launch than its kernels
-  // (ten generations of 50 individuals: 391 us in graphs of 1, 2, 4 and 2 + 1,
-  // 357 us launched directly), and capturing it costs the first call 1-3 ms;
-  // whole batches run equally fast either way and leave the host free to draw.
-  // Captured before the first launch: later, the device would wait idle.
-  const bool graphs = opt_.use_graph && B >= 8 && generations >= 3 * B;
-  if (graphs)
-    for (int k = 0; k < 2; ++k)
-      if (!pl.ga_exec[k]) capture_generations(pl, k, B, &pl.ga_graph[k], &pl.ga_exec[k]);
+  // (launched directly: replayed from a graph, ten generations of 50
+  // individuals took 391 us against 357, four hundred the same per generation
+  // on sets of 3 840 and 120 200 atoms, 31.5 and 280 us, and the capture cost a
+  // process's first long run up to 4 ms)
   const int H = dga.history_cap();
   std::vector<float> h((size_t)H * (1 + V));
   int g = 0; // generations queued
@@ -1452,10 +1388,6 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
       nb = std::min({ramp, B, n - b});
       dga.stage(ga, first_generation + g + b, nb, st);
       const int k0 = (g + b) & 1;
-      if (graphs && nb == B) {
-        GPUGA_HIP(hipGraphLaunch(pl.ga_exec[k0], st));
-        continue;
-      }
       for (int i = 0; i < nb; ++i) {
         const int k = k0 ^ (i & 1);
         PopCtl ctl = pl.ctl;
@@ -1478,7 +1410,6 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
       // the device GA, and the GA handle returns to its state before this call
       ga = before;
       pl.dga.reset();
-      pl.drop_ga_graphs();
       discard_launch(pl);
     }
     dga.history(h.data(), n, st);
@@ -1510,12 +1441,7 @@ void Fitness::discard_launch(PopPlan& pl)
 void Fitness::set_spin_limit(int spins)
 {
   spin_limit_ = spins;
-  for (auto& kv : plans_) {
-    PopPlan& pl = *kv.second;
-    pl.ctl.spin_limit = spins;
-    // the captured launches hold the old control block
-    pl.drop_ga_graphs();
-  }
+  for (auto& kv : plans_) kv.second->ctl.spin_limit = spins;
 }
 
 void Fitness::compute_wait(float* fitness, double* terms)

@@ -19,13 +19,13 @@ namespace gpuga {
 struct FitnessOptions {
   int backend = 0;        // 0: population kernel, 1: per-individual launches
   int chunk_cost = 0;     // work-item cost target; 0 = autotune on first use
-  int use_graph = 1;      // run_ga: replay whole batches of generations from HIP graphs
+  int use_graph = 1;      // accepted, and without effect: every launch is direct
   int nn2b_bf16 = 1;      // NN2B hidden layer 2 on BF16 MFMA (else FP32)
   int nn2b_grid = 1024;   // NN2B tabulation points
   int verbose = 0;
   int blocks_per_cu = 0;  // 0 = from the occupancy calculator
   int pack_lanes = 1;     // pack a last lane block of <= 16 individuals
-  int queues = 0;         // work queues of the population launch; 0 = one per XCD
+  int queues = 0;         // work queues of the population launch; 0 = four per XCD
   int ga_batch = 0;       // generations per staged batch of the device GA; 0 = up to 32
   int tail_split = 0;     // configurations smaller than one work item are cut into
                           // pieces of 1/tail_split of an item (0, 1: not cut)
@@ -49,7 +49,7 @@ struct DeviceSet {
   DeviceBuffer<int> Na, Na_sum, type, nn, bond0, nl, rev, ptype, tri0;
   DeviceBuffer<float4> bond, tri, ri_tab, rec, shell_rec, pair_tab;
   // the Tersoff population kernel's pruned list and its tables, kept when
-  // the looped kernel reads them (more than 16 neighbours within R2)
+  // the looped kernel reads them (more than 20 neighbours within R2)
   DeviceBuffer<int> p_nn, p_b0, p_nl, p_rev, p_ptype, p_tri0;
   DeviceBuffer<float4> p_bond, p_tri;
   DeviceBuffer<int4> pair_hdr;
@@ -100,7 +100,6 @@ struct PopPlan {
   DeviceBuffer<unsigned> qdone;
   QuadEval qeval{};
   NodeTable qnodes{};
-  bool ga_quad = false; // the GA graphs run the quadratic forms
   int P = 0, K = 0, n_items = 0, grid = 0, block = 256, chunk_cost = 0;
   int occ = 0;         // resident workgroups per CU the grid is sized for
   int groups_last = 1; // lane groups of the last lane block's items
@@ -116,15 +115,9 @@ struct PopPlan {
   PinnedBuffer<float> h_genes;
   PinnedBuffer<double> h_out;
   PopCtl ctl{};
-  // device GA of this population size; a whole staged batch of generations
-  // (population launch + GA step each) as a graph: ga_exec[k] starts on
-  // population buffer k (a generation on buffer b writes the next into buffer
-  // 1 - b)
+  // device GA of this population size (a generation on population buffer b
+  // writes the next into buffer 1 - b)
   std::unique_ptr<DeviceGA> dga;
-  hipGraph_t ga_graph[2] = {};
-  hipGraphExec_t ga_exec[2] = {};
-  void drop_ga_graphs();
-  ~PopPlan();
 };
 
 class Fitness {
@@ -230,8 +223,6 @@ private:
   // the same by the quadratic forms (their values, then their evaluation)
   void launch_quad(PopPlan& pl, const PopCtl& ctl, hipStream_t st);
   void launch_quad_values(PopPlan& pl, const PopCtl& ctl, int first, int count, hipStream_t st);
-  // n generations of the device GA from population buffer k, captured
-  void capture_generations(PopPlan& pl, int k, int n, hipGraph_t* graph, hipGraphExec_t* exec);
   double time_plan(int P, const LaunchShape& sh, int reps, int* occ = nullptr);
   // after a launch whose status word is set: clear the plan's counters and
   // results, then fail

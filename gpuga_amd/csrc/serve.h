@@ -10,7 +10,7 @@
 // runs on 1/n of its grid for n running jobs (up to 4).  By default every
 // launch takes the whole GPU: launches from up to four streams overlap at
 // their edges, and that measured faster than splitting.  Reading a job's files
-// and setting it up (training set on the device, work plan, graph) run on
+// and setting it up (training set on the device, work plan) run on
 // worker threads, so admissions never hold up the generations of running
 // jobs.  The work-item size of each job is a deterministic function of its
 // training set, so a job's results are the same whether it runs alone or
@@ -42,7 +42,7 @@ public:
   int finished() const;
   void job_info(int id, int* state, int* gens, float* best, float* elite) const;
   const std::vector<double>& latencies() const { return lat_ms_; }
-  // per admitted job: submission to ready (parse, set-up, plan, graph), ms
+  // per admitted job: submission to ready (parse, set-up, plan), ms
   const std::vector<double>& admissions() const { return adm_ms_; }
 
 private:

@@ -649,13 +649,13 @@ struct TersoffPop {
     if (WAVE + l < kMomWords) buf[WAVE + l] = __int_as_float(v.hi);
   }
 
-  // HDR: load the next atom's header during the current atom (the kernel
-  // instantiation without the packed path, whose register budget has room for
-  // it).  LONE (launches of at most one wave
-  // per SIMD, where a wave's time is the latency of its loads): the next
-  // atom's whole record is loaded during the current atom, spread over the
-  // wave, and written to the wave's LDS buffer at its end; the rows are read
-  // from there (an LDS round trip per atom instead of a memory one).
+  // HDR: load the next atom's header during the current atom of a force
+  // configuration (the kernel instantiation without the packed path, whose
+  // register budget has room for it).  LONE (launches of at most one wave per
+  // SIMD, where a wave's time is the latency of its loads): the next atom's
+  // whole record is loaded during the current atom, spread over the wave, and
+  // written to the wave's LDS buffer at its end; the rows are read from there
+  // (an LDS round trip per atom instead of a memory one).
   static constexpr bool kHeaderAhead = true;
   template <bool HDR = false, bool LONE = false>
   __device__ static void chunk(const DevSet& s, const TLane& q, const WorkItem& it,

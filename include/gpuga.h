@@ -26,9 +26,8 @@ typedef struct gpuga_options {
   int chunk_cost; /* work-item size of the population launch; 0 = autotune
                      the launch shape (this and the fields below left at 0
                      or, for pack_lanes, at 1) */
-  int use_graph;  /* 1: gpuga_fitness_run_ga replays whole batches of a long
-                     run's generations from HIP graphs; 0: it launches every
-                     generation by itself */
+  int use_graph;  /* accepted, and without effect: every launch is direct (a
+                     replay from a HIP graph is no faster) */
   int nn2b_bf16;  /* 1: NN2B hidden layer on BF16 MFMA; 0: FP32 */
   int nn2b_grid;  /* NN2B tabulation points (default 1024) */
   int verbose;
@@ -159,8 +158,10 @@ int gpuga_inspect_geometry(const char* input_dir, int* sizes3, float* bond, floa
 
 /* Launch shape chosen by timing candidates for population P (work-item
  * size, then the queue count, resident workgroups per CU and lane packing
- * that the options leave at 0 / on); returns the work-item size.  No
- * counterpart in the reference (its launch shape is fixed). */
+ * that the options leave at 0 / on); returns the work-item size.  (A pair
+ * potential's quadratic forms have no shape to choose: the built-in size, for
+ * the calls that take the population kernel.)  No counterpart in the
+ * reference (its launch shape is fixed). */
 int gpuga_fitness_autotune(gpuga_fitness* h, int P, int* chunk_cost);
 /* The shape the population launch for P runs with (tuned first when the
  * options ask for it): work-item cost, queues, resident workgroups per CU
@@ -257,7 +258,7 @@ int gpuga_server_job(const gpuga_server* s, int job_id, int* state, int* generat
                      float* best_fitness, float* elite);
 /* Per-generation latencies (ms) of all jobs in completion order; n in/out. */
 int gpuga_server_latencies(const gpuga_server* s, double* ms, int* n);
-/* Per admitted job, submission to ready (parsing, set-up, work plan, graph;
+/* Per admitted job, submission to ready (parsing, set-up, work plan;
  * queueing behind the memory budget included), ms, in admission order. */
 int gpuga_server_admissions(const gpuga_server* s, double* ms, int* n);
 
