@@ -6,7 +6,7 @@ displacements, 20% force configurations, labels from the ground-truth
 parameter set (computed by this library's find_force), cutoff 3.0 A.
 
 A step is one GA generation: the fitness of all 200 individuals over all
-configurations (one persistent, graph-replayed HIP launch) followed by the
+configurations (one persistent HIP launch) followed by the
 GA's sort / crossover / mutation, by default on the device as well, so the
 timed generations run back to back with the population resident (--host-ga:
 genes and fitness cross to the host GA every generation).  The metric is
@@ -36,7 +36,9 @@ MI355X_HBM_PEAK = 8.0e12     # B/s
 # Algorithmic work per individual x atom evaluation (4 neighbours per atom):
 # pair terms ~106 FLOP x 4, triplets ~57 FLOP x 12, assembly -> ~1.1 kFLOP.
 TERSOFF_FLOP_PER_UNIT = 1.1e3
-# Pair potentials: the work per pair the population kernels evaluate (each
+# Pair potentials: the work per pair of the formulas (the quadratic forms that
+# evaluate a population do not execute it per pair, so the fraction of peak is
+# a measure of time against this work and can exceed 1; each
 # unordered pair once in energy/virial configurations, every ordered pair in
 # force configurations; distance-only factors such as erfc(a r)/r come from
 # the set-up tables).  FMA = 2 FLOP; exp2 not counted.
@@ -399,8 +401,7 @@ def main():
         elapsed = time.perf_counter() - t0
         best = float(bests[-1])
         # the population launch alone, for the roofline (one untimed call
-        # first: it captures the launch's graph, which the events would
-        # otherwise count as idle device time)
+        # first)
         genes = ga.population
         fit.compute(genes)
         fit.set_timing(True)
@@ -437,14 +438,15 @@ def main():
             flop = P * (RI_FLOP_FORCE_PAIR * fp.sum() + RI_FLOP_ENERGY_PAIR * ep.sum() +
                         morse * (fp[1] + ep[1]))
             note = (f"{int(fp.sum())} ordered force-configuration pairs, {int(ep.sum())} "
-                    "unordered energy-configuration pairs per individual")
+                    "unordered energy-configuration pairs per individual: the formula's work, "
+                    "which the quadratic forms do not execute")
         else:
             n = fit.num_neurons
             flop = P * (NN2B_FLOP_FORCE_PAIR * fp.sum() + NN2B_FLOP_ENERGY_PAIR * ep.sum() +
                         NN2B_GRID * (6.0 * n * n + 23.0 * n))
             note = (f"{int(fp.sum())} ordered force-configuration pairs, {int(ep.sum())} "
                     f"unordered energy-configuration pairs and a {NN2B_GRID}-point tabulation "
-                    "per individual; time = tabulation + pair kernel")
+                    "per individual: the formula's work, which the quadratic forms do not execute")
     if args.plain:
         flop /= P  # timing covers one individual per launch group
     achieved = flop / kernel_s
