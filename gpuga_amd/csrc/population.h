@@ -406,7 +406,9 @@ __device__ inline int next_item(const PopCtl& ctl, int& q)
 // its large items end the launch.  Kernels call this once per atom with a
 // running count: the wave priority then cycles through its four levels, at
 // a phase set by the workgroup's dispatch round, so the waves of a SIMD take
-// turns at the top.
+// turns at the top (120 200 atoms, 200 individuals: the launch 284 us without,
+// 267 us so; 274 us with two levels, 268 us changing every second atom, 271 us
+// with the level by the atoms left).
 __device__ __forceinline__ void rotate_priority(unsigned step)
 {
   switch (step & 3u) {
