@@ -357,6 +357,11 @@ DeviceGA::DeviceGA(const GA& ga, float* genes0, int history_cap, hipStream_t st,
   d_.history_gen0 = hist_gen0_.get();
   max_gen_ = p.maximum_generation;
   rate_ = p.mutation_rate;
+  // (results of any run that fits one block: grown run by run, a longer run
+  // than the ones before took half a millisecond more)
+  const size_t fixed = 1 + (size_t)P + (size_t)P * V;
+  if (fixed <= kBlockWords)
+    out_.resize(std::min(kBlockWords, fixed + (size_t)d_.history_cap * (1 + V)));
   GPUGA_HIP(hipStreamSynchronize(st));
 }
 
