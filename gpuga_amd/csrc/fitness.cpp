@@ -621,12 +621,13 @@ int Fitness::quad_elements() const
     for (float x : *v)
       if (!std::isfinite(x)) return 0;
   if (spec_.nn2b()) {
-    // half as many nodes as the grid has points, in elements of 32: more
-    // accurate than the cubic interpolation on the whole grid from 256
-    // points on (fewer than 4 elements resolve a network worse than the
-    // grid's three values per point); the forms grow with the square of the
-    // nodes, so a grid finer than 2048 points (all codes together) stays with
-    // the pair loop
+    // half as many nodes as the grid has points, in elements of 32.  How sharp
+    // an individual's curve is, is judged from its nodes at each evaluation
+    // (SharpSet): from 256 points on they resolve part of a population drawn
+    // from bounds of 3 (n = 20 on 256 points a quarter of it, n = 32 on 1024 all
+    // but a few), and the pair loop takes the rest.  The forms grow with the
+    // square of the nodes, so a grid finer than 2048 points (all codes together)
+    // stays with the pair loop
     const int G = std::max(opt_.nn2b_grid, 16), codes = spec_.pair_codes();
     if (G < 256 || G > 2048) return 0;
     return codes * G > 4096 ? 0 : G / (2 * QB);
@@ -666,8 +667,9 @@ void Fitness::setup_quad()
   b.len = std::max((double)dmax_ - (double)dmin_, 1e-3) / E;
   const int CE = b.CE();
   // the elements that the pairs of energy and of force configurations use
+  if (CE > QCE) fail("internal: elements of the quadratic forms");
   DeviceBuffer<int> d_used;
-  std::vector<int> used((size_t)4 * CE, 0);
+  std::vector<int> used((size_t)6 * CE, 0);
   d_used.upload(used, st);
   launch_quad_used(ds_.view, b, d_used.get(), st);
   d_used.download(used.data(), used.size(), st);
@@ -713,6 +715,18 @@ void Fitness::setup_quad()
   quad_.basis = b;
   quad_.n_act = (int)act.size();
   quad_.act.upload(act, st);
+  std::vector<float2> pairs(CE);
+  std::vector<float> tail((size_t)QTAIL * QB);
+  if (!b.rigid) {
+    for (int ce = 0; ce < CE; ++ce)
+      pairs[ce] = make_float2((float)used[4 * CE + ce], (float)used[5 * CE + ce]);
+    for (int k = 0; k < QTAIL; ++k)
+      for (int m = 0; m < QB; ++m)
+        tail[(size_t)k * QB + m] =
+          (float)(2.0 / QB * std::cos(M_PI / QB * (m + 0.5) * (QB - QTAIL + k)));
+    quad_.pairs.upload(pairs, st);
+    quad_.tail.upload(tail, st);
+  }
   // Rows in chunks of configurations and force atoms, the Gram products
   // accumulated over the chunks.  Chunks and the split of a chunk's rows over
   // waves do not depend on the columns, so a column's sums do not depend on
@@ -768,24 +782,24 @@ void Fitness::setup_quad()
 bool Fitness::quad_for(int P, const float* genes) const
 {
   if (!quad_.on) return false;
-  if (spec_.nn2b()) return true; // (the distances alone set its elements)
+  if (spec_.nn2b()) return true; // (each individual's nodes are checked)
   for (size_t k = 0; k < (size_t)P * spec_.V; ++k)
     if (!(genes[k] >= 0.0f && genes[k] <= 1.0f)) return false;
   return true;
 }
 
-void Fitness::build_quad_plan(PopPlan& pl, int P)
+// What a plan has on every path: genes, and results in one block on either
+// side (terms [P][3] in FP64, fitness [P] in FP32, the status word).
+void Fitness::build_results(PopPlan& pl, int P)
 {
-  hipStream_t st = stream_;
   pl.P = P;
   pl.K = (P + WAVE - 1) / WAVE;
-  const size_t out_doubles = 3 * (size_t)P + ((size_t)P + 1 + 1) / 2;
-  pl.out.resize(out_doubles);
-  pl.out.zero(st);
+  pl.out.resize(pl.out_doubles());
+  pl.out.zero(stream_);
   pl.genes.resize((size_t)P * spec_.V);
   pl.h_genes.resize((size_t)P * spec_.V);
-  pl.h_out.resize(out_doubles);
-  std::memset(pl.h_out.get(), 0, sizeof(double) * out_doubles);
+  pl.h_out.resize(pl.out_doubles());
+  std::memset(pl.h_out.get(), 0, sizeof(double) * pl.out_doubles());
   PopCtl& c = pl.ctl;
   c.K = pl.K;
   c.P = P;
@@ -797,6 +811,12 @@ void Fitness::build_quad_plan(PopPlan& pl, int P)
   c.fitness = reinterpret_cast<float*>(c.terms + 3 * (size_t)P);
   c.status = reinterpret_cast<unsigned*>(c.fitness + P);
   c.norm = norm();
+}
+
+void Fitness::build_quad_plan(PopPlan& pl, int P)
+{
+  hipStream_t st = stream_;
+  build_results(pl, P);
   const int ld = (P + QP - 1) / QP * QP;
   // (the linear block: zeros and the constant 1, the parameters written by
   // each launch)
@@ -819,6 +839,22 @@ void Fitness::build_quad_plan(PopPlan& pl, int P)
   q.part = pl.qpart.get();
   q.done = pl.qdone.get();
   pl.qnodes = NodeTable{quad_.basis, quad_.act.get(), quad_.n_act, pl.qvalues.get(), ld};
+  if (spec_.nn2b()) {
+    const int parts = nn2b_node_parts(P);
+    pl.qsums.resize((size_t)parts * kTailSums * ld);
+    pl.qcount.resize(2);
+    pl.qcount.zero(st);
+    pl.qlist.resize(P);
+    pl.qnodes.pairs = quad_.pairs.get();
+    pl.qnodes.tail = quad_.tail.get();
+    pl.qnodes.sums = pl.qsums.get();
+    const float limit = opt_.nn2b_bf16 && spec_.num_neurons <= 32 ? kTailBf16 : kTailFp32;
+    q.sharp.sums = pl.qsums.get();
+    q.sharp.parts = parts;
+    q.sharp.limit2 = limit * limit;
+    q.sharp.list = pl.qlist.get();
+    q.sharp.any = pl.h_sharp();
+  }
   GPUGA_HIP(hipStreamSynchronize(st));
 }
 
@@ -832,7 +868,24 @@ void Fitness::ensure_items(PopPlan& pl)
 void Fitness::launch_quad(PopPlan& pl, const PopCtl& ctl, hipStream_t st)
 {
   launch_quad_values(pl, ctl, 0, pl.P, st);
-  launch_quad_eval(ctl, pl.qeval, st);
+  launch_quad_eval(pl, ctl, st);
+}
+
+void Fitness::launch_quad_eval(PopPlan& pl, const PopCtl& ctl, hipStream_t st)
+{
+  if (pl.qeval.sharp.sums) {
+    pl.qeval.sharp.count = pl.qcount.get() + pl.qturn;
+    pl.qturn ^= 1;
+    pl.qeval.sharp.next = pl.qcount.get() + pl.qturn;
+  }
+  gpuga::launch_quad_eval(ctl, pl.qeval, st);
+}
+
+PopCtl Fitness::sharp_ctl(const PopPlan& pl, PopCtl ctl) const
+{
+  ctl.live = pl.qeval.sharp.count;
+  ctl.index = pl.qlist.get();
+  return ctl;
 }
 
 void Fitness::launch_quad_values(PopPlan& pl, const PopCtl& ctl, int first, int count,
@@ -876,7 +929,7 @@ size_t Fitness::device_bytes() const
   size_t b = ds_.bytes() + quad_.bytes() + d_f_.bytes() + d_virial_.bytes() + d_pe_.bytes() + d_cerr_.bytes();
   for (auto& kv : plans_) {
     const PopPlan& p = *kv.second;
-    b += p.qvalues.bytes() + p.qpart.bytes();
+    b += p.qvalues.bytes() + p.qpart.bytes() + p.qsums.bytes() + p.qlist.bytes();
     b += p.items.bytes() + p.part.bytes() + p.err.bytes() + p.bondf.bytes() + p.genes.bytes() +
          p.out.bytes() + p.gpart.bytes() + p.counters.bytes() + p.nn2b_table.bytes();
   }
@@ -928,10 +981,11 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   const bool tersoff = spec_.type == POT_TERSOFF1 || spec_.type == POT_TERSOFF2;
   // neighbour counts of the list the kernel reads (Tersoff: the pruned one)
   const NeighborList& pn = tersoff ? population_neighbors() : nl_;
-  pl.P = P;
+  // (a plan of the forms has results already, perhaps of a launch whose caller
+  // has not taken them yet)
+  if (pl.P == 0) build_results(pl, P);
   // the looped Tersoff kernel: one wave per workgroup (its LDS rows)
   pl.block = tersoff && loop_path_ ? WAVE : 256;
-  pl.K = (P + WAVE - 1) / WAVE;
   pl.chunk_cost = chunk_cost;
   const int tail_split = opt_.tail_split > 0 ? opt_.tail_split : 1;
   const int K = pl.K;
@@ -1168,12 +1222,6 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   pl.cfg_slot0.upload(slot0, st);
   pl.part.resize((size_t)std::max(slots, 1) * K * 8 * WAVE);
   pl.err.resize((size_t)K * 3 * Nc * WAVE);
-  // results in one buffer, so one copy returns them: terms [P][3] (FP64),
-  // fitness [P] (FP32), status word
-  const size_t out_doubles = 3 * (size_t)P + ((size_t)P + 1 + 1) / 2;
-  pl.out.resize(out_doubles);
-  pl.out.zero(st);
-  pl.genes.resize((size_t)P * spec_.V);
   const int B_force =
     ts_.N_force > 0 ? pn.start[ts_.N_force - 1] + pn.NN[ts_.N_force - 1] : 0;
   pl.bondf.resize(tersoff ? std::max<size_t>((size_t)K * (B_force + ts_.N_force) * 3 * WAVE, 1) : 1);
@@ -1190,9 +1238,6 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   const size_t closed0 = fetch0 + (size_t)nq * kFetchStride + 64;
   pl.counters.resize(closed0 + 2);
   pl.counters.zero(st);
-  pl.h_genes.resize((size_t)P * spec_.V);
-  pl.h_out.resize(out_doubles);
-  std::memset(pl.h_out.get(), 0, sizeof(double) * out_doubles);
 
   PopCtl& c = pl.ctl;
   c.items = pl.items.get();
@@ -1201,14 +1246,8 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   c.qstart = pl.qstart.get();
   c.home = n_home > 0 ? pl.home.get() : nullptr;
   c.n_home = n_home;
-  c.K = K;
-  c.P = P;
-  c.V = spec_.V;
   c.cfg_nchunks = pl.cfg_nchunks.get();
   c.cfg_slot0 = pl.cfg_slot0.get();
-  c.genes = pl.genes.get();
-  c.pmin = d_pmin_.get();
-  c.pmax = d_pmax_.get();
   c.part = pl.part.get();
   c.bondf = pl.bondf.get();
   c.B_force = B_force + ts_.N_force; // slots per lane block: bonds, then atoms
@@ -1221,13 +1260,9 @@ void Fitness::build_plan(PopPlan& pl, int P, const LaunchShape& sh)
   c.fetch = ctr + fetch0;
   c.done = c.fetch + (size_t)nq * kFetchStride;
   c.closed = reinterpret_cast<unsigned long long*>(ctr + closed0);
-  c.terms = pl.out.get();
-  c.fitness = reinterpret_cast<float*>(c.terms + 3 * (size_t)P);
-  c.status = reinterpret_cast<unsigned*>(c.fitness + P);
   c.gpart = pl.gpart.get();
   c.cfg_group = cfg_group;
   c.spin_limit = spin_limit_;
-  c.norm = norm();
   GPUGA_HIP(hipStreamSynchronize(st));
   pl.items_built = true;
 }
@@ -1298,6 +1333,12 @@ void Fitness::compute_async(int P, const float* genes, int share)
   // (a set with quadratic forms, genes outside their range: the pair loop)
   const bool quad = quad_for(P, genes);
   if (!quad) ensure_items(pl);
+  // Where the call before this one listed individuals that the forms do not
+  // resolve, their launch follows the forms' at once, not after the host has
+  // seen this call's list (which decides, so the results are the same): 70
+  // individuals of 32 neurons, half of them listed, a call of 151 -> 121 us.
+  const bool again = quad && pl.sharp_before && pl.items_built;
+  pl.sharp_open = quad && !again;
   // The generation is launched directly (a graph of one or two kernels takes
   // 14 us longer to launch and wait for), and its last kernel writes the
   // results to the pinned block: a copy back would be one more operation on
@@ -1305,10 +1346,11 @@ void Fitness::compute_async(int P, const float* genes, int share)
   PopCtl ctl = pl.ctl;
   ctl.terms = pl.h_out.get();
   ctl.fitness = reinterpret_cast<float*>(ctl.terms + 3 * (size_t)P);
-  ctl.status = reinterpret_cast<unsigned*>(ctl.fitness + P);
+  ctl.status = pl.h_status();
   *ctl.status = 0u;
+  *pl.h_sharp() = 0u;
   float* h = pl.h_genes.get();
-  if (quad) {
+  if (quad && !again) {
     // The genes are read in place, each once or a few times.  From 64 Ki genes
     // on in two halves, the second one's copied while the first one's values
     // are computed (256 x 1153: a call of 77 us, 89 in one piece, 83 in three).
@@ -1321,7 +1363,7 @@ void Fitness::compute_async(int P, const float* genes, int share)
       std::memcpy(h + at, genes + at, sizeof(float) * (size_t)(p1 - p0) * spec_.V);
       launch_quad_values(pl, ctl, p0, p1 - p0, st);
     }
-    launch_quad_eval(ctl, pl.qeval, st);
+    launch_quad_eval(pl, ctl, st);
   } else {
     const size_t bytes = sizeof(float) * (size_t)P * spec_.V;
     std::memcpy(h, genes, bytes);
@@ -1329,6 +1371,10 @@ void Fitness::compute_async(int P, const float* genes, int share)
     if (bytes <= 64u * 1024u) launch_copy_in(h, pl.genes.get(), P * spec_.V, st);
     else GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), h, bytes, hipMemcpyHostToDevice, st));
     if (timing_) GPUGA_HIP(hipEventRecord(ev0_, st));
+    if (again) {
+      launch_quad(pl, ctl, st);
+      ctl = sharp_ctl(pl, ctl);
+    }
     // share 1, 2, 4 or 8 (rounded up, at most 8): 1/share of the grid (the
     // quadratic forms' launches are short and fill a part of the GPU by
     // themselves)
@@ -1367,6 +1413,26 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
   const GA before = ga;
   if (!pl.dga || !pl.dga->matches(ga))
     pl.dga = std::make_unique<DeviceGA>(ga, pl.genes.get(), 1024, st, opt_.ga_batch);
+  const auto run = [&] {
+    const bool done = run_generations(pl, ga, first_generation, generations, quad, best, elite);
+    if (!done) ga = before;
+    return done;
+  };
+  if (!run()) {
+    // An individual that the forms do not resolve: the pair loop's tables are
+    // built (once, and only where a run meets one), and the run starts again.
+    // Its generations up to there are the same bit for bit.
+    ensure_items(pl);
+    run();
+  }
+}
+
+bool Fitness::run_generations(PopPlan& pl, GA& ga, int first_generation, int generations,
+                              bool quad, float* best, float* elite)
+{
+  const int V = spec_.V;
+  hipStream_t st = stream_;
+  const GA before = ga;
   DeviceGA& dga = *pl.dga;
   dga.upload(ga, first_generation, st);
   // batches double from one generation up to the staging capacity, so the
@@ -1379,6 +1445,12 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
   // process's first long run up to 4 ms)
   const int H = dga.history_cap();
   std::vector<float> h((size_t)H * (1 + V));
+  // With the pair loop's tables there, each generation's listed individuals are
+  // evaluated again before the GA step (two launches that end at once when
+  // there are none); without them the run ends where there is one.
+  const bool check = quad && pl.qeval.sharp.sums, again = check && pl.items_built;
+  *pl.h_sharp() = 0u;
+  const volatile unsigned* sharp = pl.h_sharp();
   int g = 0; // generations queued
   while (g < generations) {
     const int n = std::min(H, generations - g);
@@ -1394,11 +1466,17 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
         ctl.genes = dga.genes(k);
         if (quad) launch_quad(pl, ctl, st);
         else launch_population(pl, ctl, st);
+        if (again) launch_population(pl, sharp_ctl(pl, ctl), st);
         dga.step(k, pl.ctl.fitness, st);
+      }
+      if (check && !again && *sharp) {
+        GPUGA_HIP(hipStreamSynchronize(st));
+        return false;
       }
     }
     if (timing_) GPUGA_HIP(hipEventRecord(ev1_, st));
     const unsigned status = dga.collect((g + n) & 1, n, pl.ctl.status, st);
+    if (check && !again && *sharp) return false;
     if (timing_) {
       float ms = 0.0f;
       GPUGA_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
@@ -1421,6 +1499,7 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
     g += n;
   }
   dga.download(ga, generations & 1, st);
+  return true;
 }
 
 void Fitness::discard_launch(PopPlan& pl)
@@ -1459,8 +1538,28 @@ void Fitness::compute_wait(float* fitness, double* terms)
   pending_P_ = 0;
   const double* h_terms = pl.h_out.get();
   const float* h_fitness = reinterpret_cast<const float*>(h_terms + 3 * (size_t)P);
-  const unsigned h_status = *reinterpret_cast<const unsigned*>(h_fitness + P);
-  if (h_status != 0u) discard_launch(pl);
+  pl.sharp_before = *pl.h_sharp() != 0u;
+  if (pl.sharp_open && pl.sharp_before) {
+    // the individuals that the forms do not resolve, by the pair loop
+    ensure_items(pl);
+    hipStream_t st = stream_;
+    GPUGA_HIP(hipMemcpyAsync(pl.genes.get(), pl.h_genes.get(),
+                             sizeof(float) * (size_t)P * spec_.V, hipMemcpyHostToDevice, st));
+    PopCtl ctl = sharp_ctl(pl, pl.ctl);
+    ctl.terms = pl.h_out.get();
+    ctl.fitness = reinterpret_cast<float*>(ctl.terms + 3 * (size_t)P);
+    ctl.status = pl.h_status();
+    if (timing_) GPUGA_HIP(hipEventRecord(ev0_, st));
+    launch_population(pl, ctl, st);
+    if (timing_) GPUGA_HIP(hipEventRecord(ev1_, st));
+    GPUGA_HIP(hipStreamSynchronize(st));
+    if (timing_) {
+      float ms = 0.0f;
+      GPUGA_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
+      kernel_ms_ += ms;
+    }
+  }
+  if (*pl.h_status() != 0u) discard_launch(pl);
   if (fitness) std::memcpy(fitness, h_fitness, sizeof(float) * P);
   if (terms) std::memcpy(terms, h_terms, sizeof(double) * 3 * P);
 }

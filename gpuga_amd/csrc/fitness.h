@@ -86,6 +86,8 @@ struct QuadSet {
   DeviceBuffer<double> q[3];
   DeviceBuffer<int> vblk[3];
   DeviceBuffer<int2> unit, act;
+  DeviceBuffer<float2> pairs; // NN2B's check of the nodes (SharpSet)
+  DeviceBuffer<float> tail;
   size_t bytes() const
   {
     return q[0].bytes() + q[1].bytes() + q[2].bytes() + act.bytes();
@@ -98,6 +100,14 @@ struct PopPlan {
   bool items_built = false; // the work items of the population kernel are there
   DeviceBuffer<double> qvalues, qpart; // quadratic forms: values, row-block sums
   DeviceBuffer<unsigned> qdone;
+  // individuals of the last launch that the nodes do not resolve: sums of the
+  // check, two counters (launches use them in turn), the list
+  DeviceBuffer<float> qsums;
+  DeviceBuffer<unsigned> qcount;
+  DeviceBuffer<int> qlist;
+  int qturn = 0;
+  bool sharp_open = false;   // the launch in flight may list some, unevaluated
+  bool sharp_before = false; // the call before this one listed some
   QuadEval qeval{};
   NodeTable qnodes{};
   int P = 0, K = 0, n_items = 0, grid = 0, block = 256, chunk_cost = 0;
@@ -113,7 +123,15 @@ struct PopPlan {
   DeviceBuffer<float> bondf, genes, nn2b_table;
   DeviceBuffer<unsigned> counters; // cnt | cnt2 | grp_done | blk_done | fetch
   PinnedBuffer<float> h_genes;
+  // terms, fitness, status word, and a word that is set when the launch's forms
+  // do not resolve some individual
   PinnedBuffer<double> h_out;
+  size_t out_doubles() const { return 3 * (size_t)P + ((size_t)P + 2 + 1) / 2; }
+  unsigned* h_status() const
+  {
+    return reinterpret_cast<unsigned*>(reinterpret_cast<float*>(h_out.get() + 3 * (size_t)P) + P);
+  }
+  unsigned* h_sharp() const { return h_status() + 1; }
   PopCtl ctl{};
   // device GA of this population size (a generation on population buffer b
   // writes the next into buffer 1 - b)
@@ -210,6 +228,7 @@ private:
   // of a set with quadratic forms first needs them)
   void build_pair_tables();
   void ensure_items(PopPlan& pl);
+  void build_results(PopPlan& pl, int P);
   void build_quad_plan(PopPlan& pl, int P);
   // whether genes [P][V] are evaluated by the quadratic forms
   bool quad_for(int P, const float* genes) const;
@@ -220,8 +239,16 @@ private:
   // the population launch of ctl (the plan's, or a copy with other genes or
   // results); grid 0: the plan's
   void launch_population(PopPlan& pl, const PopCtl& ctl, hipStream_t st, int grid = 0);
-  // the same by the quadratic forms (their values, then their evaluation)
+  // the same by the quadratic forms: their values, then their evaluation, which
+  // lists the individuals to be evaluated again
   void launch_quad(PopPlan& pl, const PopCtl& ctl, hipStream_t st);
+  void launch_quad_eval(PopPlan& pl, const PopCtl& ctl, hipStream_t st);
+  // ctl's launch for the individuals that the last launch_quad_eval listed
+  PopCtl sharp_ctl(const PopPlan& pl, PopCtl ctl) const;
+  // run_ga's generations; false, with the GA's state to be restored, when they
+  // need the pair loop's tables and these are not there
+  bool run_generations(PopPlan& pl, GA& ga, int first_generation, int generations, bool quad,
+                       float* best, float* elite);
   void launch_quad_values(PopPlan& pl, const PopCtl& ctl, int first, int count, hipStream_t st);
   double time_plan(int P, const LaunchShape& sh, int reps, int* occ = nullptr);
   // after a launch whose status word is set: clear the plan's counters and

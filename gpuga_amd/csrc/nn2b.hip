@@ -33,8 +33,10 @@ __global__ void __launch_bounds__(256) nn2b_tabulate_f32(PopCtl ctl, NN2BGrid gr
   extern __shared__ float w[];
   const int p = blockIdx.y, code = blockIdx.z;
   const int n = grid.n, V = ctl.V;
+  if (ctl.live && p >= (int)ldu(ctl.live, 0)) return;
+  const float* genes = ctl.genes + (size_t)(ctl.live ? ctl.index[p] : p) * V;
   for (int v = threadIdx.x; v < V; v += blockDim.x)
-    w[v] = denormalise(ctl.pmin[v], ctl.pmax[v], ctl.genes[(size_t)p * V + v]);
+    w[v] = denormalise(ctl.pmin[v], ctl.pmax[v], genes[v]);
   __syncthreads();
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= grid.G) return;
@@ -87,6 +89,7 @@ __global__ void __launch_bounds__(256) nn2b_tabulate_f32(PopCtl ctl, NN2BGrid gr
 
 struct NN2BPop {
   static constexpr int kWaves = 2, kWavesPacked = 2;
+  static constexpr bool kSubset = true;
   static constexpr bool kForcePass = false;
   static constexpr int kFoldValues = 12;
   static constexpr bool kPacked = false;

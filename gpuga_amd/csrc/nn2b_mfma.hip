@@ -50,7 +50,8 @@ __global__ void __launch_bounds__(64) nn2b_tabulate_bf16(PopCtl ctl, NN2BGrid gr
   const int p = blockIdx.y, code = blockIdx.z;
   const int l = threadIdx.x, col = l & 31, kg = l >> 5;
   const int n = grid.n, V = ctl.V;
-  const float* gp = ctl.genes + (size_t)p * V;
+  if (ctl.live && p >= (int)ldu(ctl.live, 0)) return;
+  const float* gp = ctl.genes + (size_t)(ctl.live ? ctl.index[p] : p) * V;
   auto W = [&](int v) { return denormalise(ctl.pmin[v], ctl.pmax[v], gp[v]); };
 
   // input neurons of this lane, in its A and B operands alike:

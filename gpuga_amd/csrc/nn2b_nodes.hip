@@ -15,15 +15,22 @@
 // together), a product accumulated as lo lo + lo hi + hi lo + hi hi (n <= 32).
 // Otherwise v_mfma_f32_32x32x2_f32.
 //
+// Each element's last coefficients are taken for the check of SharpSet (quadform.h).
+//
 // Bound by the 2 n tanh of a node (two transcendental instructions each) and,
-// with genes in host memory, by their transfer.  256 individuals, n = 32, 512
-// nodes: 12.5 us from device memory in BF16 (20.9 us with a wave per four
-// elements that gathered its weights and summed the output layer through
-// LDS; 14.7 us with the layers' vectors in registers, two waves a SIMD), 32 us
-// from host memory, where the transfer alone takes 20; 100 individuals, n = 20,
-// three species codes, FP32: 20 us (28.9 us with a thread per node on the
-// VALU).  BF16 costs what FP32 does here: its splits take the VALU as long as
-// FP32 products the matrix unit.
+// with genes in host memory, by their transfer.  Without the check 256
+// individuals, n = 32, 512 nodes took 12.5 us from device memory in BF16 (20.9 us
+// with a wave per four elements that gathered its weights and summed the
+// output layer through LDS; 14.7 us with the layers' vectors in registers, two
+// waves a SIMD), two halves from host memory 19.9 us each, of which the transfer
+// alone takes 10; 100 individuals, n = 20, three species codes, FP32: 21.9 us
+// (28.9 us with a thread per node on the VALU).  The check adds 1.5 and 0.6 us
+// (the magnitudes two instructions a neuron, the coefficients a chain of
+// exchanges; through LDS instead of DPP 0.5 us more).  BF16 costs what FP32
+// does here: its splits take the VALU as long as FP32 products the matrix unit.
+// (Its tanh as FP32's: 1 - t t loses the derivative of a saturated neuron, and
+// the check then takes the rounding of 1 in 100 networks of 6 neurons for
+// sharpness.)
 #include "quadform.h"
 
 namespace gpuga {
@@ -59,6 +66,25 @@ __device__ inline f32x16 mfma4(const bf16x8& ah, const bf16x8& al, const bf16x8&
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, c, 0, 0, 0);
 }
 
+// Four values of each lane summed over its 32 lanes: lane c returns the sum of
+// value 2 (c % 2) + c / 2 % 2.
+template <int CTRL>
+__device__ inline float dpp(float x)
+{
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+__device__ inline float sums_of_four(const float (&v)[4], int c)
+{
+  constexpr int XOR1 = 0xb1, XOR2 = 0x4e, ROR4 = 0x124, ROR8 = 0x128; // in rows of 16
+  const bool a = c & 1, b = c & 2;
+  const float x = (a ? v[2] : v[0]) + dpp<XOR1>(a ? v[0] : v[2]);
+  const float y = (a ? v[3] : v[1]) + dpp<XOR1>(a ? v[1] : v[3]);
+  float s = (b ? y : x) + dpp<XOR2>(b ? x : y);
+  s += dpp<ROR4>(s);
+  s += dpp<ROR8>(s);
+  return s + __shfl_xor(s, 16);
+}
+
 // KS: input neurons per half-wave (n <= 2 KS); NB: blocks of 32 output
 // neurons.  Half-wave h holds the input neurons m(s) = 2 s + h (FP32: one pair
 // per instruction) or 16 (s / 8) + 8 h + s % 8 (BF16: eight per operand), and
@@ -76,6 +102,13 @@ __global__ void __launch_bounds__(WAVES * WAVE) nn2b_nodes(PopCtl ctl, int n, in
   const int p = first + blockIdx.y;
   const int V = ctl.V, t = threadIdx.x;
   const float* genes = ctl.genes + (size_t)min(p, ctl.P - 1) * V;
+  const int lane = __lane_id(), col = lane & 31, half = lane >> 5;
+  // the check that the nodes resolve the curve (SharpSet): this lane's factors,
+  // and its sums over the energy, then the force configurations' pairs
+  static_assert(QTAIL == 4, "sums_of_four");
+  float tf[QTAIL], sums[4] = {};
+#pragma unroll
+  for (int k = 0; k < QTAIL; ++k) tf[k] = tab.tail[k * QB + col];
   constexpr int T = WAVES * WAVE, LOADS = 4;
   for (int k = t; k < 2 * KS; k += T) l1[k] = make_float4(0, 0, 0, 0);
   for (int k = t; k < NB * 32; k += T) l2[k] = make_float2(0, 0);
@@ -107,7 +140,6 @@ __global__ void __launch_bounds__(WAVES * WAVE) nn2b_nodes(PopCtl ctl, int n, in
     }
   }
   __syncthreads();
-  const int lane = __lane_id(), col = lane & 31, half = lane >> 5;
   auto m_of = [&](int s) { return BF16 ? 16 * (s / 8) + 8 * half + s % 8 : 2 * s + half; };
   auto A = [&](int row, int s) {
     const int m = m_of(s);
@@ -133,21 +165,14 @@ __global__ void __launch_bounds__(WAVES * WAVE) nn2b_nodes(PopCtl ctl, int n, in
     float base = 0.0f; // code 0's U (half 0) or U' (half 1) at the node
     for (int code = 0; code < tab.b.codes; ++code) {
       if (!((el.y >> code) & 1)) continue;
+      const float2 pairs = ldu(tab.pairs, code * E + el.x);
       f32x16 z[NB] = {}, zd[NB] = {};
-      auto tanh_s = [](float x, float& t, float& s) {
-        if constexpr (BF16) { // (the operands' 16 bits set the error)
-          t = ftanh(x);
-          s = fmaf(-t, t, 1.0f);
-        } else {
-          tanh_sech2(x, t, s);
-        }
-      };
       auto layer1 = [&](int s, float& x, float& y) {
         const float4 l = l1[m_of(s)];
         // the species-pair input as a shift of the bias
         const float bias = species ? l.y - l.z * (float)code : l.y;
         float sg;
-        tanh_s(l.x * d - bias, x, sg);
+        tanh_sech2(l.x * d - bias, x, sg);
         y = sg * l.x;
       };
       if constexpr (BF16) {
@@ -177,25 +202,49 @@ __global__ void __launch_bounds__(WAVES * WAVE) nn2b_nodes(PopCtl ctl, int n, in
           }
         }
       }
-      float u = 0.0f, g = 0.0f;
+      float u = 0.0f, g = 0.0f, um = 0.0f, gm = 0.0f;
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float2 l = l2[32 * b + 8 * (r >> 2) + 4 * half + (r & 3)];
           float x, sg;
-          tanh_s(z[b][r] - l.x, x, sg);
+          tanh_sech2(z[b][r] - l.x, x, sg);
           u = fmaf(l.y, x, u);
           g = fmaf(l.y * sg, zd[b][r], g);
+          um = fmaf(__builtin_fabsf(l.y), __builtin_fabsf(x), um);
+          gm = fmaf(__builtin_fabsf(l.y * sg), __builtin_fabsf(zd[b][r]), gm);
         }
-      u = (u + __shfl_xor(u, 32)) - bias2;
-      g += __shfl_xor(g, 32);
-      const float mine = half ? g : u;
+      // half 0 takes U, half 1 takes U'
+      float mine = (half ? g : u) + __shfl_xor(half ? u : g, 32);
+      float mag = (half ? gm : um) + __shfl_xor(half ? um : gm, 32);
+      if (!half) {
+        mine -= bias2;
+        mag += __builtin_fabsf(bias2);
+      }
+      // one of the last coefficients in each lane
+      const float c =
+        sums_of_four({tf[0] * mine, tf[1] * mine, tf[2] * mine, tf[3] * mine}, col);
+      sums[0] = fmaf(pairs.x * c, c, sums[0]);
+      sums[1] = fmaf(pairs.x * mag, mag, sums[1]);
+      sums[2] = fmaf(pairs.y * c, c, sums[2]);
+      sums[3] = fmaf(pairs.y * mag, mag, sums[3]);
       if (code == 0) base = mine;
       // (the codes above 0 as differences from code 0, quadform.h)
       tab.values[((long)(half * CE + code * E + el.x) * QB + col) * tab.ld + p] =
         code == 0 ? (double)mine : (double)mine - (double)base;
     }
+  }
+  __shared__ float all[WAVES][kTailSums];
+  const float sum = sums_of_four(sums, col);
+  const int k = 2 * (col & 1) + (col >> 1); // energy: U; virial and force: U'
+  if (col < 4 && k + 2 * half < kTailSums && (half || k < 2)) all[t / WAVE][k + 2 * half] = sum;
+  __syncthreads();
+  if (t < kTailSums) {
+    float x = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) x += all[w][t];
+    tab.sums[((long)blockIdx.x * kTailSums + t) * tab.ld + p] = x;
   }
 }
 
@@ -207,7 +256,7 @@ void launch(const PopCtl& ctl, const NN2BGrid& g, const NodeTable& t, int first,
 {
   const size_t lds = sizeof(float) * g.n * (g.n + 1);
   const int species = g.codes > 1 ? 1 : 0;
-  if (ctl.P >= 128)
+  if (nn2b_node_parts(ctl.P) == 1)
     nn2b_nodes<BF16, KS, NB, WAVES>
       <<<dim3(1, count), WAVES * WAVE, lds, st>>>(ctl, g.n, species, t, first);
   else

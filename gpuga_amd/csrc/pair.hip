@@ -128,6 +128,7 @@ __device__ inline RILane ri_lane(const RIParams& p)
 
 struct RIPop {
   static constexpr int kWaves = 2, kWavesPacked = 2;
+  static constexpr bool kSubset = false;
   static constexpr bool kForcePass = false;
   static constexpr int kFoldValues = 12;
   static constexpr bool kPacked = false;

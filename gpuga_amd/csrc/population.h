@@ -93,6 +93,11 @@ struct PopCtl {
   int n_home;
   int K;                  // lane blocks
   int P, V;
+  // NN2B, a launch for a part of the population: individuals index[0], ...,
+  // index[*live - 1] (device memory), lane by lane; nothing runs where *live is
+  // 0.  Null: all of it.
+  const unsigned* live;
+  const int* index;
   const int* cfg_nchunks; // [Nc]
   const int* cfg_slot0;   // [Nc] first partial slot of configuration c
   const float* genes;     // [P][V] in [0,1]
@@ -230,9 +235,15 @@ __device__ inline void sum_rows(const double* const (&a)[NA], long stride, int n
 }
 
 // Fitness and terms of individual p (nothing past the population) from the
-// sums of the three error terms over all configurations.
+// sums of the three error terms over all configurations.  SUBSET: p counts the
+// launch's part of the population (PopCtl::live).
+template <bool SUBSET = false>
 __device__ inline void write_fitness(const PopCtl& ctl, int p, const double (&s)[3])
 {
+  if (SUBSET && ctl.live) {
+    if (p >= (int)ldu(ctl.live, 0)) return;
+    p = ctl.index[p];
+  }
   const double tE = sqrt(s[0] * ctl.norm.inv_pss);
   const double tW = sqrt(s[1] * ctl.norm.inv_vss);
   const double tF = sqrt(s[2] * ctl.norm.inv_fss);
@@ -250,7 +261,7 @@ __device__ inline void write_fitness(const PopCtl& ctl, int p, const double (&s)
 // through the group and lane-block reductions, writing the fitness when the
 // lane block is complete (then it returns true).  Only the terms a
 // configuration has are stored and read back.
-template <int VALS>
+template <int VALS, bool SUBSET>
 __device__ inline bool config_done(const PopCtl& ctl, int Nc, int Nc_force, int c, int k,
                                    int lane, double eE, double eW, double eF)
 {
@@ -281,7 +292,7 @@ __device__ inline bool config_done(const PopCtl& ctl, int Nc, int Nc_force, int 
   sum_rows<2, VALS>(ee, WAVE, g0 + gn - fe, s);
   s[2] = f[0];
   if (groups == 1) {
-    write_fitness(ctl, k * WAVE + lane, s);
+    write_fitness<SUBSET>(ctl, k * WAVE + lane, s);
     return true;
   }
   double* gp = ctl.gpart + ((long)k * groups + g) * 3 * WAVE + lane;
@@ -296,7 +307,7 @@ __device__ inline bool config_done(const PopCtl& ctl, int Nc, int Nc_force, int 
   const double* gb = ctl.gpart + (long)k * groups * 3 * WAVE + lane;
   const double* const eg[3] = {gb, gb + WAVE, gb + 2 * WAVE};
   sum_rows<3, VALS>(eg, 3 * WAVE, groups, s);
-  write_fitness(ctl, k * WAVE + lane, s);
+  write_fitness<SUBSET>(ctl, k * WAVE + lane, s);
   return true;
 }
 
@@ -472,6 +483,8 @@ __device__ __forceinline__ KernelArgs<Extra> kernel_args()
 //   static constexpr int kWaves, kWavesPacked;      waves per SIMD that the
 //                                                   registers must allow (with
 //                                                   the packed code)
+//   static constexpr bool kSubset;                  serves a part of the population
+//                                                   (PopCtl::live; no packed items)
 //   static constexpr bool kForcePass;               three-body force assembly
 //   static double force_pass(set, ctl, ex, a0, a1, k, lane)
 //                                                   sum |F-F_ref|^2 over [a0, a1)
@@ -500,6 +513,9 @@ __global__ void __launch_bounds__(256, LONE ? 1 : PACK ? Pot::kWavesPacked : Pot
   const unsigned wave_slot = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
   unsigned prev = 0xffffffffu;
   const PopCtl& ctl0 = kernel_args<Extra>().ctl;
+  if constexpr (Pot::kSubset) {
+    if (ctl0.live && ldu(ctl0.live, 0) == 0u) return; // (all waves alike)
+  }
   const unsigned long long t_entry = ctl0.trace ? wall_clock64() : 0ull;
   // home queue: one of the queues of this wave's XCD (workgroups of one XCD
   // spread over its queues)
@@ -565,6 +581,9 @@ __global__ void __launch_bounds__(256, LONE ? 1 : PACK ? Pot::kWavesPacked : Pot
     }
     const WorkItem item = ldu(ctl.items, it);
     const int c = item.c, k = item.k;
+    if constexpr (Pot::kSubset) {
+      if (ctl.live && k * WAVE >= (int)ldu(ctl.live, 0)) continue;
+    }
     const int nch = ldu(ctl.cfg_nchunks, c);
     const bool is_force = c < set.Nc_force;
     unsigned* cnt = &ctl.cnt[(long)c * ctl.K + k];
@@ -669,7 +688,7 @@ __global__ void __launch_bounds__(256, LONE ? 1 : PACK ? Pot::kWavesPacked : Pot
     // the launch has finished, so every queue is empty: this wave goes
     // straight to the exit (two memory round trips less at the end of the
     // launch's longest chain).
-    if (config_done<FV>(done.ctl, done.set.Nc, done.set.Nc_force, c, k, lane, eE, eW, eF) &&
+    if (config_done<FV, Pot::kSubset>(done.ctl, done.set.Nc, done.set.Nc_force, c, k, lane, eE, eW, eF) &&
         done.ctl.K == 1)
       skip_fetch = true;
   }

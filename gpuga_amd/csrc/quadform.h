@@ -56,6 +56,35 @@ struct QuadForm {
 };
 constexpr long quad_tiles(long nb) { return nb * (nb + 1) / 2; }
 
+// Do the nodes resolve an individual's curve?  Its last QTAIL Chebyshev
+// coefficients in each element show it: where they are small the series has
+// converged and the interpolation error is about theirs, else the individual's
+// fitness by the forms is not to be used.  Compared are the mean squares, over
+// the pairs of the set, of the coefficients and of the terms' magnitude (the
+// sum of |w2 tanh| for U, of |w2 sech^2 dz/dr| for U'), which is what the
+// nodes' rounding is relative to: of U and U' over the energy configurations'
+// pairs, of U' over the force configurations'.
+//
+// Limits: the coefficients of smooth networks, rounding alone, reach 3.4e-7 of
+// the magnitude with the FP32 layer and 7e-6 with the split BF16 one (6000
+// networks of 6 to 32 neurons with weights up to 3, and weights up to 6); at the
+// limits the interpolation errs by up to 1.8e-6 and 2e-5 of U' (root mean
+// square), the BF16 layer's rounding of the nodes by 2e-5 to 1e-4.  The pair
+// loop's interpolation errs by up to 6e-6 for networks with weights uniform in
+// [-3, 3] and 32 neurons on 1024 points, more for sharper ones.
+constexpr int QTAIL = 4;
+constexpr int kTailSums = 6; // (coefficients, magnitude) of energy, virial, force
+constexpr float kTailFp32 = 1e-6f, kTailBf16 = 1e-5f;
+struct SharpSet {
+  const float* sums; // [parts][kTailSums][ld]; null: no check (rigid ion)
+  int parts;
+  float limit2;      // square of the limit
+  unsigned* count;   // individuals found by this launch, and, cleared by it,
+  unsigned* next;    // the counter of the next one
+  int* list;         // [P] the individuals, in any order
+  unsigned* any;     // set to 1 when there are some (pinned host memory)
+};
+
 // Evaluation of all forms for a population: values [blocks][QB][ld].
 struct QuadEval {
   QuadForm form[3]; // energy, virial, force
@@ -65,6 +94,7 @@ struct QuadEval {
   int ld;           // individuals, padded to a multiple of QP
   double* part;     // [units][ld] row-block sums
   unsigned* done;   // [ld / QP]
+  SharpSet sharp;   // individuals that the nodes do not resolve
 };
 
 // Where the tabulation kernels put U and U' of the nodes.
@@ -76,6 +106,12 @@ struct NodeTable {
   int n_act;
   double* values;
   int ld;
+  // NN2B: pairs of energy and force configurations in each element of each
+  // code, and the rows k = QB - QTAIL, ... of the transform to Chebyshev
+  // coefficients, (2 / QB) cos(k theta_m); where the check's sums go
+  const float2* pairs; // [CE]
+  const float* tail;   // [QTAIL][QB]
+  float* sums;
 };
 
 // A training set's rows, for the set-up.  col[0][form][block]: column block
@@ -93,7 +129,9 @@ void launch_bond_range(int B, const float4* bond, unsigned* range, hipStream_t s
 // per-bond rigid-ion factors (r^-6, erfc(a r)/r, -(d/dr) erfc(a r)/r, 1/r)
 void launch_ri_table(int B, const float4* bond, float4* tab, hipStream_t st);
 // used[force][taper][CE]: elements the pairs of energy / force configurations
-// fall into (taper: those of pairs inside the NN2B taper)
+// fall into (taper: those of pairs inside the NN2B taper); then [force][CE]: how
+// many pairs (at most QCE elements of all codes)
+constexpr int QCE = 64;
 void launch_quad_used(const DevSet& s, const QuadBasis& b, int* used, hipStream_t st);
 size_t quad_energy_lds(const QuadRows& q);
 void quad_prepare(const QuadRows& q); // raises the row kernels' LDS limits
@@ -111,6 +149,8 @@ void launch_quad_gram(const double* R, int rows, int nb, int splits, bool first,
 void launch_quad_finish(const double* part, int nb, int splits, double* q, hipStream_t st);
 
 void launch_ri_values(const PopCtl& ctl, const NodeTable& t, hipStream_t st);
+// workgroups an individual (parts of its check's sums)
+constexpr int nn2b_node_parts(int P) { return P >= 128 ? 1 : 2; }
 // the individuals [first, first + count)
 void launch_nn2b_nodes(const PopCtl& ctl, const NN2BGrid& g, const NodeTable& t, int first,
                        int count, hipStream_t st);

@@ -88,10 +88,13 @@ __device__ __forceinline__ void nn2b_taper(double d, double& fc, double& fcp)
 
 __global__ void __launch_bounds__(256) quad_used(DevSet s, QuadBasis b, int* used)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= s.N) return;
-  const int force = i < s.N_force ? 1 : 0, CE = b.CE();
-  for (int k = s.bond0[i]; k < s.bond0[i] + s.nn[i]; ++k) {
+  __shared__ int pairs[2 * QCE];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, CE = b.CE();
+  for (int x = threadIdx.x; x < 2 * CE; x += blockDim.x) pairs[x] = 0;
+  __syncthreads();
+  const int force = i < s.N_force ? 1 : 0;
+  const int k0 = i < s.N ? s.bond0[i] : 0, k1 = i < s.N ? k0 + s.nn[i] : 0;
+  for (int k = k0; k < k1; ++k) {
     if (!force && s.nl[k] < i) continue;
     const float d = s.bond[k].w;
     const int ce = locate(b, d, b.codes > 1 ? s.ptype[k] : 0, nullptr);
@@ -99,12 +102,16 @@ __global__ void __launch_bounds__(256) quad_used(DevSet s, QuadBasis b, int* use
     const bool taper = !b.rigid && d >= NN2B_R1 && d < NN2B_R2;
     int* u = used + 2 * force * CE;
     u[ce] = 1;
+    atomicAdd(&pairs[force * CE + ce], 1);
     if (b.species()) u[ce % b.E] = 1;
     if (taper) {
       u[CE + ce] = 1;
       if (b.species()) u[CE + ce % b.E] = 1;
     }
   }
+  __syncthreads();
+  for (int x = threadIdx.x; x < 2 * CE; x += blockDim.x)
+    if (pairs[x]) atomicAdd(&used[4 * CE + x], pairs[x]);
 }
 
 // A pair as the row kernels read it from LDS.
@@ -453,6 +460,7 @@ __global__ void __launch_bounds__(EVAL_WAVES * WAVE, 4) quad_eval(PopCtl ctl, Qu
   const int groups = q.ld / QP;
   const int unit = (int)blockIdx.x / kXcds / groups * kXcds + (int)blockIdx.x % kXcds;
   const int pb = (int)blockIdx.x / kXcds % groups;
+  if (q.sharp.sums && blockIdx.x == 0 && threadIdx.x == 0) *q.sharp.next = 0u;
   if (unit >= q.units) return;
   const int2 fi = ldu(q.unit, unit);
   const int f = fi.x, I = fi.y;
@@ -520,12 +528,34 @@ __global__ void __launch_bounds__(EVAL_WAVES * WAVE, 4) quad_eval(PopCtl ctl, Qu
   // row block r of a form in slice r % SLICES, then the slices in order
   const int l = t % QP, sl = t / QP;
   int first = 0;
+  float tail[2][kTailSums] = {};
+  if (q.sharp.sums && t < QP)
+#pragma unroll
+    for (int k = 0; k < kTailSums; ++k) {
+      tail[0][k] = q.sharp.sums[(long)k * ld + p0 + t];
+      if (q.sharp.parts > 1) tail[1][k] = q.sharp.sums[(long)(kTailSums + k) * ld + p0 + t];
+    }
 #pragma unroll
   for (int s = 0; s < 3; ++s) {
     double x = 0.0;
     for (int r = sl; r < q.form[s].nb; r += SLICES) x += cload(part + (first + r) * ld + l);
     fold[s][sl][l] = x;
     first += q.form[s].nb;
+  }
+  bool resolved = true;
+  if (q.sharp.sums && t < QP && p0 + t < ctl.P) {
+#pragma unroll
+    for (int k = 0; k < kTailSums; k += 2) { // (a NaN or an infinite sum: not)
+      const float c = tail[0][k] + tail[1][k], size = tail[0][k + 1] + tail[1][k + 1];
+      resolved = resolved && c <= q.sharp.limit2 * size && size < __builtin_inff();
+    }
+  }
+  const unsigned long long m = __ballot(!resolved);
+  if (w == 0 && m) {
+    const int at = (int)wave_atomic_add(q.sharp.count, (unsigned)__popcll(m));
+    if (!resolved) q.sharp.list[at + __popcll(m & ((1ull << lane) - 1ull))] = p0 + t;
+    if (lane == 0)
+      __hip_atomic_store(q.sharp.any, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   if (t == 0) q.done[pb] = 0u;
   __syncthreads();

@@ -225,6 +225,7 @@ template <bool TWO>
 struct TersoffPop {
   static constexpr int NMAX = 4;
   static constexpr int kWaves = 4, kWavesPacked = TWO ? 3 : 4;
+  static constexpr bool kSubset = false;
   static constexpr bool kForcePass = true;
   static constexpr int kFoldValues = 24;
   using Lane = TLane;
@@ -875,6 +876,7 @@ struct TersoffPop {
 template <bool TWO>
 struct TersoffLoop {
   static constexpr int kWaves = 4, kWavesPacked = 4;
+  static constexpr bool kSubset = false;
   static constexpr bool kForcePass = true;
   static constexpr int kFoldValues = 24;
   static constexpr bool kPacked = false;

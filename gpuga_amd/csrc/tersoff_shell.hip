@@ -64,6 +64,7 @@ __device__ __forceinline__ void upto(F&& f)
 template <int M, bool TWO>
 struct TersoffShell {
   static constexpr int kWaves = 2, kWavesPacked = 2;
+  static constexpr bool kSubset = false;
   static constexpr bool kForcePass = true;
   static constexpr int kFoldValues = 24;
   static constexpr bool kPacked = false;
