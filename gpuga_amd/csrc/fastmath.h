@@ -51,15 +51,37 @@ __device__ __forceinline__ float ftanh(float x)
   return 1.0f - 2.0f * frcp(fexp2(x * (2.0f * LOG2E)) + 1.0f);
 }
 
-// tanh x = sgn(x) (1 - 2 r) and 1 - tanh^2 x = 4 r (1 - r) with
-// r = 1 / (exp(2 |x|) + 1): tanh about 1e-7 absolute, the derivative (r is at
-// most a half) without a difference of nearly equal numbers.
+// tanh x = sgn(x) (1 - e) / (1 + e) and s = (1 - tanh^2 x) / 4 = e / (1 + e)^2
+// with e = exp(-2 |x|): about 1e-7 absolute, the derivative without a
+// difference of nearly equal numbers.  (A quarter of it: callers multiply once,
+// at the end.)
 __device__ __forceinline__ void tanh_sech2(float x, float& t, float& s)
+{
+  const float e = fexp2(-2.0f * LOG2E * __builtin_fabsf(x));
+  const float r = frcp(1.0f + e);
+  t = __builtin_copysignf((1.0f - e) * r, x);
+  s = e * r * r;
+}
+
+// tanh x = sgn(x) (1 - 2 r) and s = (1 - tanh^2 x) / 4 = r (1 - r) with
+// r = 1 / (exp(2 |x|) + 1): the error of ftanh, the derivative as above.
+__device__ __forceinline__ void ftanh_sech2(float x, float& t, float& s)
 {
   const float r = frcp(fexp2(2.0f * LOG2E * __builtin_fabsf(x)) + 1.0f);
   t = __builtin_copysignf(fmaf(-2.0f, r, 1.0f), x);
-  const float r4 = 4.0f * r;
-  s = fmaf(-r4, r, r4);
+  s = fmaf(-r, r, r);
+}
+
+// The same with tanh to about 1e-7 of its value: below 1/2 as x + x^3 p(x^2)
+// (p: least-maximum fit of degree 3, 1.5e-8 of tanh x).
+__device__ __forceinline__ void tanh_sech2_relative(float x, float& t, float& s)
+{
+  ftanh_sech2(x, t, s);
+  const float y = x * x;
+  float p = fmaf(0.01724139f, y, -0.05304545f);
+  p = fmaf(p, y, 0.13325878f);
+  p = fmaf(p, y, -0.33333144f);
+  t = __builtin_fabsf(x) < 0.5f ? fmaf(x * y, p, x) : t;
 }
 
 // sin(pi t) and cos(pi t) for 0 <= t <= 1

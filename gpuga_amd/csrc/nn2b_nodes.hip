@@ -28,7 +28,7 @@
 // (the magnitudes two instructions a neuron, the coefficients a chain of
 // exchanges; through LDS instead of DPP 0.5 us more).  BF16 costs what FP32
 // does here: its splits take the VALU as long as FP32 products the matrix unit.
-// (Its tanh as FP32's: 1 - t t loses the derivative of a saturated neuron, and
+// (Its tanh's derivative not as 1 - t t, which loses it for saturated neurons:
 // the check then takes the rounding of 1 in 100 networks of 6 neurons for
 // sharpness.)
 #include "quadform.h"
@@ -167,12 +167,16 @@ __global__ void __launch_bounds__(WAVES * WAVE) nn2b_nodes(PopCtl ctl, int n, in
       if (!((el.y >> code) & 1)) continue;
       const float2 pairs = ldu(tab.pairs, code * E + el.x);
       f32x16 z[NB] = {}, zd[NB] = {};
+      auto tanh_s = [](float x, float& t, float& s) {
+        if constexpr (BF16) ftanh_sech2(x, t, s); // (the operands' 16 bits set the error)
+        else tanh_sech2(x, t, s);
+      };
       auto layer1 = [&](int s, float& x, float& y) {
         const float4 l = l1[m_of(s)];
         // the species-pair input as a shift of the bias
         const float bias = species ? l.y - l.z * (float)code : l.y;
         float sg;
-        tanh_sech2(l.x * d - bias, x, sg);
+        tanh_s(l.x * d - bias, x, sg);
         y = sg * l.x;
       };
       if constexpr (BF16) {
@@ -209,7 +213,7 @@ __global__ void __launch_bounds__(WAVES * WAVE) nn2b_nodes(PopCtl ctl, int n, in
         for (int r = 0; r < 16; ++r) {
           const float2 l = l2[32 * b + 8 * (r >> 2) + 4 * half + (r & 3)];
           float x, sg;
-          tanh_sech2(z[b][r] - l.x, x, sg);
+          tanh_s(z[b][r] - l.x, x, sg);
           u = fmaf(l.y, x, u);
           g = fmaf(l.y * sg, zd[b][r], g);
           um = fmaf(__builtin_fabsf(l.y), __builtin_fabsf(x), um);
@@ -221,6 +225,9 @@ __global__ void __launch_bounds__(WAVES * WAVE) nn2b_nodes(PopCtl ctl, int n, in
       if (!half) {
         mine -= bias2;
         mag += __builtin_fabsf(bias2);
+      } else { // (tanh_s: two quarters)
+        mine *= 16.0f;
+        mag *= 16.0f;
       }
       // one of the last coefficients in each lane
       const float c =

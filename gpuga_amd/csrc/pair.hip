@@ -338,9 +338,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // Bound by the hidden layer's MFMAs and the 2 n tanh per bond.  One thread
 // per atom with both layers in scratch memory (two scratch accesses an FMA,
 // 450 waves for 1024 SIMDs) took 4617 us on 28 800 atoms with 42 neighbours
-// and n = 32; this form 103 us.  Eight atoms a wave leave 5% of the tiles'
-// bonds empty there and give 3600 waves; with species, the code t_i + t_j
-// shifts the first layer's bias.
+// and n = 32; this form 118 us (106 us with a tanh of 1e-7 absolute and the
+// bias among the products' sum, which left networks with weights of 0.02 five
+// to seventeen times the error of the scalar form).  Eight atoms a wave leave
+// 5% of the tiles' bonds empty there and give 3600 waves; with species, the
+// code t_i + t_j shifts the first layer's bias.
 constexpr int NN2B_ATOMS = 8;
 
 template <int KS, int NB>
@@ -397,19 +399,14 @@ __global__ void __launch_bounds__(WAVE) nn2b_plain(DevSet s, int n, int species,
     const float4 rij = s.bond[k];
     const float d = rij.w;
     const float code = species ? (float)s.ptype[k] : 0.0f;
-    f32x16 z[NB], zd[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        z[b][r] = -c1[b][r];
-        zd[b][r] = 0.0f;
-      }
+    // (the bias is subtracted after the products: summed with them, it loses
+    // digits of small ones)
+    f32x16 z[NB] = {}, zd[NB] = {};
 #pragma unroll
     for (int q = 0; q < KS; ++q) {
       // the species-pair input as a shift of the bias
       float x, sg;
-      tanh_sech2(fmaf(p0[q], d, fmaf(ps[q], code, -pb[q])), x, sg);
+      tanh_sech2_relative(fmaf(p0[q], d, fmaf(ps[q], code, -pb[q])), x, sg);
       const float y = sg * p0[q];
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
@@ -423,12 +420,12 @@ __global__ void __launch_bounds__(WAVE) nn2b_plain(DevSet s, int n, int species,
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         float x, sg;
-        tanh_sech2(z[b][r], x, sg);
+        tanh_sech2_relative(z[b][r] - c1[b][r], x, sg);
         p = fmaf(c2[b][r], x, p);
         g = fmaf(c2[b][r] * sg, zd[b][r], g);
       }
     p = (p + __shfl_xor(p, 32)) - bias2;
-    g += __shfl_xor(g, 32);
+    g = 16.0f * (g + __shfl_xor(g, 32)); // (two quarters)
     float fc = 0.0f, fcp = 0.0f;
     if (d < NN2B_R1) {
       fc = 1.0f;
