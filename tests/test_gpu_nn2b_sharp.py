@@ -116,18 +116,21 @@ def test_sharp_networks_match_oracle(n, grid, kind, bf16, P, species):
 
 @pytest.mark.parametrize("P", [30, 150])
 def test_device_generations_with_sharp_networks_equal_the_host_loop(P):
-    """A run that starts without the pair loop's tables, and one that has them."""
+    """A run that starts without the pair loop's tables and meets individuals that
+    need them, and one that has them."""
     import gpuga_amd as G
     print_case("sharp networks, device GA", P)
     d = _dimers(60, 25, 20, 12)
-    d["pmin"], d["pmax"] = 2 * d["pmin"], 2 * d["pmax"]
 
     def ga():
         return G.GA(P, P // 2 + P // 2 % 2, len(d["pmin"]), maximum_generation=40, seed=5)
 
-    with G.Fitness(arrays=d, nn2b_bf16=0, chunk_cost=200) as fit:
+    with G.Fitness(arrays=d, nn2b_bf16=0, nn2b_grid=256, chunk_cost=200) as fit:
         first, second, host = ga(), ga(), ga()
+        before = fit.device_bytes()
         got, _ = fit.run_ga(first, 0, 6)
+        tables = 3 * 256 * 64 * 4 * ((P + 63) // 64)  # of the tabulation
+        assert fit.device_bytes() - before >= tables
         got2, _ = fit.run_ga(second, 0, 6)
         best = []
         for k in range(6):
