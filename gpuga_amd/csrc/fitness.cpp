@@ -1887,7 +1887,19 @@ LaunchShape Fitness::launch_shape(int P)
   if (opt_.chunk_cost > 0) return option_shape();
   auto t = tuned_.find(P);
   if (t == tuned_.end()) {
-    autotune(P);
+    if (quad_.on && spec_.nn2b()) {
+      // The loop serves parts of the population, of any size, for which a full
+      // launch's timing is no guide; nor is it worth 95 ms of the first call.
+      // Items of this cost, against 100 and 700: all of 256 individuals on
+      // 57 600 wurtzite atoms 352 (386, 403) us a call, 3 of them 285 (310, 417),
+      // 70 individuals 223 (251, 345); 100 on 10 800 atoms with species 197 (200,
+      // 248).
+      LaunchShape sh = option_shape();
+      sh.chunk_cost = 300;
+      tuned_[P] = sh;
+    } else {
+      tune(P);
+    }
     t = tuned_.find(P);
   }
   return t->second;
@@ -1907,6 +1919,18 @@ void Fitness::plan_shape(int P, int& chunk_cost, int& queues, int& blocks_per_cu
 
 int Fitness::autotune(int P)
 {
+  if (!quad_.on) return tune(P);
+  // Of a set with quadratic forms only the calls that they do not take run the
+  // population kernel, and its tables may not be there: the first such call
+  // chooses its shape (ensure_items).  With the built-in size, too coarse for
+  // rigid ion, calls of 200 individuals on 48 000 oxide atoms with a gene
+  // outside [0, 1] took 592 us; 361 us tuned.
+  const auto t = tuned_.find(P);
+  return t == tuned_.end() ? heuristic_chunk_cost(P) : t->second.chunk_cost;
+}
+
+int Fitness::tune(int P)
+{
   // Candidate work-item sizes: the whole-configuration cost spread over
   // 1/2 .. 1/32 of the resident waves, and the largest configuration's cost
   // halved step by step (small sets, where latency rather than balance
@@ -1916,14 +1940,6 @@ int Fitness::autotune(int P)
   // lane block qualifies, packing it or not.  Each choice is kept only if
   // its launch is faster.
   const bool tersoff = spec_.type == POT_TERSOFF1 || spec_.type == POT_TERSOFF2;
-  if (quad_.on) {
-    // nothing to tune: the population kernel only serves a trace, or genes
-    // outside [0, 1]
-    LaunchShape sh = option_shape();
-    sh.chunk_cost = heuristic_chunk_cost(P);
-    tuned_[P] = sh;
-    return sh.chunk_cost;
-  }
   const std::vector<int>& pnn = tersoff ? population_neighbors().NN : nl_.NN;
   long long total = 0, maxcfg = 0;
   for (int c = 0; c < ts_.Nc; ++c) {

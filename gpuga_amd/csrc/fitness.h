@@ -250,6 +250,7 @@ private:
   bool run_generations(PopPlan& pl, GA& ga, int first_generation, int generations, bool quad,
                        float* best, float* elite);
   void launch_quad_values(PopPlan& pl, const PopCtl& ctl, int first, int count, hipStream_t st);
+  int tune(int P);
   double time_plan(int P, const LaunchShape& sh, int reps, int* occ = nullptr);
   // after a launch whose status word is set: clear the plan's counters and
   // results, then fail

@@ -159,8 +159,8 @@ int gpuga_inspect_geometry(const char* input_dir, int* sizes3, float* bond, floa
 /* Launch shape chosen by timing candidates for population P (work-item
  * size, then the queue count, resident workgroups per CU and lane packing
  * that the options leave at 0 / on); returns the work-item size.  (A pair
- * potential's quadratic forms have no shape to choose: the built-in size, for
- * the calls that take the population kernel.)  No counterpart in the
+ * potential's quadratic forms have no shape to choose: the built-in size, until
+ * the first call that needs the population kernel has tuned it.)  No counterpart in the
  * reference (its launch shape is fixed). */
 int gpuga_fitness_autotune(gpuga_fitness* h, int P, int* chunk_cost);
 /* The shape the population launch for P runs with (tuned first when the
