@@ -39,14 +39,13 @@ struct DevSet {
   const float4* bond;     // [B] r_ij.x, r_ij.y, r_ij.z, |r_ij|
   const int* tri0;        // [N] first triplet of atom i (Tersoff only)
   const float4* tri;      // [T] cos theta, d cos / d r_ij (Tersoff only)
-  // Tersoff atom records, one per atom at a fixed stride of 1 + M + M*M +
-  // M/2 float4 (M = neighbour bound of the set): header {nn, unlike-type bit
+  // Tersoff atom records of sets with at most M = 4 neighbours, one per atom at
+  // a fixed stride of 1 + M + M*M + M/2 float4: header {nn, unlike-type bit
   // mask, first bond, longest bond's length}, then M bonds (x, y, z, d),
   // then the M x M triplets (cos theta_jik, d cos / d r_ij), then M
   // reverse-bond indices (int) and M inverse distances 1/d.  Every load of
   // an atom is independent of the others, so they issue together.
   const float4* rec;
-  int rec_nmax;
   // Moment records of the energy configurations' atoms with four bonds (the
   // Tersoff population kernel; atom N_force + i at i kMomWords floats).  With
   // c'_uv = cos theta_uv - kMomCos and G_uv = r_u (x) d cos / d r_u + r_v (x)

@@ -170,15 +170,94 @@ Fitness::~Fitness()
 }
 
 void Fitness::device_geometry(std::vector<float4>& bond, std::vector<float4>& tri,
-                              std::vector<float4>& rec) const
+                              std::vector<float4>& rec)
 {
+  hipStream_t st = stream_;
+  // with 5 to 16 neighbours the population kernel has records of its own, and
+  // these are built to be looked at
+  const bool tersoff = spec_.type == POT_TERSOFF1 || spec_.type == POT_TERSOFF2;
+  const int M = tersoff ? record_slots(population_neighbors().max_nn) : 0;
+  DeviceBuffer<float4> built;
+  if (shell_M_ > 0 && M > 0) {
+    built.resize((size_t)ts_.N * record_floats4(M));
+    const DeviceNeighbors pd = build_population_tables();
+    build_records_device(ts_.N, M, pd, loop_.ptype, loop_.bond, loop_.tri, built.get(), st);
+    GPUGA_HIP(hipStreamSynchronize(st));
+    drop_population_tables();
+  }
+  const DeviceBuffer<float4>& r = built.size() > 0 ? built : ds_.rec;
   bond.resize(ds_.bond.size());
   tri.resize(ds_.tri.size());
-  rec.resize(ds_.rec.size());
-  ds_.bond.download(bond.data(), bond.size(), stream_);
-  ds_.tri.download(tri.data(), tri.size(), stream_);
-  ds_.rec.download(rec.data(), rec.size(), stream_);
-  GPUGA_HIP(hipStreamSynchronize(stream_));
+  rec.resize(r.size());
+  ds_.bond.download(bond.data(), bond.size(), st);
+  ds_.tri.download(tri.data(), tri.size(), st);
+  r.download(rec.data(), rec.size(), st);
+  GPUGA_HIP(hipStreamSynchronize(st));
+}
+
+DeviceNeighbors Fitness::device_neighbors() const
+{
+  DeviceNeighbors dn;
+  dn.NN = ds_.nn.get();
+  dn.start = ds_.bond0.get();
+  dn.NL = ds_.nl.get();
+  dn.rev = ds_.rev.get();
+  dn.tri0 = ds_.tri0.get();
+  dn.total = nl_.total;
+  return dn;
+}
+
+// Tables of the list the Tersoff population kernel reads, in loop_: the full
+// ones, or the pruned list's (geometry bit-identical to the full tables' entries
+// for the same bonds).
+DeviceNeighbors Fitness::build_population_tables()
+{
+  hipStream_t st = stream_;
+  const NeighborList& pn = population_neighbors();
+  DeviceNeighbors pd = device_neighbors();
+  loop_.ptype = ds_.ptype.get();
+  loop_.bond = ds_.bond.get();
+  loop_.tri = ds_.tri.get();
+  if (pruned_) {
+    long long tri_total = 0;
+    const std::vector<int> t0 = triplet_offsets(pn, &tri_total);
+    ds_.p_nn.upload(pn.NN, st);
+    ds_.p_b0.upload(pn.start, st);
+    ds_.p_nl.upload(pn.NL.empty() ? std::vector<int>{0} : pn.NL, st);
+    ds_.p_rev.upload(pn.rev.empty() ? std::vector<int>{0} : pn.rev, st);
+    const std::vector<int> pt = bond_types(ts_, pn, true);
+    ds_.p_ptype.upload(pt.empty() ? std::vector<int>{0} : pt, st);
+    ds_.p_tri0.upload(t0, st);
+    ds_.p_bond.resize(std::max(pn.total, 1));
+    ds_.p_tri.resize((size_t)std::max<long long>(tri_total, 1));
+    pd.NN = ds_.p_nn.get();
+    pd.start = ds_.p_b0.get();
+    pd.NL = ds_.p_nl.get();
+    pd.rev = ds_.p_rev.get();
+    pd.tri0 = ds_.p_tri0.get();
+    pd.total = pn.total;
+    build_geometry_device(ts_, pd, ds_.p_bond.get(), ds_.p_tri.get(), st);
+    loop_.ptype = ds_.p_ptype.get();
+    loop_.bond = ds_.p_bond.get();
+    loop_.tri = ds_.p_tri.get();
+    // (the host vectors above are read before this scope ends)
+    GPUGA_HIP(hipStreamSynchronize(st));
+  }
+  loop_.nn = pd.NN;
+  loop_.b0 = pd.start;
+  loop_.tri0 = pd.tri0;
+  loop_.rev = pd.rev;
+  loop_.max_nn = pn.max_nn;
+  return pd;
+}
+
+void Fitness::drop_population_tables()
+{
+  for (auto* b : {&ds_.p_nn, &ds_.p_b0, &ds_.p_nl, &ds_.p_rev, &ds_.p_ptype, &ds_.p_tri0})
+    b->resize(0);
+  ds_.p_bond.resize(0);
+  ds_.p_tri.resize(0);
+  loop_ = LoopTab{};
 }
 
 void Fitness::setup()
@@ -220,12 +299,7 @@ void Fitness::setup()
   ds_.nl.upload(nl_.NL.empty() ? std::vector<int>{0} : nl_.NL, st);
   ds_.rev.upload(nl_.rev.empty() ? std::vector<int>{0} : nl_.rev, st);
   ds_.ptype.upload(ptype.empty() ? std::vector<int>{0} : ptype, st);
-  DeviceNeighbors dn;
-  dn.NN = ds_.nn.get();
-  dn.start = ds_.bond0.get();
-  dn.NL = ds_.nl.get();
-  dn.rev = ds_.rev.get();
-  dn.total = nl_.total;
+  DeviceNeighbors dn = device_neighbors();
   if (nl_.total == 0) ds_.bond.upload(std::vector<float4>{make_float4(0, 0, 0, 1)}, st);
   else ds_.bond.resize(nl_.total);
   std::vector<int> tri0;
@@ -254,81 +328,35 @@ void Fitness::setup()
     const NeighborList& pn = population_neighbors();
     const int M = record_slots(pn.max_nn);
     shell_M_ = pn.max_nn > 4 ? tersoff_shell_slots(pn.max_nn) : 0;
-    loop_path_ = M == 0 && shell_M_ == 0;
+    loop_path_ = pn.max_nn > 4 && shell_M_ == 0;
     if (loop_path_ && pn.max_nn > kLoopMaxNeighbors)
       fail(strfmt("the population kernel supports at most %d neighbours per atom within the "
                   "largest R2 (found %d); use the per-individual backend",
                   kLoopMaxNeighbors, pn.max_nn));
-    // tables of the list the population kernel reads: the full ones, or
-    // the pruned list's (geometry bit-identical to the full tables' entries
-    // for the same bonds)
-    DeviceNeighbors pd = dn;
-    const int* pptype = ds_.ptype.get();
-    const float4 *pbond = ds_.bond.get(), *ptri = ds_.tri.get();
-    if (pruned_) {
-      long long ptri_total = 0;
-      const std::vector<int> t0 = triplet_offsets(pn, &ptri_total);
-      ds_.p_nn.upload(pn.NN, st);
-      ds_.p_b0.upload(pn.start, st);
-      ds_.p_nl.upload(pn.NL.empty() ? std::vector<int>{0} : pn.NL, st);
-      ds_.p_rev.upload(pn.rev.empty() ? std::vector<int>{0} : pn.rev, st);
-      const std::vector<int> pt = bond_types(ts_, pn, true);
-      ds_.p_ptype.upload(pt.empty() ? std::vector<int>{0} : pt, st);
-      ds_.p_tri0.upload(t0, st);
-      ds_.p_bond.resize(std::max(pn.total, 1));
-      ds_.p_tri.resize((size_t)std::max<long long>(ptri_total, 1));
-      pd.NN = ds_.p_nn.get();
-      pd.start = ds_.p_b0.get();
-      pd.NL = ds_.p_nl.get();
-      pd.rev = ds_.p_rev.get();
-      pd.tri0 = ds_.p_tri0.get();
-      pd.total = pn.total;
-      build_geometry_device(ts_, pd, ds_.p_bond.get(), ds_.p_tri.get(), st);
-      pptype = ds_.p_ptype.get();
-      pbond = ds_.p_bond.get();
-      ptri = ds_.p_tri.get();
-      // (the host vectors above are read before this scope ends)
-      GPUGA_HIP(hipStreamSynchronize(st));
-    }
-    loop_.nn = pd.NN;
-    loop_.b0 = pd.start;
-    loop_.tri0 = pd.tri0;
-    loop_.rev = pd.rev;
-    loop_.ptype = pptype;
-    loop_.bond = pbond;
-    loop_.tri = ptri;
-    loop_.max_nn = pn.max_nn;
+    const DeviceNeighbors pd = build_population_tables();
     if (shell_M_ > 0) {
       ds_.shell_rec.resize(tersoff_shell_floats4(ts_.N, shell_M_));
       build_shell_records(ts_.N, shell_M_, loop_, ds_.shell_rec.get(), st);
     }
-    if (M > 0) {
-      const size_t RS = 1 + M + (size_t)M * M + M / 2;
-      ds_.rec.resize((size_t)ts_.N * RS);
-      build_records_device(ts_.N, M, pd, pptype, pbond, ptri, ds_.rec.get(), st);
-      ds_.view.rec_nmax = M;
-      if (M == 4) {
-        // An atom's moment record serves a wave when its bonds are shorter than
-        // every lane's R1, whose smallest is near the parameter's lower bound.
-        // Kept where nine atoms in ten pass at that bound: with half of them,
-        // 120 200 atoms and 200 individuals, a call took 335 us with the
-        // records and 318 us without (all: 280 and 297 us).
-        const int n = ts_.N - ts_.N_force;
-        const float r1 = std::min(spec_.pmin[spec_.V - 2], spec_.pmax[spec_.V - 2]);
-        ds_.mom.resize((size_t)std::max(n, 1) * kMomWords);
-        const int inside =
-          build_moments_device(ts_.N_force, ts_.N, pd, pptype, pbond, r1, ds_.mom.get(), st);
-        if (10LL * inside < 9LL * n || n == 0) ds_.mom.resize(0);
-      }
+    if (pn.max_nn <= 4) {
+      ds_.rec.resize((size_t)ts_.N * record_floats4(M));
+      build_records_device(ts_.N, M, pd, loop_.ptype, loop_.bond, loop_.tri, ds_.rec.get(), st);
+      // An atom's moment record serves a wave when its bonds are shorter than
+      // every lane's R1, whose smallest is near the parameter's lower bound.
+      // Kept where nine atoms in ten pass at that bound: with half of them,
+      // 120 200 atoms and 200 individuals, a call took 335 us with the records
+      // and 318 us without (all: 280 and 297 us).
+      const int n = ts_.N - ts_.N_force;
+      const float r1 = std::min(spec_.pmin[spec_.V - 2], spec_.pmax[spec_.V - 2]);
+      ds_.mom.resize((size_t)std::max(n, 1) * kMomWords);
+      const int inside =
+        build_moments_device(ts_.N_force, ts_.N, pd, loop_.ptype, loop_.bond, r1, ds_.mom.get(), st);
+      if (10LL * inside < 9LL * n || n == 0) ds_.mom.resize(0);
     }
     if (!loop_path_) {
       GPUGA_HIP(hipStreamSynchronize(st));
       // the records hold everything the kernel reads of the pruned list
-      for (auto* b : {&ds_.p_nn, &ds_.p_b0, &ds_.p_nl, &ds_.p_rev, &ds_.p_ptype, &ds_.p_tri0})
-        b->resize(0);
-      ds_.p_bond.resize(0);
-      ds_.p_tri.resize(0);
-      loop_ = LoopTab{};
+      drop_population_tables();
     }
     ds_.view.bond_force =
       ts_.N_force > 0 ? pn.start[ts_.N_force - 1] + pn.NN[ts_.N_force - 1] : 0;

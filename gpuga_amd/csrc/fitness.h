@@ -201,7 +201,7 @@ public:
   const NeighborList& population_neighbors() const { return pruned_ ? pnl_ : nl_; }
   // The device geometry tables (bond, triplet, atom records), copied back.
   void device_geometry(std::vector<float4>& bond, std::vector<float4>& tri,
-                       std::vector<float4>& rec) const;
+                       std::vector<float4>& rec);
   hipStream_t stream() const { return stream_; }
   size_t device_bytes() const;
   size_t plan_bytes(int P) const;
@@ -218,6 +218,9 @@ public:
 
 private:
   void setup();
+  DeviceNeighbors device_neighbors() const; // the full list's tables
+  DeviceNeighbors build_population_tables();
+  void drop_population_tables();
   // Quadratic forms of a pair potential's set, when the rule of
   // quad_elements() takes it.
   void setup_quad();

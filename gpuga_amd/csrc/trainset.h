@@ -102,7 +102,9 @@ std::vector<int> bond_types(const TrainSet& ts, const NeighborList& nl, bool thr
 // holds 1 + M + M*M + M/2 float4: header (nn, species-pair bit mask, first
 // bond as ints, the longest bond's length as a float), M bonds, M x M
 // triplets (s, t), M reverse-bond ints and M inverse distances, zero-padded.
+// (The kernel reads them up to M = 4; larger ones are built to be looked at.)
 int record_slots(int max_nn);
+constexpr size_t record_floats4(int M) { return 1 + M + (size_t)M * M + M / 2; }
 // Largest outer cut-off radius R2 any individual of a minimal-Tersoff
 // potential can have: the last parameter's pmin + (pmax - pmin) g at g = 1,
 // in the float arithmetic of the denormalisation (monotonic in g, so every
