@@ -759,45 +759,43 @@ void Fitness::setup_quad()
   // accumulated over the chunks.  Chunks and the split of a chunk's rows over
   // waves do not depend on the columns, so a column's sums do not depend on
   // which others the form has.
-  constexpr int kConfigs = 512, kAtoms = 2048, kSplits = 16;
   DeviceBuffer<double> R, part;
-  auto finish = [&](int f, const double* p) {
+  size_t most = 0;
+  for (int f = 0; f < 3; ++f) {
     quad_.nb[f] = nb[f];
     quad_.q[f].resize((size_t)quad_tiles(nb[f]) * QB * QB);
     quad_.vblk[f].upload(vblk[f], st);
-    launch_quad_finish(p, nb[f], kSplits, quad_.q[f].get(), st);
+    most = std::max(most, quad_part_size(nb[f]));
+  }
+  part.resize(most);
+  auto gram = [&](int f, const double* r, int n, bool first) {
+    launch_quad_gram(r, n, nb[f], first, part.get(), quad_.q[f].get(), st);
   };
-  auto part_size = [&](int f) { return (size_t)kSplits * quad_tiles(nb[f]) * QB * QB; };
-  auto pad4 = [](int n) { return (std::max(n, 1) + 3) / 4 * 4; };
   { // energy and virial rows
-    const int ne = ts_.Nc - ts_.Nc_force, step = std::min(kConfigs, pad4(ne));
+    const int ne = ts_.Nc - ts_.Nc_force, step = quad_step(kQuadConfigs, ne);
     const size_t D0 = rows.D(0), D1 = rows.D(1);
     R.resize(step * (D0 + 6 * D1));
-    part.resize(part_size(0) + part_size(1));
-    double *re = R.get(), *rw = re + step * D0, *pw = part.get() + part_size(0);
+    double *re = R.get(), *rw = re + step * D0;
     for (int c0 = 0; c0 < std::max(ne, 1); c0 += step) {
-      const int n = std::min(step, ne - c0), n4 = pad4(n), c = ts_.Nc_force + c0;
+      const int n = std::min(step, ne - c0), n4 = quad_step(step, n), c = ts_.Nc_force + c0;
       R.zero(st);
       if (n > 0) launch_quad_energy_rows(ds_.view, rows, c, c + n, re, rw, st);
-      launch_quad_gram(re, n4, nb[0], kSplits, c0 == 0, part.get(), st);
-      launch_quad_gram(rw, 6 * n4, nb[1], kSplits, c0 == 0, pw, st);
+      gram(0, re, n4, c0 == 0);
+      gram(1, rw, 6 * n4, c0 == 0);
     }
-    finish(0, part.get());
-    finish(1, pw);
   }
   GPUGA_HIP(hipStreamSynchronize(st));
   { // force rows
-    const int na = ts_.N_force, step = std::min(kAtoms, pad4(na));
+    const int na = ts_.N_force, step = quad_step(kQuadAtoms, na);
     R.resize((size_t)step * 3 * rows.D(2));
-    part.resize(part_size(2));
     for (int i0 = 0; i0 < std::max(na, 1); i0 += step) {
       const int n = std::min(step, na - i0);
       R.zero(st);
       if (n > 0) launch_quad_force_rows(ds_.view, rows, i0, i0 + n, R.get(), st);
-      launch_quad_gram(R.get(), 3 * pad4(n), nb[2], kSplits, i0 == 0, part.get(), st);
+      gram(2, R.get(), 3 * quad_step(step, n), i0 == 0);
     }
-    finish(2, part.get());
   }
+  for (int f = 0; f < 3; ++f) launch_quad_finish(nb[f], quad_.q[f].get(), st);
   std::vector<int2> unit;
   for (int I = std::max({nb[0], nb[1], nb[2]}) - 1; I >= 0; --I)
     for (int f = 0; f < 3; ++f)
@@ -1807,42 +1805,76 @@ int Fitness::heuristic_chunk_cost(int P) const
 size_t Fitness::estimate_bytes(const PotentialSpec& s, const TrainSet& ts, int P,
                                const FitnessOptions& opt)
 {
-  // neighbour counts on the device (a counting pass of the list build)
+  // neighbour counts on the device (counting passes of the list build): of the
+  // list, and of the bonds that the Tersoff population kernel reads
+  const bool tersoff = s.type == POT_TERSOFF1 || s.type == POT_TERSOFF2;
+  const float reach = std::max(0.0f, std::min(s.cutoff, tersoff_reach(s)));
   hipStream_t st = nullptr;
   GPUGA_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-  std::vector<int> nn;
+  std::vector<int> nn, pnn;
   try {
     nn = count_neighbors_device(ts, s.cutoff, st);
+    if (tersoff && reach < s.cutoff) pnn = count_neighbors_device(ts, reach, st);
   } catch (...) {
     (void)hipStreamDestroy(st);
     throw;
   }
   GPUGA_HIP(hipStreamDestroy(st));
-  long long bonds = 0;
-  size_t tri = 0;
-  for (int i = 0; i < ts.N; ++i) {
-    bonds += nn[i];
-    tri += (size_t)nn[i] * nn[i];
-  }
-  const size_t N = ts.N, Nc = ts.Nc, B = std::max<long long>(bonds, 1);
-  const bool tersoff = s.type == POT_TERSOFF1 || s.type == POT_TERSOFF2;
+  struct Lists {
+    size_t bonds = 0, tri = 0, force_bonds = 0, cost = 0;
+    int most = 0;
+  };
+  auto lists = [&](const std::vector<int>& c) {
+    Lists l;
+    for (int i = 0; i < (int)c.size(); ++i) {
+      l.bonds += c[i];
+      l.tri += (size_t)c[i] * c[i];
+      if (i < ts.N_force) l.force_bonds += c[i];
+      l.cost += atom_cost(s.type, c[i], i < ts.N_force);
+      l.most = std::max(l.most, c[i]);
+    }
+    l.bonds = std::max<size_t>(l.bonds, 1);
+    return l;
+  };
+  const Lists full = lists(nn), used = pnn.empty() ? full : lists(pnn);
+  const size_t N = ts.N, Nc = ts.Nc, B = full.bonds;
   size_t b = N * sizeof(int) * 5 + Nc * sizeof(int) * 2 + B * (3 * sizeof(int) + 16);
-  b += (tersoff ? tri * 16 + B * 4 * 5 : 0) + (s.type == POT_RI ? B * 48 + N * 16 : 0);
-  b += s.nn2b() ? B * 48 + N * 16 : 0;
+  if (tersoff) {
+    b += full.tri * 16 + B * 4 * 5; // triplets, per-individual scratch
+    // the pruned list's tables (dropped after set-up where records are built)
+    if (!pnn.empty()) b += N * 4 * 3 + used.bonds * (3 * sizeof(int) + 16) + used.tri * 16;
+    if (used.most <= 4)
+      b += N * record_floats4(4) * 16 + (N - ts.N_force) * kMomWords * sizeof(float);
+    else if (const int M = tersoff_shell_slots(used.most))
+      b += tersoff_shell_floats4(ts.N, M) * 16;
+  } else {
+    b += B * 48 + N * 16; // the pair loop's tables
+    if (s.type == POT_RI) b += B * 16;
+  }
   b += Nc * 7 * sizeof(float) + N * 3 * sizeof(float);  // references
   b += N * 10 * sizeof(float) + Nc * 3 * sizeof(double); // per-atom outputs
   const size_t K = (P + WAVE - 1) / WAVE;
-  size_t B_force = 0;
-  for (int i = 0; i < ts.N_force; ++i) B_force += nn[i];
-  b += K * 3 * Nc * WAVE * sizeof(double) + 2 * Nc * K * 8 * WAVE * sizeof(double);
-  if (tersoff) b += K * (B_force + ts.N_force) * 3 * WAVE * sizeof(float);
+  // error terms, and partials of the work items: at most 16 a CU beside one per
+  // configuration and lane block, where the options set no other size
+  const size_t items = opt.chunk_cost > 0
+                         ? K * used.cost / opt.chunk_cost
+                         : std::min<size_t>(K * used.cost / 64, 16 * 256);
+  b += K * 3 * Nc * WAVE * sizeof(double) + (Nc * K + items) * 8 * WAVE * sizeof(double);
+  if (tersoff) b += K * (used.force_bonds + ts.N_force) * 3 * WAVE * sizeof(float);
   if (s.nn2b()) b += (size_t)3 * s.pair_codes() * opt.nn2b_grid * K * WAVE * sizeof(float);
-  if (!tersoff) {
-    // quadratic forms: value blocks of the population and the three forms
-    // (rigid ion: at most 8 elements per type)
-    const size_t ce = s.nn2b() ? s.pair_codes() * (size_t)std::max(opt.nn2b_grid, 64) / (2 * QB) : 24;
+  const int points = s.pair_codes() * opt.nn2b_grid;
+  if (s.type == POT_RI || (s.nn2b() && opt.nn2b_grid >= 256 && opt.nn2b_grid <= 2048 && points <= 4096)) {
+    // Quadratic forms, with every element in use (rigid ion: at most 8 a type;
+    // U's columns enter its virials and forces nowhere): value blocks of the
+    // population, the three forms, and while they are built the rows and the
+    // partial tiles.
+    const size_t ce = s.nn2b() ? points / (2 * QB) : 24;
+    const size_t nb[3] = {ce + 1, s.nn2b() ? 2 * ce + 1 : ce + 1, s.nn2b() ? 2 * ce + 1 : ce + 1};
     b += (2 * ce + 1) * QB * sizeof(double) * (size_t)(P + QP);
-    b += 3 * quad_tiles(s.nn2b() ? 2 * ce + 1 : ce + 1) * QB * QB * sizeof(double);
+    for (size_t n : nb) b += quad_tiles((long)n) * QB * QB * sizeof(double);
+    const size_t er = (nb[0] + 6 * nb[1]) * quad_step(kQuadConfigs, ts.Nc - ts.Nc_force);
+    const size_t fr = 3 * nb[2] * quad_step(kQuadAtoms, ts.N_force);
+    b += (std::max(er, fr) * QB + quad_part_size((long)nb[1])) * sizeof(double);
   }
   b += (size_t)P * s.V * sizeof(float) + (size_t)P * 4 * sizeof(double);
   return b;

@@ -141,12 +141,26 @@ void launch_quad_energy_rows(const DevSet& s, const QuadRows& q, int c0, int c1,
                              double* rw, hipStream_t st);
 void launch_quad_force_rows(const DevSet& s, const QuadRows& q, int i0, int i1, double* rf,
                             hipStream_t st);
-// part[splits][tiles][QB * QB] (+)= R^T R of R [rows][nb * QB]; rows a
-// multiple of 4
-void launch_quad_gram(const double* R, int rows, int nb, int splits, bool first, double* part,
+// q[tiles][QB * QB] (+)= R^T R of R [rows][nb * QB]; rows a multiple of 4.
+// The rows are split over waves whose partial tiles, of kQuadGroup tiles at a
+// time, meet in part (quad_part_size).
+constexpr int kQuadSplits = 16, kQuadGroup = 512;
+constexpr size_t quad_part_size(long nb)
+{
+  const long t = quad_tiles(nb);
+  return (size_t)(t < kQuadGroup ? t : kQuadGroup) * kQuadSplits * QB * QB;
+}
+void launch_quad_gram(const double* R, int rows, int nb, bool first, double* part, double* q,
                       hipStream_t st);
-// Q's tiles in nodal values from the splits' partial sums
-void launch_quad_finish(const double* part, int nb, int splits, double* q, hipStream_t st);
+// Q's tiles, in place, from Chebyshev coefficients to nodal values
+void launch_quad_finish(int nb, double* q, hipStream_t st);
+// configurations and force atoms whose rows are taken at a time
+constexpr int kQuadConfigs = 512, kQuadAtoms = 2048;
+constexpr int quad_step(int most, int n) // (rows come in fours)
+{
+  const int n4 = n < 1 ? 4 : (n + 3) / 4 * 4;
+  return n4 < most ? n4 : most;
+}
 
 void launch_ri_values(const PopCtl& ctl, const NodeTable& t, hipStream_t st);
 // workgroups an individual (parts of its check's sums)

@@ -289,25 +289,18 @@ __device__ __forceinline__ void tile_of(int tile, int& I, int& J)
 // r + l / 16 of either operand (R is row-major: coalesced), and the results'
 // rows 4 x + l / 16, column l % 16.
 __global__ void __launch_bounds__(256) quad_gram(const double* __restrict__ R, int rows, int nb,
-                                                 int splits, int first, double* __restrict__ part)
+                                                 int tile0, double* __restrict__ part)
 {
+  constexpr int splits = kQuadSplits;
   const int lane = __lane_id(), split = blockIdx.y * 4 + wave_first((int)(threadIdx.x / WAVE));
   if (split >= splits) return;
   int I, J;
-  tile_of(blockIdx.x, I, J);
+  tile_of(tile0 + blockIdx.x, I, J);
   const long D = (long)nb * QB;
   const int quads = rows / 4;
   const int q0 = (int)((long)quads * split / splits), q1 = (int)((long)quads * (split + 1) / splits);
   double* out = part + ((long)split * gridDim.x + blockIdx.x) * QB * QB;
-  f64x4 c[2][2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int v = 0; v < 2; ++v)
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-        c[u][v][x] =
-          first ? 0.0 : out[(16 * u + 4 * x + lane / 16) * QB + 16 * v + lane % 16];
+  f64x4 c[2][2] = {};
   const double* p = R + (4L * q0 + lane / 16) * D + lane % 16;
 #pragma unroll 4
   for (int r = q0; r < q1; ++r, p += 4 * D) {
@@ -326,12 +319,23 @@ __global__ void __launch_bounds__(256) quad_gram(const double* __restrict__ R, i
         out[(16 * u + 4 * x + lane / 16) * QB + 16 * v + lane % 16] = c[u][v][x];
 }
 
-// The splits' partial tiles summed in order and transformed to nodal values:
-// coefficient k of an element is sum_m C[k][m] f(x_m) with C[k][m] =
+// The splits' partial tiles, in order, into (first) or onto the sums.
+__global__ void __launch_bounds__(256) quad_fold(const double* __restrict__ part, int first,
+                                                 double* __restrict__ q)
+{
+  for (int x = threadIdx.x; x < QB * QB; x += 256) {
+    double* o = q + (long)blockIdx.x * QB * QB + x;
+    double sum = first ? 0.0 : *o;
+    for (int sp = 0; sp < kQuadSplits; ++sp)
+      sum += part[((long)sp * gridDim.x + blockIdx.x) * QB * QB + x];
+    *o = sum;
+  }
+}
+
+// The tiles transformed to nodal values: coefficient k of an element is sum_m C[k][m] f(x_m) with C[k][m] =
 // (2 / QB) cos(k theta_m) (half of it for k = 0), so Q <- C^T Q C, block by
 // block; the linear block stays.  A tile off the diagonal counts twice.
-__global__ void __launch_bounds__(256) quad_finish(const double* __restrict__ part, int nb,
-                                                   int splits, double* __restrict__ q)
+__global__ void __launch_bounds__(256) quad_finish(double* __restrict__ q)
 {
   __shared__ double T[QB][QB + 1], C[QB][QB + 1];
   int I, J;
@@ -340,10 +344,7 @@ __global__ void __launch_bounds__(256) quad_finish(const double* __restrict__ pa
   for (int x = t; x < QB * QB; x += 256) {
     const int k = x / QB, m = x % QB;
     C[k][m] = (k == 0 ? 1.0 : 2.0) / QB * cos(k * (PI_D * (m + 0.5) / QB));
-    double sum = 0.0;
-    for (int sp = 0; sp < splits; ++sp)
-      sum += part[((long)sp * gridDim.x + blockIdx.x) * QB * QB + x];
-    T[k][m] = sum;
+    T[k][m] = q[(long)blockIdx.x * QB * QB + x];
   }
   __syncthreads();
   double o[4];
@@ -627,18 +628,23 @@ void launch_quad_force_rows(const DevSet& s, const QuadRows& q, int i0, int i1, 
   GPUGA_HIP(hipGetLastError());
 }
 
-void launch_quad_gram(const double* R, int rows, int nb, int splits, bool first, double* part,
+void launch_quad_gram(const double* R, int rows, int nb, bool first, double* part, double* q,
                       hipStream_t st)
 {
   if (rows % 4 != 0) fail("internal: rows of a Gram matrix in fours");
-  const dim3 grid((unsigned)quad_tiles(nb), (splits + 3) / 4);
-  quad_gram<<<grid, 256, 0, st>>>(R, rows, nb, splits, first ? 1 : 0, part);
-  GPUGA_HIP(hipGetLastError());
+  const long tiles = quad_tiles(nb);
+  for (long t = 0; t < tiles; t += kQuadGroup) {
+    const unsigned n = (unsigned)std::min<long>(kQuadGroup, tiles - t);
+    quad_gram<<<dim3(n, (kQuadSplits + 3) / 4), 256, 0, st>>>(R, rows, nb, (int)t, part);
+    GPUGA_HIP(hipGetLastError());
+    quad_fold<<<n, 256, 0, st>>>(part, first ? 1 : 0, q + t * QB * QB);
+    GPUGA_HIP(hipGetLastError());
+  }
 }
 
-void launch_quad_finish(const double* part, int nb, int splits, double* q, hipStream_t st)
+void launch_quad_finish(int nb, double* q, hipStream_t st)
 {
-  quad_finish<<<(unsigned)quad_tiles(nb), 256, 0, st>>>(part, nb, splits, q);
+  quad_finish<<<(unsigned)quad_tiles(nb), 256, 0, st>>>(q);
   GPUGA_HIP(hipGetLastError());
 }
 
