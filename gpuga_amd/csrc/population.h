@@ -164,6 +164,11 @@ __device__ __forceinline__ int lane_here()
   return l;
 }
 
+// A word of a record, whatever its type: stores of records word by word through
+// it stay in order with the reads of their floats and integers (through int the
+// compiler may move them past reads of another type).
+typedef int record_word __attribute__((may_alias));
+
 // x of lane `lane ^ m`
 __device__ __forceinline__ float wave_xor(float x, int m, int lane)
 {

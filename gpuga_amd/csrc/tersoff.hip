@@ -430,7 +430,7 @@ struct TersoffPop {
         if (FORCE) {
           // f_ij goes to the slot of the reverse bond, where atom j reads it
           // back as f_ji; F_i's own part sum_j f_ij stays in registers
-          const int rb = ldr<U, LR>(reinterpret_cast<const int*>(R + REV), u);
+          const int rb = ldr<U, LR>(reinterpret_cast<const record_word*>(R + REV), u);
           float* o = fblk + (size_t)rb * 3 * WAVE + lane;
           cstore(o, fx);
           cstore(o + WAVE, fy);
@@ -627,7 +627,7 @@ struct TersoffPop {
   }
   __device__ static void spread_store(float4* buf, const Spread& v, int l)
   {
-    int* w = reinterpret_cast<int*>(buf);
+    record_word* w = reinterpret_cast<record_word*>(buf);
     w[l] = v.lo;
     if (WAVE + l < RW) w[WAVE + l] = v.hi;
   }

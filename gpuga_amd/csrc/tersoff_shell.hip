@@ -164,7 +164,7 @@ struct TersoffShell {
         const float fy = fmaf(coef, r.y, -hc * fmaf(-m[u], eu.y, cy[u]));
         const float fz = fmaf(coef, r.z, -hc * fmaf(-m[u], eu.z, cz[u]));
         if (FORCE) {
-          const int rb = wave_first(reinterpret_cast<const int*>(R + 1 + 2 * M)[u]);
+          const int rb = wave_first(reinterpret_cast<const record_word*>(R + 1 + 2 * M)[u]);
           float* o = fblk + (size_t)rb * 3 * WAVE + lane;
           cstore(o, fx);
           cstore(o + WAVE, fy);
@@ -213,7 +213,7 @@ struct TersoffShell {
   }
   __device__ static void spread_store(float4* buf, const Spread& v)
   {
-    int* w = reinterpret_cast<int*>(buf);
+    record_word* w = reinterpret_cast<record_word*>(buf);
 #pragma unroll
     for (int k = 0; k < NW; ++k)
       if (WAVE * k + (int)__lane_id() < RW) w[WAVE * k + __lane_id()] = v.w[k];
