@@ -738,8 +738,7 @@ void Fitness::setup_quad()
   rows.b = b;
   rows.col = d_col.get();
   for (int f = 0; f < 3; ++f) rows.nb[f] = nb[f];
-  if (quad_energy_lds(rows) > 156u * 1024u) return;
-  quad_prepare(rows);
+  if (!quad_prepare(rows)) return;
   quad_.basis = b;
   quad_.n_act = (int)act.size();
   quad_.act.upload(act, st);

@@ -133,8 +133,8 @@ void launch_ri_table(int B, const float4* bond, float4* tab, hipStream_t st);
 // many pairs (at most QCE elements of all codes)
 constexpr int QCE = 64;
 void launch_quad_used(const DevSet& s, const QuadBasis& b, int* used, hipStream_t st);
-size_t quad_energy_lds(const QuadRows& q);
-void quad_prepare(const QuadRows& q); // raises the row kernels' LDS limits
+// raises the row kernels' LDS limits; false: the rows do not fit
+bool quad_prepare(const QuadRows& q);
 // rows of the configurations [c0, c1) (energy [c1 - c0][D0], virial
 // 6 rows each [..][D1]) and of the force atoms [i0, i1) (3 rows each)
 void launch_quad_energy_rows(const DevSet& s, const QuadRows& q, int c0, int c1, double* re,

@@ -183,6 +183,7 @@ __device__ __forceinline__ void add_pair(double* row, const int* mu, const int* 
 }
 
 constexpr int ENERGY_THREADS = 256, FORCE_THREADS = 96;
+constexpr size_t kRowLds = 156 * 1024; // their dynamic LDS at most
 
 // Rows of one energy configuration per workgroup: half-wave 0 its energy,
 // half-waves 1-6 its virial components, each over the unordered pairs in bond
@@ -598,20 +599,23 @@ static size_t force_lds(const QuadRows& q)
   return FORCE_THREADS * sizeof(PairRec) + sizeof(double) * 3 * q.D(2);
 }
 
-size_t quad_energy_lds(const QuadRows& q)
+static size_t quad_energy_lds(const QuadRows& q)
 {
   return ENERGY_THREADS * sizeof(PairRec) + sizeof(double) * (q.D(0) + 6 * q.D(1));
 }
 
-void quad_prepare(const QuadRows& q)
+bool quad_prepare(const QuadRows& q)
 {
-  const std::pair<const void*, size_t> k[2] = {
-    {reinterpret_cast<const void*>(&quad_energy_rows), quad_energy_lds(q)},
-    {reinterpret_cast<const void*>(&quad_force_rows), force_lds(q)}};
-  for (const auto& x : k)
-    if (x.second > 64u * 1024u)
-      GPUGA_HIP(hipFuncSetAttribute(x.first, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)x.second));
+  const size_t lds[2] = {quad_energy_lds(q), force_lds(q)};
+  if (std::max(lds[0], lds[1]) > kRowLds) return false;
+  // (a kernel's limit is the process's: the same for every set, of which several
+  // may be set up at once on different threads)
+  const void* k[2] = {reinterpret_cast<const void*>(&quad_energy_rows),
+                      reinterpret_cast<const void*>(&quad_force_rows)};
+  for (int i = 0; i < 2; ++i)
+    if (lds[i] > 64u * 1024u)
+      GPUGA_HIP(hipFuncSetAttribute(k[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRowLds));
+  return true;
 }
 
 void launch_quad_energy_rows(const DevSet& s, const QuadRows& q, int c0, int c1, double* re,
