@@ -1438,26 +1438,26 @@ void Fitness::run_ga(GA& ga, int first_generation, int generations, float* best,
   const GA before = ga;
   if (!pl.dga || !pl.dga->matches(ga))
     pl.dga = std::make_unique<DeviceGA>(ga, pl.genes.get(), 1024, st, opt_.ga_batch);
-  const auto run = [&] {
-    const bool done = run_generations(pl, ga, first_generation, generations, quad, best, elite);
-    if (!done) ga = before;
-    return done;
-  };
-  if (!run()) {
-    // An individual that the forms do not resolve: the pair loop's tables are
-    // built (once, and only where a run meets one), and the run starts again.
-    // Its generations up to there are the same bit for bit.
+  // Individuals that the forms do not resolve are evaluated again in their
+  // generation from the start where the plan's last run or call had some, else
+  // from the first generation that has, in which case the run starts again (its
+  // generations up to there are the same bit for bit): a generation that needs none
+  // is spared two launches.
+  bool again = quad && pl.sharp_before && pl.items_built;
+  if (!run_generations(pl, ga, before, first_generation, generations, quad, again, best, elite)) {
+    ga = before;
     ensure_items(pl);
-    run();
+    again = true;
+    run_generations(pl, ga, before, first_generation, generations, quad, again, best, elite);
   }
+  if (quad) pl.sharp_before = *pl.h_sharp() != 0u;
 }
 
-bool Fitness::run_generations(PopPlan& pl, GA& ga, int first_generation, int generations,
-                              bool quad, float* best, float* elite)
+bool Fitness::run_generations(PopPlan& pl, GA& ga, const GA& before, int first_generation,
+                              int generations, bool quad, bool again, float* best, float* elite)
 {
   const int V = spec_.V;
   hipStream_t st = stream_;
-  const GA before = ga;
   DeviceGA& dga = *pl.dga;
   dga.upload(ga, first_generation, st);
   // batches double from one generation up to the staging capacity, so the
@@ -1470,10 +1470,7 @@ bool Fitness::run_generations(PopPlan& pl, GA& ga, int first_generation, int gen
   // process's first long run up to 4 ms)
   const int H = dga.history_cap();
   std::vector<float> h((size_t)H * (1 + V));
-  // With the pair loop's tables there, each generation's listed individuals are
-  // evaluated again before the GA step (two launches that end at once when
-  // there are none); without them the run ends where there is one.
-  const bool check = quad && pl.qeval.sharp.sums, again = check && pl.items_built;
+  const bool check = quad && pl.qeval.sharp.sums && !again;
   *pl.h_sharp() = 0u;
   const volatile unsigned* sharp = pl.h_sharp();
   int g = 0; // generations queued
@@ -1494,14 +1491,14 @@ bool Fitness::run_generations(PopPlan& pl, GA& ga, int first_generation, int gen
         if (again) launch_population(pl, sharp_ctl(pl, ctl), st);
         dga.step(k, pl.ctl.fitness, st);
       }
-      if (check && !again && *sharp) {
+      if (check && *sharp) {
         GPUGA_HIP(hipStreamSynchronize(st));
         return false;
       }
     }
     if (timing_) GPUGA_HIP(hipEventRecord(ev1_, st));
     const unsigned status = dga.collect((g + n) & 1, n, pl.ctl.status, st);
-    if (check && !again && *sharp) return false;
+    if (check && *sharp) return false;
     if (timing_) {
       float ms = 0.0f;
       GPUGA_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));

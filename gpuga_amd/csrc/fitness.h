@@ -248,10 +248,11 @@ private:
   void launch_quad_eval(PopPlan& pl, const PopCtl& ctl, hipStream_t st);
   // ctl's launch for the individuals that the last launch_quad_eval listed
   PopCtl sharp_ctl(const PopPlan& pl, PopCtl ctl) const;
-  // run_ga's generations; false, with the GA's state to be restored, when they
-  // need the pair loop's tables and these are not there
-  bool run_generations(PopPlan& pl, GA& ga, int first_generation, int generations, bool quad,
-                       float* best, float* elite);
+  // run_ga's generations.  again: with the individuals that the forms do not
+  // resolve evaluated again; else false, the GA's state to be restored, where
+  // there are some.
+  bool run_generations(PopPlan& pl, GA& ga, const GA& before, int first_generation,
+                       int generations, bool quad, bool again, float* best, float* elite);
   void launch_quad_values(PopPlan& pl, const PopCtl& ctl, int first, int count, hipStream_t st);
   int tune(int P);
   double time_plan(int P, const LaunchShape& sh, int reps, int* occ = nullptr);
