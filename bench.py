@@ -36,10 +36,9 @@ MI355X_HBM_PEAK = 8.0e12     # B/s
 # Algorithmic work per individual x atom evaluation (4 neighbours per atom):
 # pair terms ~106 FLOP x 4, triplets ~57 FLOP x 12, assembly -> ~1.1 kFLOP.
 TERSOFF_FLOP_PER_UNIT = 1.1e3
-# Pair potentials: the work per pair of the formulas (the quadratic forms that
-# evaluate a population do not execute it per pair, so the fraction of peak is
-# a measure of time against this work and can exceed 1; each
-# unordered pair once in energy/virial configurations, every ordered pair in
+# Pair potentials: the work per pair of the formulas, which the per-individual
+# kernels execute (the quadratic forms that evaluate a population do not, and have
+# no rate; each unordered pair once in energy/virial configurations, every ordered pair in
 # force configurations; distance-only factors such as erfc(a r)/r come from
 # the set-up tables).  FMA = 2 FLOP; exp2 not counted.
 #  RI, per pair: Buckingham + shifted-force Coulomb value and derivative
@@ -378,8 +377,9 @@ def main():
     P, V, N = (args.population or w["P"]), fit.V, fit.N
     chunk = args.chunk_cost
     shape = None
-    if not args.plain:
-        # (tunes the shape first when --chunk-cost is 0)
+    if not args.plain and w["kind"] == "tersoff":
+        # (tunes the shape first when --chunk-cost is 0; the pair potentials'
+        # quadratic forms have none)
         shape = fit.launch_shape(P)
         chunk = shape["chunk_cost"]
     parents = P // 2 + (P - P // 2) % 2  # the GA pairs the children: P - parents even
@@ -449,7 +449,11 @@ def main():
                     "per individual: the formula's work, which the quadratic forms do not execute")
     if args.plain:
         flop /= P  # timing covers one individual per launch group
-    achieved = flop / kernel_s
+    achieved, frac = flop / kernel_s / 1e12, flop / kernel_s / peak
+    if w["kind"] != "tersoff" and not args.plain:
+        # work that is not executed has no rate
+        achieved = frac = None
+        bound = "latency"
     data = {"tersoff": "seeded diamond-Si cells", "ri": "seeded AB2 fluorite cells",
             "nn2b": "seeded AB wurtzite cells"}[w["kind"]]
     out = {
@@ -472,8 +476,8 @@ def main():
                    "chunk_cost": chunk, "launch_shape": shape,
                    "s_per_generation": ms_step / 1e3,
                    "best_fitness": best},
-        "roofline": {"bound": bound, "achieved": achieved / 1e12, "peak": peak / 1e12,
-                     "unit": "TFLOP/s", "frac": achieved / peak,
+        "roofline": {"bound": bound, "achieved": achieved, "peak": peak / 1e12,
+                     "unit": "TFLOP/s", "frac": frac,
                      "traffic": None if args.plain else measured_traffic(args.workload),
                      "kernel_ms": kernel_s * 1e3},
     }

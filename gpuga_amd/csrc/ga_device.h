@@ -50,7 +50,7 @@ constexpr int kGaMaxBatch = 32;
 // rows per workgroup and LDS bytes of the step for shape (P, V)
 void ga_step_shape(int P, int V, int* rows, size_t* lds);
 // checks the shape fits a workgroup and raises the LDS limit when needed
-// (once per shape, outside graph capture)
+// (once per shape)
 void ga_step_prepare(int P, int V);
 void launch_ga_step(const GaDev& d, hipStream_t st);
 void launch_ga_begin(const GaDev& d, float* genes, const float* from, int generation,
@@ -85,7 +85,7 @@ public:
   // stage().
   void stage(GA& ga, int generation, int n, hipStream_t st);
   // one step reading population buffer k and writing buffer 1 - k, on
-  // fitness (device pointer); graph-capturable
+  // fitness (device pointer)
   void step(int k, const float* fitness, hipStream_t st) const;
   // Wait for the steps queued so far, with what download() and history() are
   // asked for next (population buffer k, n history rows) on the host; returns

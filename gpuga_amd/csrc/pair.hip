@@ -339,8 +339,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // per atom with both layers in scratch memory (two scratch accesses an FMA,
 // 450 waves for 1024 SIMDs) took 4617 us on 28 800 atoms with 42 neighbours
 // and n = 32; this form 118 us (106 us with a tanh of 1e-7 absolute and the
-// bias among the products' sum, which left networks with weights of 0.02 five
-// to seventeen times the error of the scalar form).  Eight atoms a wave leave
+// bias among the products' sum, which left networks with weights of 0.02 eight
+// to fourteen times the error of the scalar form).  Eight atoms a wave leave
 // 5% of the tiles' bonds empty there and give 3600 waves; with species, the
 // code t_i + t_j shifts the first layer's bias.
 constexpr int NN2B_ATOMS = 8;

@@ -43,8 +43,7 @@
 // fitness (with one group, its last configuration does).  Every reduction
 // has a fixed order, so results do not depend on scheduling or on what else
 // runs on the device.  All counters are returned to zero by their last user,
-// so launches follow one another (or replay from a captured graph) without
-// clearing memory.
+// so launches follow one another without clearing memory.
 //
 // Replaces the per-individual host loop of Fitness::compute
 // (src/fitness.cu:316-333) and its reductions (src/fitness.cu:392-555).
