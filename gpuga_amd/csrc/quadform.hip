@@ -333,9 +333,10 @@ __global__ void __launch_bounds__(256) quad_fold(const double* __restrict__ part
   }
 }
 
-// The tiles transformed to nodal values: coefficient k of an element is sum_m C[k][m] f(x_m) with C[k][m] =
-// (2 / QB) cos(k theta_m) (half of it for k = 0), so Q <- C^T Q C, block by
-// block; the linear block stays.  A tile off the diagonal counts twice.
+// The tiles transformed to nodal values: coefficient k of an element is
+// sum_m C[k][m] f(x_m) with C[k][m] = (2 / QB) cos(k theta_m) (half of it for
+// k = 0), so Q <- C^T Q C, block by block; the linear block stays.  A tile off
+// the diagonal counts twice.
 __global__ void __launch_bounds__(256) quad_finish(double* __restrict__ q)
 {
   __shared__ double T[QB][QB + 1], C[QB][QB + 1];
