@@ -451,6 +451,9 @@ __global__ void __launch_bounds__(256) ri_values(PopCtl ctl, NodeTable tab)
 // us with a unit's workgroups on all XCDs, each fetching the form, 21.8 us so.
 constexpr int EVAL_WAVES = 4;
 
+// CHECK: with the individuals that the nodes do not resolve listed (NN2B; rigid
+// ion's calls are 0.4 us of 27 shorter without).
+template <bool CHECK>
 __global__ void __launch_bounds__(EVAL_WAVES * WAVE, 4) quad_eval(PopCtl ctl, QuadEval q)
 {
   constexpr int SLICES = EVAL_WAVES * WAVE / QP;
@@ -463,7 +466,7 @@ __global__ void __launch_bounds__(EVAL_WAVES * WAVE, 4) quad_eval(PopCtl ctl, Qu
   const int groups = q.ld / QP;
   const int unit = (int)blockIdx.x / kXcds / groups * kXcds + (int)blockIdx.x % kXcds;
   const int pb = (int)blockIdx.x / kXcds % groups;
-  if (q.sharp.sums && blockIdx.x == 0 && threadIdx.x == 0) *q.sharp.next = 0u;
+  if (CHECK && blockIdx.x == 0 && threadIdx.x == 0) *q.sharp.next = 0u;
   if (unit >= q.units) return;
   const int2 fi = ldu(q.unit, unit);
   const int f = fi.x, I = fi.y;
@@ -532,7 +535,7 @@ __global__ void __launch_bounds__(EVAL_WAVES * WAVE, 4) quad_eval(PopCtl ctl, Qu
   const int l = t % QP, sl = t / QP;
   int first = 0;
   float tail[2][kTailSums] = {};
-  if (q.sharp.sums && t < QP)
+  if (CHECK && t < QP)
 #pragma unroll
     for (int k = 0; k < kTailSums; ++k) {
       tail[0][k] = q.sharp.sums[(long)k * ld + p0 + t];
@@ -546,14 +549,14 @@ __global__ void __launch_bounds__(EVAL_WAVES * WAVE, 4) quad_eval(PopCtl ctl, Qu
     first += q.form[s].nb;
   }
   bool resolved = true;
-  if (q.sharp.sums && t < QP && p0 + t < ctl.P) {
+  if (CHECK && t < QP && p0 + t < ctl.P) {
 #pragma unroll
     for (int k = 0; k < kTailSums; k += 2) { // (a NaN or an infinite sum: not)
       const float c = tail[0][k] + tail[1][k], size = tail[0][k + 1] + tail[1][k + 1];
       resolved = resolved && c <= q.sharp.limit2 * size && size < __builtin_inff();
     }
   }
-  const unsigned long long m = __ballot(!resolved);
+  const unsigned long long m = CHECK ? __ballot(!resolved) : 0ull;
   if (w == 0 && m) {
     const int at = (int)wave_atomic_add(q.sharp.count, (unsigned)__popcll(m));
     if (!resolved) q.sharp.list[at + __popcll(m & ((1ull << lane) - 1ull))] = p0 + t;
@@ -662,7 +665,8 @@ void launch_ri_values(const PopCtl& ctl, const NodeTable& t, hipStream_t st)
 void launch_quad_eval(const PopCtl& ctl, const QuadEval& q, hipStream_t st)
 {
   const int blocks = (q.units + kXcds - 1) / kXcds * kXcds * (q.ld / QP);
-  quad_eval<<<blocks, EVAL_WAVES * WAVE, 0, st>>>(ctl, q);
+  if (q.sharp.sums) quad_eval<true><<<blocks, EVAL_WAVES * WAVE, 0, st>>>(ctl, q);
+  else quad_eval<false><<<blocks, EVAL_WAVES * WAVE, 0, st>>>(ctl, q);
   GPUGA_HIP(hipGetLastError());
 }
 
